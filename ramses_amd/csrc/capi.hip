@@ -94,11 +94,12 @@ thread_local std::string g_err;
 // by every entry point: hydro parameters, prolongation and refinement
 // criteria.
 struct Config {
-  ramses::HydroParams hp{1.4, 1e-10, 1e-10, 1.5, 0.5, 1, ramses::kLLF, 10};
+  ramses::HydroParams hp{1.4, 1e-10, 1e-10, 1.5, 0.5, 1, ramses::kLLF, 10, 0};
   int precision = RAMSES_FP64;
   int nvector = 32;
   bool set = false;
   int interpol_type = 1, interpol_var = 0;  // hydro/hydro_parameters.f90:88-89
+  Config() { hp.div_hi = ramses::div_range(hp); }
   ramses::RefineParams rp{-1.0, -1.0, -1.0, 1e-10, 1e-10, 1e-10, 1};
 };
 
@@ -189,6 +190,7 @@ int ramses_hydro_config(const ramses_hydro_params* p) {
   c.hp.slope_type = p->slope_type;
   c.hp.riemann = p->riemann;
   c.hp.niter_riemann = p->niter_riemann;
+  c.hp.div_hi = ramses::div_range(c.hp);
   c.precision = p->precision;
   c.nvector = p->nvector;
   c.set = true;

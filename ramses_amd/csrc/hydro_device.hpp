@@ -30,7 +30,20 @@ struct HydroParams {
   int slope_type;  // 0,1,2,3,7,8
   int riemann;     // Riemann enum
   int niter_riemann;  // Newton iterations of the exact solver
+  unsigned div_hi;    // upper word of the bound below which FP64 values may take the shared reciprocals (0: none)
 };
+
+// The bound on densities and pressures for the unscaled FP64 division and
+// square root below (quotients): 2^50, as the upper word of the double, when
+// the floors keep every value that is divided by, and every root's argument,
+// far from underflow; else 0, and no value passes.
+inline unsigned div_range(const HydroParams& hp) {
+  const double lo = 0x1p-60, hi = 0x1p40;
+  const bool ok = hp.smallr >= lo && hp.smallr <= hi && hp.smallc >= lo && hp.smallc <= hi &&
+                  hp.gamma - 1.0 >= 0x1p-20 && hp.gamma <= 0x1p10 && hp.slope_theta >= -0x1p10 &&
+                  hp.slope_theta <= 0x1p10;
+  return ok ? (1023u + 50u) << 20 : 0u;
+}
 
 // Launch-shape knobs set through ramses_tune (0 = built-in default).
 struct Tuning {
@@ -71,6 +84,44 @@ __device__ __forceinline__ double abs_w(double a) { return __builtin_fabs(a); }
 __device__ __forceinline__ float abs_w(float a) { return __builtin_fabsf(a); }
 __device__ __forceinline__ double copysign_w(double a, double b) { return __builtin_copysign(a, b); }
 __device__ __forceinline__ float copysign_w(float a, float b) { return __builtin_copysignf(a, b); }
+
+// FP64 division and square root without the compiler's scaling.  a / b
+// compiles to eleven instructions: two v_div_scale, the reciprocal estimate,
+// two Newton steps on it, the quotient with its remainder correction
+// (Markstein, 1990) and v_div_fixup.  Scaling by powers of two and the fixup
+// change nothing while every operand and remainder is a normal number, so in
+// that range quotients by one divisor share its reciprocal (five
+// instructions) and cost three each, bit for bit the same.  The callers test
+// the range and a wavefront with a lane outside it takes a / b instead.
+__device__ __forceinline__ double rcp_newton(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  double e = __builtin_fma(-d, y, 1.0);
+  y = __builtin_fma(y, e, y);
+  e = __builtin_fma(-d, y, 1.0);
+  return __builtin_fma(y, e, y);
+}
+// n / d with y = rcp_newton(d); n zero or normal, not -0.0
+__device__ __forceinline__ double quot(double n, double d, double y) {
+  const double q = n * y;
+  return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+// sqrt(x) for x normal and >= 2^-767, where the compiler's sequence (Goldschmidt
+// steps on v_rsq, then two residual corrections) does not scale either
+__device__ __forceinline__ double sqrt_normal(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = y * 0.5;
+  const double r = __builtin_fma(-h, g, 0.5);
+  h = __builtin_fma(h, r, h);
+  g = __builtin_fma(g, r, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+__device__ __forceinline__ unsigned hi_word(double x) {
+  return (unsigned)((unsigned long long)__builtin_bit_cast(long long, x) >> 32);
+}
+__device__ __forceinline__ unsigned max_u(unsigned a, unsigned b) { return a > b ? a : b; }
+// Whether any active lane's flag is clear: a scalar branch.
+__device__ __forceinline__ bool any_not(bool ok) { return __builtin_expect(__ballot(!ok) != 0, 0); }
 
 // Primitive state of one cell: rho, vx, vy, vz, p.
 template <typename R>
@@ -134,8 +185,11 @@ __device__ __forceinline__ R slope1(R qm1, R q0, R qp1, int st_run, R theta) {
   if (st == 1) {
     const R dlft = q0 - qm1;
     const R drgt = qp1 - q0;
-    if ((dlft * drgt) <= zero) return zero;
-    return (dlft > zero) ? fmin_f(dlft, drgt) : fmax_f(dlft, drgt);
+    // Both selects as selects: written with an early `return zero`, each of
+    // the 15 slopes of a cell is an exec-mask branch that cuts the trace into
+    // small blocks.
+    const R lim = (dlft > zero) ? fmin_f(dlft, drgt) : fmax_f(dlft, drgt);
+    return (dlft * drgt) <= zero ? zero : lim;
   } else if (st == 2) {
     const R two = (R)2;
     const R dlft = two * (q0 - qm1);
@@ -181,16 +235,50 @@ struct Source {
   R sr0, su0, sv0, sw0, sp0;
 };
 
-template <typename R>
+// The quotients of the three pressure slopes by rho.  In FP64 they share
+// rho's reciprocal where rho, p and the slopes are below the bound of
+// div_range: rho and p have floors, so a slope is zero or far above
+// underflow.  Minmod (ST = 1) gives slopes of the positive p that are never
+// larger than p itself, and no -0.0, so it needs neither their test nor the
+// fixup that keeps a zero's sign.
+template <typename R, int ST>
+__device__ __forceinline__ void pressure_terms(const Prim<R>& q, R px, R py, R pz, unsigned div_hi, R& ax, R& ay, R& az) {
+  if constexpr (sizeof(R) == 8) {
+    const double y = rcp_newton(q.r);
+    ax = quot(px, q.r, y);
+    ay = quot(py, q.r, y);
+    az = quot(pz, q.r, y);
+    unsigned m = max_u(hi_word(q.r), hi_word(q.p));
+    if constexpr (ST != 1) {
+      ax = __builtin_amdgcn_div_fixup(ax, q.r, px);
+      ay = __builtin_amdgcn_div_fixup(ay, q.r, py);
+      az = __builtin_amdgcn_div_fixup(az, q.r, pz);
+      m = max_u(max_u(m, hi_word(px) & 0x7fffffffu), max_u(hi_word(py) & 0x7fffffffu, hi_word(pz) & 0x7fffffffu));
+    }
+    if (any_not(m < div_hi)) {
+      ax = px / q.r;
+      ay = py / q.r;
+      az = pz / q.r;
+    }
+  } else {
+    ax = div_w(px, q.r);
+    ay = div_w(py, q.r);
+    az = div_w(pz, q.r);
+  }
+}
+
+template <typename R, int ST = -1>
 __device__ __forceinline__ Source<R> trace_sources(const Prim<R>& q, const Prim<R>& dx_,
-                                                   const Prim<R>& dy_, const Prim<R>& dz_, R gamma) {
+                                                   const Prim<R>& dy_, const Prim<R>& dz_, R gamma, unsigned div_hi) {
   const R r = q.r, u = q.u, v = q.v, w = q.w, p = q.p;
+  R ax, ay, az;
+  pressure_terms<R, ST>(q, dx_.p, dy_.p, dz_.p, div_hi, ax, ay, az);
   Source<R> s;
   s.sr0 = -u * dx_.r - v * dy_.r - w * dz_.r - (dx_.u + dy_.v + dz_.w) * r;
   s.sp0 = -u * dx_.p - v * dy_.p - w * dz_.p - (dx_.u + dy_.v + dz_.w) * gamma * p;
-  s.su0 = -u * dx_.u - v * dy_.u - w * dz_.u - div_w((dx_.p), r);
-  s.sv0 = -u * dx_.v - v * dy_.v - w * dz_.v - div_w((dy_.p), r);
-  s.sw0 = -u * dx_.w - v * dy_.w - w * dz_.w - div_w((dz_.p), r);
+  s.su0 = -u * dx_.u - v * dy_.u - w * dz_.u - ax;
+  s.sv0 = -u * dx_.v - v * dy_.v - w * dz_.v - ay;
+  s.sw0 = -u * dx_.w - v * dy_.w - w * dz_.w - az;
   return s;
 }
 
@@ -232,23 +320,59 @@ __device__ __forceinline__ Face<R> rotate(const Prim<R>& q, int d) {
   return f;
 }
 
+// N quotients of any values by one divisor.  The shared reciprocal serves
+// where the divisor lies in [2^-120, 2^120) in magnitude and every numerator
+// is zero, infinite, a NaN (v_frexp gives them exponent 0, and the fixup
+// their quotients) or in [2^-800, 2^800): a wavefront with a lane outside
+// divides in full.
+template <int N, typename R>
+__device__ __forceinline__ void quotients(const R* n, R d, R* out) {
+  if constexpr (sizeof(R) == 8) {
+    const double y = rcp_newton(d);
+    int lo = 0, hi = 0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const int e = __builtin_amdgcn_frexp_exp(n[k]);
+      lo = e < lo ? e : lo;
+      hi = e > hi ? e : hi;
+      out[k] = __builtin_amdgcn_div_fixup(quot(n[k], d, y), d, n[k]);
+    }
+    const unsigned dh = (hi_word(d) & 0x7fffffffu) - ((1023u - 120u) << 20);
+    if (!any_not(dh < (240u << 20) && lo > -800 && hi < 800)) return;
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) out[k] = div_w(n[k], d);
+}
+
 // Godunov flux in rotated order plus the internal-energy flux (fgdnv(1:6)).
 template <typename R>
 struct Flux6 {
   R f[6];
 };
 
+// The sound speeds sqrt(gamma*p/rho) of both sides of a face, p and rho at
+// or above their floors.
+template <typename R>
+__device__ __forceinline__ void sound_speeds(R rl, R pl, R rr, R pr, R gamma, unsigned div_hi, R& cl, R& cr) {
+  const R nl = gamma * pl, nr = gamma * pr;
+  if constexpr (sizeof(R) == 8) {
+    cl = sqrt_normal(quot(nl, rl, rcp_newton(rl)));
+    cr = sqrt_normal(quot(nr, rr, rcp_newton(rr)));
+    if (!any_not(max_u(max_u(hi_word(rl), hi_word(rr)), max_u(hi_word(pl), hi_word(pr))) < div_hi)) return;
+  }
+  cl = sqrt_w(div_w(nl, rl));
+  cr = sqrt_w(div_w(nr, rr));
+}
+
 // riemann_llf: hydro/godunov_utils.f90:660-820
 template <typename R>
 __device__ __forceinline__ Flux6<R> riemann_llf(const Face<R>& L, const Face<R>& Rt, R gamma, R smallr,
-                                                R smallp, R entho) {
+                                                R smallp, R entho, unsigned div_hi) {
   const R half = (R)0.5;
   const R rl = fmax_f(L.r, smallr), ul = L.un, pl = fmax_f(L.p, rl * smallp);
-  R cl = gamma * pl;
-  cl = sqrt_w(div_w(cl, rl));
   const R rr = fmax_f(Rt.r, smallr), ur = Rt.un, pr = fmax_f(Rt.p, rr * smallp);
-  R cr = gamma * pr;
-  cr = sqrt_w(div_w(cr, rr));
+  R cl, cr;
+  sound_speeds(rl, pl, rr, pr, gamma, div_hi, cl, cr);
   const R cmax = fmax_f(abs_w(ul) + cl, abs_w(ur) + cr);
   R uL[6], uR[6], fL[6], fR[6];
   uL[0] = L.r;
@@ -287,14 +411,12 @@ __device__ __forceinline__ Flux6<R> riemann_llf(const Face<R>& L, const Face<R>&
 // riemann_hll: hydro/godunov_utils.f90:825-983
 template <typename R>
 __device__ __forceinline__ Flux6<R> riemann_hll(const Face<R>& L, const Face<R>& Rt, R gamma, R smallr,
-                                                R smallp, R entho) {
+                                                R smallp, R entho, unsigned div_hi) {
   const R half = (R)0.5, zero = (R)0;
   const R rl = fmax_f(L.r, smallr), ul = L.un, pl = fmax_f(L.p, rl * smallp);
-  R cl = gamma * pl;
-  cl = sqrt_w(div_w(cl, rl));
   const R rr = fmax_f(Rt.r, smallr), ur = Rt.un, pr = fmax_f(Rt.p, rr * smallp);
-  R cr = gamma * pr;
-  cr = sqrt_w(div_w(cr, rr));
+  R cl, cr;
+  sound_speeds(rl, pl, rr, pr, gamma, div_hi, cl, cr);
   const R SL = fmin_f(fmin_f(ul, ur) - fmax_f(cl, cr), zero);
   const R SR = fmax_f(fmax_f(ul, ur) + fmax_f(cl, cr), zero);
   R uL[6], uR[6], fL[6], fR[6];
@@ -327,17 +449,30 @@ __device__ __forceinline__ Flux6<R> riemann_hll(const Face<R>& L, const Face<R>&
   }
   Flux6<R> g;
   const R den = SR - SL;
+  R num[6];
 #pragma unroll
-  for (int n = 0; n < 6; ++n) g.f[n] = div_w(SR * fL[n] - SL * fR[n] + SR * SL * (uR[n] - uL[n]), den);
+  for (int n = 0; n < 6; ++n) num[n] = SR * fL[n] - SL * fR[n] + SR * SL * (uR[n] - uL[n]);
+  quotients<6>(num, den, g.f);
   return g;
 }
 
 // riemann_hllc: hydro/godunov_utils.f90:988-1209.  Only the star state of
 // the sampled branch feeds the flux, so the other branch's divisions are
 // skipped; the values of the sampled quantities are unchanged.
+//
+// In FP64 the nine divisions and roots of a face take shared reciprocals
+// (quot) where this cannot be seen.  Why the tests suffice, with rho and P
+// below 2^50 and floors of at least 2^-60 and 2^-190 (div_range): c lies in
+// [2^-60, 2^60].  rcl and rcr are not negative, so their sum in [2^-100,
+// 2^110) bounds |ul - ur| by 2^170, hence |u| by 2^225 (beyond, u - SL
+// rounds to 0), and every intermediate below is at most 2^926.  A sum of
+// such terms is zero or above 2^-310 unless a single tiny term stands alone;
+// only the velocities can be tiny, and the test of ustar's numerator excludes
+// it.  |S - ustar| >= 2^-90 and a total energy below 2^800 (which also
+// excludes infinite and NaN tangential velocities) close the star state.
 template <typename R>
 __device__ __forceinline__ Flux6<R> riemann_hllc(const Face<R>& L, const Face<R>& Rt, R gamma, R smallr,
-                                                 R smallp, R entho, R smallc2) {
+                                                 R smallp, R entho, R smallc2, unsigned div_hi) {
   const R half = (R)0.5, zero = (R)0;
   const R rl = fmax_f(L.r, smallr);
   const R Pl = fmax_f(L.p, rl * smallp);
@@ -357,20 +492,39 @@ __device__ __forceinline__ Flux6<R> riemann_hllc(const Face<R>& L, const Face<R>
   ecinr = ecinr + half * rr * (Rt.ut2 * Rt.ut2);
   const R etotr = er + ecinr;
   const R Ptotr = Pr;
-  R cfastl = gamma * Pl;
-  cfastl = sqrt_w(fmax_f(div_w(cfastl, rl), smallc2));
-  R cfastr = gamma * Pr;
-  cfastr = sqrt_w(fmax_f(div_w(cfastr, rr), smallc2));
-  const R SL = fmin_f(ul, ur) - fmax_f(cfastl, cfastr);
-  const R SR = fmax_f(ul, ur) + fmax_f(cfastl, cfastr);
-  const R rcl = rl * (ul - SL);
-  const R rcr = rr * (SR - ur);
-  const R ustar = div_w(rcr * ur + rcl * ul + (Ptotl - Ptotr), (rcr + rcl));
+  R SL, SR, rcl, rcr, ustar, Ptotstar;
+  // the waves from the two sound speeds, and the numerators and the divisor
+  // of the star velocity and pressure
+  R nu, np, den;
+  auto waves = [&](R cfastl, R cfastr) {
+    SL = fmin_f(ul, ur) - fmax_f(cfastl, cfastr);
+    SR = fmax_f(ul, ur) + fmax_f(cfastl, cfastr);
+    rcl = rl * (ul - SL);
+    rcr = rr * (SR - ur);
+    nu = rcr * ur + rcl * ul + (Ptotl - Ptotr);
+    np = rcr * Ptotl + rcl * Ptotr + rcl * rcr * (ul - ur);
+    den = rcr + rcl;
+  };
+  bool full = true;
+  if constexpr (sizeof(R) == 8) {
+    waves(sqrt_normal(fmax_f(quot(gamma * Pl, rl, rcp_newton(rl)), smallc2)),
+          sqrt_normal(fmax_f(quot(gamma * Pr, rr, rcp_newton(rr)), smallc2)));
+    const double y = rcp_newton(den);
+    ustar = quot(nu, den, y);
+    Ptotstar = quot(np, den, y);
+    const unsigned m = max_u(max_u(hi_word(rl), hi_word(rr)), max_u(hi_word(Pl), hi_word(Pr)));
+    const unsigned dh = hi_word(den) - ((1023u - 100u) << 20);
+    full = any_not(m < div_hi && dh < (210u << 20) && __builtin_amdgcn_frexp_exp(nu) > -200);
+  }
+  if (full) {
+    waves(sqrt_w(fmax_f(div_w(gamma * Pl, rl), smallc2)), sqrt_w(fmax_f(div_w(gamma * Pr, rr), smallc2)));
+    ustar = div_w(nu, den);
+    Ptotstar = div_w(np, den);
+  }
   R ro, uo, Ptoto, etoto, eo;
   if (SL > zero) {
     ro = rl; uo = ul; Ptoto = Ptotl; etoto = etotl; eo = el;
   } else if (SR > zero || ustar > zero) {
-    const R Ptotstar = div_w(rcr * Ptotl + rcl * Ptotr + rcl * rcr * (ul - ur), (rcr + rcl));
     // left star state when ustar>0, right star state otherwise (SR>0)
     const bool left = ustar > zero;
     const R S = left ? SL : SR;
@@ -379,10 +533,21 @@ __device__ __forceinline__ Flux6<R> riemann_hllc(const Face<R>& L, const Face<R>
     const R es = left ? el : er;
     const R ets = left ? etotl : etotr;
     const R Pts = left ? Ptotl : Ptotr;
-    const R den = S - ustar;
-    ro = div_w(rs * (S - us), den);
-    etoto = div_w((S - us) * ets - Pts * us + Ptotstar * ustar, den);
-    eo = div_w(es * (S - us), den);
+    const R dS = S - ustar;
+    const R nr = rs * (S - us), ne = (S - us) * ets - Pts * us + Ptotstar * ustar, ni = es * (S - us);
+    bool fulls = true;
+    if constexpr (sizeof(R) == 8) {
+      const double y = rcp_newton(dS);
+      ro = quot(nr, dS, y);
+      etoto = quot(ne, dS, y);
+      eo = quot(ni, dS, y);
+      fulls = full || any_not(abs_w(dS) >= 0x1p-90 && ets < 0x1p800);
+    }
+    if (fulls) {
+      ro = div_w(nr, dS);
+      etoto = div_w(ne, dS);
+      eo = div_w(ni, dS);
+    }
     uo = ustar;
     Ptoto = Ptotstar;
   } else {
@@ -547,13 +712,23 @@ __host__ __device__ inline FluxScale make_scale(double dt, double dx) {
   return s;
 }
 
-template <typename R>
-__device__ __forceinline__ double scale_flux(R f, const FluxScale& s) {
+// N values of a face at once: one scalar branch for all, and where dx is no
+// power of two its reciprocal shared by their divisions.
+template <int N, typename R>
+__device__ __forceinline__ void scale_flux(const R* f, const FluxScale& s, double* out) {
   if constexpr (sizeof(R) == 8) {
-    const double fd = (double)f * s.dt;
-    return s.inv_dx != 0.0 ? fd * s.inv_dx : fd / s.dx;
+    double fd[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) fd[k] = f[k] * s.dt;
+    if (s.inv_dx != 0.0) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) out[k] = fd[k] * s.inv_dx;
+    } else {
+      quotients<N>(fd, s.dx, out);
+    }
   } else {
-    return (double)f * s.dtdx;
+#pragma unroll
+    for (int k = 0; k < N; ++k) out[k] = (double)f[k] * s.dtdx;
   }
 }
 
@@ -561,6 +736,7 @@ __device__ __forceinline__ double scale_flux(R f, const FluxScale& s) {
 template <typename R>
 struct SolverConsts {
   R gamma, smallr, smallp, entho, smallc2, theta, smallc;
+  unsigned div_hi;
   int riemann, slope_type, niter;
 };
 
@@ -573,6 +749,7 @@ __host__ __device__ inline SolverConsts<R> make_consts(const HydroParams& hp) {
   c.entho = (R)(1.0 / (hp.gamma - 1.0));
   c.smallc2 = (R)(hp.smallc * hp.smallc);
   c.theta = (R)hp.slope_theta;
+  c.div_hi = hp.div_hi;
   c.riemann = hp.riemann;
   c.slope_type = hp.slope_type;
   c.smallc = (R)hp.smallc;
@@ -582,19 +759,19 @@ __host__ __device__ inline SolverConsts<R> make_consts(const HydroParams& hp) {
 
 template <typename R>
 __device__ __forceinline__ Flux6<R> riemann_solve(const Face<R>& L, const Face<R>& Rt, const SolverConsts<R>& c) {
-  if (c.riemann == kHLLC) return riemann_hllc(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc2);
-  if (c.riemann == kHLL) return riemann_hll(L, Rt, c.gamma, c.smallr, c.smallp, c.entho);
+  if (c.riemann == kHLLC) return riemann_hllc(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc2, c.div_hi);
+  if (c.riemann == kHLL) return riemann_hll(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
   if (c.riemann == kACOUSTIC) return riemann_acoustic(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc);
   if (c.riemann == kEXACT) return riemann_exact(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc, c.niter);
-  return riemann_llf(L, Rt, c.gamma, c.smallr, c.smallp, c.entho);
+  return riemann_llf(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
 }
 
 template <typename R, int RS>
 __device__ __forceinline__ Flux6<R> riemann_fixed(const Face<R>& L, const Face<R>& Rt, const SolverConsts<R>& c) {
-  if constexpr (RS == kHLLC) return riemann_hllc(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc2);
-  else if constexpr (RS == kHLL) return riemann_hll(L, Rt, c.gamma, c.smallr, c.smallp, c.entho);
+  if constexpr (RS == kHLLC) return riemann_hllc(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc2, c.div_hi);
+  else if constexpr (RS == kHLL) return riemann_hll(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
   else if constexpr (RS == kDynamicRiemann) return riemann_solve(L, Rt, c);
-  else return riemann_llf(L, Rt, c.gamma, c.smallr, c.smallp, c.entho);
+  else return riemann_llf(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
 }
 
 // Conservative-variable flux of a face in (rho, mx, my, mz, E) order
@@ -644,23 +821,34 @@ __device__ __forceinline__ double cmpdt_cell(double u0, double u1, double u2, do
 // monotone), and min over cells equals its value at max over cells of w.
 // cmpdt_w is the per-cell part (hydro/godunov_utils.f90:24-97), cmpdt_from_w
 // the rest (:108-118), bitwise the reference when combined.
+//
+// Its four divisions by rho take the shared reciprocal (quot), its root
+// sqrt_normal, while rho is below the bound of div_range and the resulting w
+// below 2^400 (an operand that overflows on the way, is infinite or a NaN
+// leaves w no such number).  A momentum too small for an exact remainder
+// changes nothing: its velocity is added to c >= 2^-60.
 __device__ __forceinline__ double cmpdt_w(double u0, double u1, double u2, double u3, double u4,
                                           const HydroParams& hp) {
   const double gamma = hp.gamma;
   const double smallp = hp.smallc * hp.smallc / gamma;
   const double rho = fmax_f(u0, hp.smallr);
-  const double vx = u1 / rho, vy = u2 / rho, vz = u3 / rho;
-  double e = u4;
-  e = e - 0.5 * rho * (vx * vx);
-  e = e - 0.5 * rho * (vy * vy);
-  e = e - 0.5 * rho * (vz * vz);
-  double c = fmax_f((gamma - 1.0) * e, rho * smallp);
-  c = gamma * c;
-  c = __builtin_sqrt(c / rho);
-  double w = 3.0 * c;
-  w = w + __builtin_fabs(vx);
-  w = w + __builtin_fabs(vy);
-  w = w + __builtin_fabs(vz);
+  auto wave = [&](double vx, double vy, double vz, auto speed) {
+    double e = u4;
+    e = e - 0.5 * rho * (vx * vx);
+    e = e - 0.5 * rho * (vy * vy);
+    e = e - 0.5 * rho * (vz * vz);
+    double c = fmax_f((gamma - 1.0) * e, rho * smallp);
+    c = speed(gamma * c);
+    double w = 3.0 * c;
+    w = w + __builtin_fabs(vx);
+    w = w + __builtin_fabs(vy);
+    return w + __builtin_fabs(vz);
+  };
+  const double y = rcp_newton(rho);
+  double w = wave(quot(u1, rho, y), quot(u2, rho, y), quot(u3, rho, y),
+                  [&](double c) { return sqrt_normal(quot(c, rho, y)); });
+  if (any_not(hi_word(rho) < hp.div_hi && w < 0x1p400))
+    w = wave(u1 / rho, u2 / rho, u3 / rho, [&](double c) { return __builtin_sqrt(c / rho); });
   return w;
 }
 

@@ -210,7 +210,7 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
       const Prim<R> dqx = slope_prim<R, ST>(xm, qcur, xp, sc.slope_type, sc.theta);
       const Prim<R> dqy = slope_prim<R, ST>(ym, qcur, yp, sc.slope_type, sc.theta);
       const Prim<R> dqz = slope_prim<R, ST>(qprev, qcur, qnext, sc.slope_type, sc.theta);
-      const Source<R> src = trace_sources(qcur, dqx, dqy, dqz, sc.gamma);
+      const Source<R> src = trace_sources<R, ST>(qcur, dqx, dqy, dqz, sc.gamma, sc.div_hi);
       if constexpr (kWaves == 0) {
         trace_dir(qcur, dqx, src, dtdx, sc.smallr, qp_x, qm_x);
         trace_dir(qcur, dqy, src, dtdx, sc.smallr, qp_y, qm_y);
@@ -238,8 +238,7 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
         const Flux6<R> g = riemann_fixed<R, RS>(rotate(l, 0), rotate(qp_x, 0), sc);
         R fc[5];
         unrotate(g, 0, fc);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) fxs[v] = scale_flux(fc[v], fs);  // hydro/umuscl.f90:106
+        scale_flux<5>(fc, fs, fxs);  // hydro/umuscl.f90:106
       }
       if (interior || kind == kTop) {  // y face at y-1/2
         const int lo = e - EX;
@@ -247,8 +246,7 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
         const Flux6<R> g = riemann_fixed<R, RS>(rotate(l, 1), rotate(qp_y, 1), sc);
         R fc[5];
         unrotate(g, 1, fc);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) fys[v] = scale_flux(fc[v], fs);  // :129
+        scale_flux<5>(fc, fs, fys);  // :129
       }
       __syncthreads();
       // The fluxes, in double, go through the exchange area reinterpreted:
@@ -306,8 +304,7 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
       const Flux6<R> g = riemann_fixed<R, RS>(fz_left, rotate(qp_z, 2), sc);
       R fc[5];
       unrotate(g, 2, fc);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) fz[v] = scale_flux(fc[v], fs);  // :153
+      scale_flux<5>(fc, fs, fz);  // :153
     }
     // plane p-1 is complete: hydro/godunov_fine.f90:751-792 in idim order x, y, z
     if (interior && p >= z0 + 1) {

@@ -48,9 +48,11 @@ __device__ __forceinline__ unsigned xcd_contiguous(unsigned b, unsigned G) {
   return x * q + (x < r ? x : r) + b / X;
 }
 
-// One thread per (group, row, lane) task; G: a.grav is non-null.
+// One thread per (group, row, lane) task; G: a.grav is non-null.  The
+// gravity-free FP64 rows are held to 128 VGPRs (four waves per SIMD), which
+// they fit without a spill; left alone they take 134.
 template <typename R, int RS, bool S27, int ST, bool G>
-__global__ __launch_bounds__(768) void unsplit_rows(UnsplitArgs a) {
+__global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(!G && !S27 && ST >= 0 ? 4 : 3, 8))) void unsplit_rows(UnsplitArgs a) {
   const long t = (long)xcd_contiguous(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (t >= a.ngroups * 12L * a.nv) return;
   unsplit_task<R, RS, S27, false, ST, G>(a, t, a.ngroups, a.ngrid_last);

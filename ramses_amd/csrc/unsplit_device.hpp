@@ -107,11 +107,14 @@ __device__ __forceinline__ void store_face(double* flux, double* tmp, size_t fba
                                            const FluxScale& fs) {
   R fc[5];
   unrotate(g, d, fc);
+  const R t[2] = {(R)0.5 * (L.un + Rt.un), g.f[5]};  // :845
+  double o[5], ot[2];
+  scale_flux<5>(fc, fs, o);                          // :106,129,153
+  scale_flux<2>(t, fs, ot);                          // :111
 #pragma unroll
-  for (int v = 0; v < 5; ++v) flux[fbase + (size_t)v * fvs] = scale_flux(fc[v], fs);  // :106,129,153
-  const R t1 = (R)0.5 * (L.un + Rt.un);                                                // :845
-  tmp[tbase] = scale_flux(t1, fs);                                                    // :111
-  tmp[tbase + fvs] = scale_flux(g.f[5], fs);
+  for (int v = 0; v < 5; ++v) flux[fbase + (size_t)v * fvs] = o[v];
+  tmp[tbase] = ot[0];
+  tmp[tbase + fvs] = ot[1];
 }
 
 // One row of faces along direction D of one oct (see the file comment).
@@ -160,7 +163,7 @@ __device__ __forceinline__ void row_faces(const Ctx& c, const SolverConsts<R>& s
     const Prim<R>& dqx = (D == 0) ? dqd : dq1;
     const Prim<R>& dqy = (D == 1) ? dqd : ((D == 0) ? dq1 : dq2);
     const Prim<R>& dqz = (D == 2) ? dqd : dq2;
-    const Source<R> src = trace_sources(qb, dqx, dqy, dqz, sc.gamma);
+    const Source<R> src = trace_sources<R, S27 ? -1 : ST>(qb, dqx, dqy, dqz, sc.gamma, sc.div_hi);
     Prim<R> qp, qm;
     trace_dir(qb, dqd, src, dtdx, sc.smallr, qp, qm);
     if (s >= 1) {
@@ -199,7 +202,7 @@ __device__ __forceinline__ void trace_cell(const Ctx& c, const SolverConsts<R>& 
     dqy = slope_prim<R, ST>(c.prim(i, j - 1, k), q, c.prim(i, j + 1, k), sc.slope_type, sc.theta);
     dqz = slope_prim<R, ST>(c.prim(i, j, k - 1), q, c.prim(i, j, k + 1), sc.slope_type, sc.theta);
   }
-  const Source<R> src = trace_sources(q, dqx, dqy, dqz, sc.gamma);
+  const Source<R> src = trace_sources<R, S27 ? -1 : ST>(q, dqx, dqy, dqz, sc.gamma, sc.div_hi);
   trace_dir(q, D == 0 ? dqx : (D == 1 ? dqy : dqz), src, dtdx, sc.smallr, qp, qm);
 }
 
