@@ -68,19 +68,10 @@ def warm_device(torch, seconds=0.3):
     del x
 
 
-def time_variant(torch, ra, uin, flux, tmp, dt, riemann, precision, steps, warmup, tune=True, block=0):
-    from ramses_amd import autotune
+def time_variant(torch, ra, uin, flux, tmp, dt, riemann, precision, steps, warmup):
     ra.configure(gamma=GAMMA, riemann=riemann, slope_type=1, courant_factor=CFL, precision=precision)
     stream = torch.cuda.current_stream()
-    tuned = None
-    if precision == "fp32":  # nvector 32 runs the LDS-staged kernel: fixed 192-thread workgroups
-        tuned = (192, None)
-    elif not tune:
-        autotune._set(autotune.UNSPLIT_BLOCK, block)
-        tuned = (block or 256, None)
-    else:  # untimed: pick the workgroup size on these inputs
-        tuned = autotune.tune_unsplit(lambda: ra.unsplit_device(uin, None, flux, tmp, DX, dt, stream=stream),
-                                      key=("unsplit", uin.shape[0], precision, riemann))
+    tuned = (512, None)  # tiles of 16 octs: fixed 512-thread workgroups, nothing to tune
     # Untimed warm-up: at least `warmup` launches and at least WARM_S seconds.
     # The FP64 launches take tens of launches to settle (2.0 ms down to
     # 1.75-1.8 ms on the default workload; FP32 is flat), so a fixed short
@@ -561,7 +552,7 @@ def main():
     ap.add_argument("--load", default="1.2,0.8", help="serve: offered loads / measured capacity (comma list)")
     ap.add_argument("--steps-per-tick", type=int, default=8, help="serve: level steps per scheduler tick")
     ap.add_argument("--no-tune", action="store_true", help="use the shapes given below instead of autotuning")
-    ap.add_argument("--unsplit-block", type=int, default=0, help="with --no-tune: unsplit workgroup size")
+    ap.add_argument("--unsplit-block", type=int, default=0, help="without effect: the tiles have one workgroup size")
     ap.add_argument("--level-tile", type=int, default=0, help="with --no-tune: 1=32x8, 2=16x8, 3=8x8, 4=32x16, 5=16x12")
     ap.add_argument("--level-tz", type=int, default=0, help="with --no-tune: z planes per workgroup")
     ap.add_argument("--calibrate-copy", type=int, default=0,
@@ -608,8 +599,7 @@ def main():
     results = {}
     for v in args.variants.split(","):
         prec, riemann = v.split("-")
-        results[v] = time_variant(torch, ra, uin, flux, tmp, dt, riemann, prec, args.steps, args.warmup,
-                                  tune=not args.no_tune, block=args.unsplit_block)
+        results[v] = time_variant(torch, ra, uin, flux, tmp, dt, riemann, prec, args.steps, args.warmup)
     ra.configure()
 
     cells = 8 * noct

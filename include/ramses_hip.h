@@ -101,7 +101,7 @@ int ramses_unsplit_noalloc(const double *uin, const double *gravin, double *flux
  * (hydro/godunov_fine.f90:24-31) calling unsplit once per batch.  Enqueued
  * on `stream` (a hipStream_t; NULL = default stream), asynchronous.
  * gravin may be NULL (gravity zero, the same bits as a zero array): that
- * selects kernels with no gravity loads, 1.51 ms against 1.97 ms with a
+ * selects kernels with no gravity loads, 1.40 ms against 1.60 ms with a
  * zero array for 2^20 octs in FP64. */
 int ramses_unsplit_device(const double *uin, const double *gravin, double *flux, double *tmp, double dx,
                           double dy, double dz, double dt, long ngroups, int ngrid_last, void *stream);
@@ -405,12 +405,13 @@ int ramses_amr_mesh_release(ramses_amr_mesh *m);
  * tile shapes below, picked per device and workload by the autotuner
  * (ramses_amd/autotune.py).  value 0 restores the built-in default.
  * --------------------------------------------------------------------- */
-#define RAMSES_TUNE_UNSPLIT_BLOCK 1 /* threads per unsplit workgroup: multiple of 64, <= 768 */
+#define RAMSES_TUNE_UNSPLIT_BLOCK 1 /* threads per unsplit workgroup (27-point slopes): multiple of 64, <= 768 */
 #define RAMSES_TUNE_LEVEL_TILE 2    /* level tile: 1 = 32x8, 2 = 16x8, 3 = 8x8, 4 = 32x16, 5 = 16x12 columns */
 #define RAMSES_TUNE_LEVEL_TZ 3      /* z planes per level workgroup: a divisor of n, >= 4 */
 #define RAMSES_TUNE_PERSIST_BLOCKS 4 /* workgroups of a captured AMR step's fixed grids (0: 1024) */
-#define RAMSES_TUNE_AMR_FACE_OCTS 5  /* levels of at most this many octs run the AMR unsplit one face per
-                                        thread instead of one row per thread (0: 8192, -1: never) */
+#define RAMSES_TUNE_AMR_FACE_OCTS 5  /* levels of at most this many octs run the staged AMR unsplit (27-point
+                                        slopes, interpol_var 1 and 2) one face per thread instead of one row
+                                        per thread (0: 8192, -1: never) */
 
 /* Set one tuning knob (amr/amr_parameters.f90:49-53 is the reference's
  * counterpart); returns 0, or < 0 for an unknown knob or invalid value.

@@ -1,27 +1,32 @@
 // One level of an oct-tree (AMR) godunov sweep on the GPU:
-// godfine1 (hydro/godunov_fine.f90:486-911) split into four launches over
-// the level's active octs, all reading the tree (son / father / nbor) and
-// the state (uold / unew) resident in HBM in the reference's memory model:
-//   amr_gather   6x6x6 stencil of every oct in nvector-strided batches
-//                (get3cubefather/get3cubepos, amr/nbors_utils.f90:5-300; a
+// godfine1 (hydro/godunov_fine.f90:486-911) over the level's active octs, all
+// reading the tree (son / father / nbor) and the state (uold / unew) resident
+// in HBM in the reference's memory model:
+//   amr_tile     16 octs per workgroup: their 80-cell stencils gathered into
+//                LDS (get3cubefather/get3cubepos, amr/nbors_utils.f90:5-300; a
 //                missing neighbour oct is a buffer oct interpolated from its
 //                father's 7-point neighbourhood: getnborfather :404-525 and
-//                interpol_hydro, hydro/interpol_hydro.f90:268-637);
-//   amr_unsplit  unsplit of every batch (the device code of unsplit.hip),
-//                storing a zero flux at faces next to a refined cell
-//                (:720-749);
-//   amr_update   the level update unew += F(i) - F(i+1) (:751-792);
+//                interpol_hydro, hydro/interpol_hydro.f90:268-637), unsplit
+//                with a zero flux at faces next to a refined cell (:720-749),
+//                and the level update unew += F(i) - F(i+1) (:751-792);
 //   amr_reflux   the conservative correction of coarser leaf neighbours
 //                (:798-908), gathered per coarse cell and summed in the
 //                reference's order (batch, dimension, side, face) so the
 //                result is bitwise and deterministic without atomics.
+// The 27-point slopes and the prolongations of interpol_var 1 and 2 take the
+// staged form of amr_tile: amr_gather (6x6x6 stencils in nvector-strided
+// batches), amr_unsplit (the rows or faces of unsplit_device.hpp) and
+// amr_update.
 // Index conventions are the reference's (1-based cells and grids; arrays
 // are passed so that element i of the reference is p[i]).
+#include <type_traits>
+
 #include "hydro_device.hpp"
 #include "unsplit_args.hpp"
 #include "amr_args.hpp"
 #include "amr_device.hpp"
 #include "unsplit_device.hpp"
+#include "oct_tile.hpp"
 
 namespace ramses {
 hipError_t launch_cons_finish(const double* partials, long nblocks, double* out, int accumulate, hipStream_t s);
@@ -171,34 +176,228 @@ __global__ __launch_bounds__(256) void amr_update(AmrLevelArgs a) {
   }
 }
 
-// Minmod (the reference's default slope) with the limiter fixed at compile
-// time; other slope types take it at run time.
-template <typename R, int RS, bool S27>
-void launch_solve_t(const AmrLevelArgs& a, const UnsplitArgs& u, unsigned grid, unsigned block, hipStream_t s) {
-  if (!S27 && a.hp.slope_type == 1)
-    hipLaunchKernelGGL((amr_unsplit<R, RS, S27, 1>), dim3(grid), dim3(block), 0, s, a, u);
-  else
-    hipLaunchKernelGGL((amr_unsplit<R, RS, S27, -1>), dim3(grid), dim3(block), 0, s, a, u);
+// godfine1 of one level without its reflux, 16 octs per workgroup
+// (oct_tile.hpp): the stencil gather, the unsplit chain and the level update
+// in one kernel, the stencil and the fluxes in LDS.  Global memory sees the
+// tree, the state, the update, and the fluxes through the sides where the
+// neighbour oct is missing, which are all that amr_reflux reads.
+//
+// The separate kernels stage 13.4 KB per oct through memory: on a level of
+// 2^17 octs the gather took 0.40 ms, the solve 0.20 and the update 0.05; and
+// a level of a thousand octs paid three launches of 5 to 17 us.
+//
+// Gather: one (father neighbour, oct) task per thread, 27 x 16 of the 512.
+// The neighbours are ordered by how many of their cells a face depends on
+// (centre and sides 8, edges 2, corners none, which are only checked to
+// exist), so a wavefront loads alike.  The conserved state goes to LDS one
+// variable at a time, which keeps a task's prolongation in registers.
+// interpol_var 0 only: the other modes mix the variables.
+template <typename R, int RS, int ST>
+__global__ __launch_bounds__(oct_tile::kThreads)
+__attribute__((amdgpu_waves_per_eu(4, 8))) void amr_tile(AmrLevelArgs a, double dx, const double* d_dt) {
+  using namespace oct_tile;
+  // the conserved state of the 80 cells, then their primitives, then the
+  // traced states (R), then the fluxes
+  __shared__ double sd[kLds];
+  __shared__ unsigned char refined[kPairs];   // by slot and oct
+  __shared__ unsigned char missing[6][kOcts]; // by side
+  R* s = reinterpret_cast<R*>(sd);
+  const int noct = level_count(a.noct, a.dnoct);
+  const int ntiles = (noct + kOcts - 1) / kOcts;
+  const AmrTreeView& t = a.t;
+  const HydroParams hp = a.hp;
+  const double dt = *d_dt;
+  const SolverConsts<R> sc = make_consts<R>(hp);
+  const FluxScale fs = make_scale(dt, dx);
+  const double dtxhalf = dt * 0.5;
+  const double smalle = hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0);  // hydro/umuscl.f90:884
+  const R h = (R)(dt / dx);
+  const R dtdx[3] = {h, h, h};
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    // opaque to the compiler, which would otherwise carry the addresses of
+    // every step across the loop and spill them
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int l = tid % kOcts;
+    const int o = tile * kOcts + l;
+    const bool valid = o < noct;
+    const int igrid = a.active[valid ? o : noct - 1];
+    const int k27 = tid / kOcts;
+    if (k27 < 27) {
+      const int j = kTab.order[k27];
+      const int i1 = j % 3, j1 = (j / 3) % 3, k1 = j / 9;
+      const long nf = nbor_father_cell(t, t.father[igrid], i1, j1, k1, a.ilevel);
+      if (nf <= 0) atomicOr(a.error, 1);
+      if (nf > 0 && k27 < 19) {
+        const int gn = t.son[nf];
+        unsigned long long sub = kTab.sub[j];
+        if (k27 >= 1 && k27 < 7) {  // side 2*d + (plus side)
+          const int side = i1 != 1 ? (i1 >> 1) : (j1 != 1 ? 2 + (j1 >> 1) : 4 + (k1 >> 1));
+          missing[side][l] = gn <= 0;
+        }
+        if (gn > 0) {
+          if (k27 < 7) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) refined[(int)(sub >> 8 * i & 255) * kOcts + l] = t.son[cell_of(t, i + 1, gn)] > 0;
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+              double w[8];
+#pragma unroll
+              for (int i = 0; i < 8; ++i) w[i] = a.uold[(long)v * a.ustride + cell_of(t, i + 1, gn)];
+#pragma unroll
+              for (int i = 0; i < 8; ++i) sd[(int)(sub >> 8 * i & 255) * kCellStride + v * kOcts + l] = w[i];
+            }
+          } else {
+            // an edge neighbour's two cells on the oct's side of it
+            const int free_bit = i1 == 1 ? 1 : (j1 == 1 ? 2 : 4);
+            const int i0 = (i1 == 0 ? 1 : 0) + (j1 == 0 ? 2 : 0) + (k1 == 0 ? 4 : 0);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              const int i = i0 + (q ? free_bit : 0);
+              const long c = cell_of(t, i + 1, gn);
+              double* p = sd + (int)(sub >> 8 * i & 255) * kCellStride + l;
+              double w[5];
+#pragma unroll
+              for (int v = 0; v < 5; ++v) w[v] = a.uold[(long)v * a.ustride + c];
+#pragma unroll
+              for (int v = 0; v < 5; ++v) p[v * kOcts] = w[v];
+            }
+          }
+        } else {
+          long nb7[7];
+          nbor_father7(t, nf, a.ilevel, nb7);
+#pragma unroll 1
+          for (int v = 0; v < 5; ++v) {
+            double u7[7], u8[8];
+#pragma unroll
+            for (int q = 0; q < 7; ++q) u7[q] = a.uold[(long)v * a.ustride + nb7[q]];
+            interpol_cons(u7, u8, a.interpol_type);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const int slot = (int)(sub >> 8 * i & 255);
+              if (slot != 255) sd[slot * kCellStride + v * kOcts + l] = u8[i];
+            }
+          }
+          if (k27 < 7) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) refined[(int)(sub >> 8 * i & 255) * kOcts + l] = 0;
+          }
+        }
+      }
+    }
+    __syncthreads();
+    // In FP64 a cell's primitives go over its conserved state; FP32's
+    // packed ones go over other cells' state, after a barrier.
+    Prim<R> q[kLoads];
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+      const int e = tid + k * kThreads;
+      if (e < kPairs) {
+        const double* p = sd + (e / kOcts) * kCellStride + e % kOcts;
+        q[k] = ctoprim_cell<R>(p[0], p[kOcts], p[2 * kOcts], p[3 * kOcts], p[4 * kOcts], 0.0, 0.0, 0.0, dtxhalf,
+                               smalle, hp);
+        if constexpr (sizeof(R) == 8) put_prim(s, e, q[k]);
+      }
+    }
+    __syncthreads();
+    if constexpr (sizeof(R) == 4) {
+#pragma unroll
+      for (int k = 0; k < kLoads; ++k) {
+        const int e = tid + k * kThreads;
+        if (e < kPairs) put_prim(s, e, q[k]);
+      }
+      __syncthreads();
+    }
+    trace_tile<R, ST>(s, tid, sc, dtdx);
+    // fluxes, (f*dt)/dx in conserved order, zero next to a refined cell
+    // (hydro/godunov_fine.f90:720-749); each face's go over its own traced
+    // states, which only its wavefront reads
+    for (int k = 0; k < 2; ++k) {
+      const int f = tile_face(tid, k);
+      if (f < 0) continue;
+      const Face<R> fl = get_side(s, f, 0, l), fr = get_side(s, f, 1, l);
+      const Flux6<R> fg = riemann_fixed<R, RS>(fl, fr, sc);
+      const R val[5] = {fg.f[0], fg.f[1], fg.f[3], fg.f[4], fg.f[2]};
+      double out[5];
+      scale_flux<5>(val, fs, out);
+      if (refined[kTab.side[f][0] * kOcts + l] | refined[kTab.side[f][1] * kOcts + l]) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) out[v] = 0.0;
+      }
+      const int d = __builtin_amdgcn_readfirstlane(f) / 12, x = __builtin_amdgcn_readfirstlane(f) / 4 % 3;
+      const int m1 = 1 + d, m2 = d == 0 ? 2 : 1, m3 = d == 2 ? 2 : 3;  // the momenta in their own order
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the reads above stay above
+      double* p = reinterpret_cast<double*>(s + f * kFaceStride) + l;
+      p[0] = out[0];
+      p[m1 * kOcts] = out[1];
+      p[m2 * kOcts] = out[2];
+      p[m3 * kOcts] = out[3];
+      p[4 * kOcts] = out[4];
+      if (x != 1 && valid && missing[2 * d + (x >> 1)][l]) {
+        const size_t fvs = (size_t)a.nv * 27;
+        double* flux = a.flux + (size_t)(o / a.nv) * fvs * 15 + (size_t)(kTab.out[f] + 27 * 5 * d) * a.nv + o % a.nv;
+        flux[0] = out[0];
+        flux[m1 * fvs] = out[1];
+        flux[m2 * fvs] = out[2];
+        flux[m3 * fvs] = out[3];
+        flux[4 * fvs] = out[4];
+      }
+    }
+    __syncthreads();
+    // unew += flux(i) - flux(i+1) for x, y, z in order (:751-792): 8 cells x
+    // 5 variables x 16 octs
+    for (int e = tid; e < 40 * kOcts; e += kThreads) {
+      const int ind = e / (5 * kOcts), v = e / kOcts % 5;
+      const int x[3] = {ind & 1, (ind >> 1) & 1, ind >> 2};
+      if (valid) {
+        const long c = (long)v * a.ustride + cell_of(t, ind + 1, igrid);
+        double acc = a.unew[c];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const int T = d == 0 ? x[1] + 2 * x[2] : (d == 1 ? x[0] + 2 * x[2] : x[0] + 2 * x[1]);
+          const R* p = s + (12 * d + 4 * x[d] + T) * kFaceStride;
+          acc = acc + (reinterpret_cast<const double*>(p)[v * kOcts + l] -
+                       reinterpret_cast<const double*>(p + 4 * kFaceStride)[v * kOcts + l]);
+        }
+        a.unew[c] = acc;
+      }
+    }
+    __syncthreads();
+  }
 }
 
-template <typename R>
-void launch_solve_r(const AmrLevelArgs& a, const UnsplitArgs& u, unsigned grid, unsigned block, hipStream_t s) {
-  const bool s27 = a.hp.slope_type == 3;
-  switch (a.hp.riemann) {
-    case kHLLC:
-      s27 ? launch_solve_t<R, kHLLC, true>(a, u, grid, block, s) : launch_solve_t<R, kHLLC, false>(a, u, grid, block, s);
-      break;
-    case kHLL:
-      s27 ? launch_solve_t<R, kHLL, true>(a, u, grid, block, s) : launch_solve_t<R, kHLL, false>(a, u, grid, block, s);
-      break;
+// The solve of the staged path: the 27-point slopes, whose faces depend on
+// the whole 6^3 stencil, and prolongations that mix the variables (minmod
+// there too with the limiter fixed at compile time).
+template <typename R, int RS>
+void launch_solve(const AmrLevelArgs& a, const UnsplitArgs& u, unsigned grid, unsigned block, hipStream_t s) {
+  if (a.hp.slope_type == 3)
+    hipLaunchKernelGGL((amr_unsplit<R, RS, true, -1>), dim3(grid), dim3(block), 0, s, a, u);
+  else if (a.hp.slope_type == 1)
+    hipLaunchKernelGGL((amr_unsplit<R, RS, false, 1>), dim3(grid), dim3(block), 0, s, a, u);
+  else
+    hipLaunchKernelGGL((amr_unsplit<R, RS, false, -1>), dim3(grid), dim3(block), 0, s, a, u);
+}
+
+// Minmod (the reference's default slope) has the limiter fixed at compile
+// time; other slope types take it at run time.
+template <typename R, int RS>
+void launch_tile(const AmrLevelArgs& a, double dx, const double* d_dt, unsigned grid, hipStream_t s) {
+  if (a.hp.slope_type == 1)
+    hipLaunchKernelGGL((amr_tile<R, RS, 1>), dim3(grid), dim3(oct_tile::kThreads), 0, s, a, dx, d_dt);
+  else
+    hipLaunchKernelGGL((amr_tile<R, RS, -1>), dim3(grid), dim3(oct_tile::kThreads), 0, s, a, dx, d_dt);
+}
+
+// f(std::integral_constant<int, RS>) for the configured solver.
+template <typename F>
+void with_solver(int riemann, F f) {
+  switch (riemann) {
+    case kHLLC: f(std::integral_constant<int, kHLLC>{}); break;
+    case kHLL: f(std::integral_constant<int, kHLL>{}); break;
     case kACOUSTIC:
-    case kEXACT:
-      s27 ? launch_solve_t<R, kDynamicRiemann, true>(a, u, grid, block, s)
-          : launch_solve_t<R, kDynamicRiemann, false>(a, u, grid, block, s);
-      break;
-    default:
-      s27 ? launch_solve_t<R, kLLF, true>(a, u, grid, block, s) : launch_solve_t<R, kLLF, false>(a, u, grid, block, s);
-      break;
+    case kEXACT: f(std::integral_constant<int, kDynamicRiemann>{}); break;
+    default: f(std::integral_constant<int, kLLF>{}); break;
   }
 }
 
@@ -605,40 +804,51 @@ hipError_t launch_amr_godunov(const AmrLevelArgs& a, double dx, const double* d_
                               hipStream_t s) {
   const bool dev = a.dnoct != nullptr;
   if (!dev && a.noct <= 0) return hipSuccess;
-  const int nbatch = (a.noct + a.nv - 1) / a.nv;
-  const unsigned gblocks = (unsigned)(((long)nbatch * 27 * a.nv + 255) / 256);
-  hipLaunchKernelGGL(amr_gather, dim3(dev ? persist_blocks() : gblocks), dim3(256), 0, s, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  UnsplitArgs u;
-  u.uin = a.uin;
-  u.grav = nullptr;
-  u.flux = a.flux;
-  u.tmp = tmp;
-  u.dx[0] = u.dx[1] = u.dx[2] = dx;
-  u.dt = 0.0;
-  u.d_dt = d_dt;
-  u.ngroups = nbatch;
-  u.ngrid_last = a.noct - (nbatch - 1) * a.nv;
-  u.nv = a.nv;
-  u.hp = a.hp;
-  u.ok = a.ok;
-  u.face_octs = amr_face_octs();
-  const unsigned block = 128;
-  const long tasks = (long)nbatch * (a.noct <= u.face_octs ? 36 : 12) * a.nv;
-  // the fixed grids of the captured mode keep the 384 x persist_blocks()
-  // threads of one batch per 384-thread workgroup
-  const unsigned grid = dev ? 3 * persist_blocks() : (unsigned)((tasks + block - 1) / block);
-  if (fp32)
-    launch_solve_r<float>(a, u, grid, block, s);
-  else
-    launch_solve_r<double>(a, u, grid, block, s);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const unsigned ugrid = dev ? 2 * persist_blocks() : (unsigned)(((long)nbatch * 40 * a.nv + 255) / 256);
-  hipLaunchKernelGGL(amr_update, dim3(ugrid), dim3(256), 0, s, a);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  hipError_t e;
+  if (a.hp.slope_type != 3 && a.interpol_var == 0) {
+    const unsigned grid = dev ? persist_blocks() : (unsigned)((a.noct + oct_tile::kOcts - 1) / oct_tile::kOcts);
+    with_solver(a.hp.riemann, [&](auto rs) {
+      if (fp32)
+        launch_tile<float, decltype(rs)::value>(a, dx, d_dt, grid, s);
+      else
+        launch_tile<double, decltype(rs)::value>(a, dx, d_dt, grid, s);
+    });
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  } else {
+    const int nbatch = (a.noct + a.nv - 1) / a.nv;
+    const unsigned gblocks = (unsigned)(((long)nbatch * 27 * a.nv + 255) / 256);
+    hipLaunchKernelGGL(amr_gather, dim3(dev ? persist_blocks() : gblocks), dim3(256), 0, s, a);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    UnsplitArgs u;
+    u.uin = a.uin;
+    u.grav = nullptr;
+    u.flux = a.flux;
+    u.tmp = tmp;
+    u.dx[0] = u.dx[1] = u.dx[2] = dx;
+    u.dt = 0.0;
+    u.d_dt = d_dt;
+    u.ngroups = nbatch;
+    u.ngrid_last = a.noct - (nbatch - 1) * a.nv;
+    u.nv = a.nv;
+    u.hp = a.hp;
+    u.ok = a.ok;
+    u.face_octs = amr_face_octs();
+    const unsigned block = 128;
+    const long tasks = (long)nbatch * (a.noct <= u.face_octs ? 36 : 12) * a.nv;
+    // the fixed grids of the captured mode keep the 384 x persist_blocks()
+    // threads of one batch per 384-thread workgroup
+    const unsigned grid = dev ? 3 * persist_blocks() : (unsigned)((tasks + block - 1) / block);
+    with_solver(a.hp.riemann, [&](auto rs) {
+      if (fp32)
+        launch_solve<float, decltype(rs)::value>(a, u, grid, block, s);
+      else
+        launch_solve<double, decltype(rs)::value>(a, u, grid, block, s);
+    });
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const unsigned ugrid = dev ? 2 * persist_blocks() : (unsigned)(((long)nbatch * 40 * a.nv + 255) / 256);
+    hipLaunchKernelGGL(amr_update, dim3(ugrid), dim3(256), 0, s, a);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
   if (a.active_coarse && (a.dnoct_coarse || a.noct_coarse > 0)) {
     const long n = 40L * a.noct_coarse;
     hipLaunchKernelGGL(amr_reflux, dim3(cell_grid(n, a.dnoct_coarse)), dim3(256), 0, s, a);

@@ -191,6 +191,21 @@ __device__ inline void interpol_oct(double u1[7][5], double u2[8][5], int itype,
   }
 }
 
+// One variable of a buffer oct prolongated in conserved form (interpol_var
+// 0): its cell and six neighbours u7 -> the eight cells u8, exactly as
+// interpol_oct does with every variable (type 4 needs interpol_var 2).
+__device__ __forceinline__ void interpol_cons(const double u7[7], double u8[8], int itype) {
+  double w[3] = {0.0, 0.0, 0.0};
+  if (itype >= 1 && itype <= 3) interp_slopes(u7, itype, w);
+#pragma unroll
+  for (int ind = 0; ind < 8; ++ind) {
+    double s = u7[0];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) s = s + w[d] * ((double)((ind >> d) & 1) - 0.5);
+    u8[ind] = s;
+  }
+}
+
 // Cell `in` (1..6: -x,+x,-y,+y,-z,+z) next to cell ind of grid g at the same
 // level, or 0 where that neighbour grid does not exist: getnborgrids +
 // getnborcells (amr/nbors_utils.f90:530-555, 363-399).

@@ -492,10 +492,10 @@ __device__ __forceinline__ Flux6<R> riemann_hllc(const Face<R>& L, const Face<R>
   ecinr = ecinr + half * rr * (Rt.ut2 * Rt.ut2);
   const R etotr = er + ecinr;
   const R Ptotr = Pr;
-  R SL, SR, rcl, rcr, ustar, Ptotstar;
+  R SL = zero, SR = zero, rcl = zero, rcr = zero, ustar = zero, Ptotstar = zero;
   // the waves from the two sound speeds, and the numerators and the divisor
   // of the star velocity and pressure
-  R nu, np, den;
+  R nu = zero, np = zero, den = zero;
   auto waves = [&](R cfastl, R cfastr) {
     SL = fmin_f(ul, ur) - fmax_f(cfastl, cfastr);
     SR = fmax_f(ul, ur) + fmax_f(cfastl, cfastr);
@@ -535,6 +535,7 @@ __device__ __forceinline__ Flux6<R> riemann_hllc(const Face<R>& L, const Face<R>
     const R Pts = left ? Ptotl : Ptotr;
     const R dS = S - ustar;
     const R nr = rs * (S - us), ne = (S - us) * ets - Pts * us + Ptotstar * ustar, ni = es * (S - us);
+    ro = etoto = eo = zero;
     bool fulls = true;
     if constexpr (sizeof(R) == 8) {
       const double y = rcp_newton(dS);

@@ -1,6 +1,6 @@
-// Device code of the batched `unsplit` (hydro/umuscl.f90:22-171), shared by
-// unsplit.hip (the batched boundary kernel) and amr.hip (the fused
-// oct-tree level kernel).  See unsplit.hip for the work decomposition.
+// Device code of the batched `unsplit` (hydro/umuscl.f90:22-171) by rows or
+// single faces: unsplit.hip's 27-point slopes, and amr.hip's staged sweep.
+// See unsplit.hip for the work decomposition.
 #pragma once
 
 #include "hydro_device.hpp"
@@ -13,11 +13,10 @@ namespace unsplit_dev {
 __device__ __forceinline__ int cell6(int i, int j, int k) { return (i + 1) + 6 * ((j + 1) + 6 * (k + 1)); }
 
 // G: whether the call may have a gravity array.  The kernels without one
-// (G = false) carry no test of g, which frees registers (FP64 minmod rows:
-// 126 VGPRs against 162, four waves per SIMD instead of three); zero
-// acceleration enters ctoprim_cell either way, the same operations on the
-// same values.  With G the test stays: loading g unconditionally made the
-// FP64 kernels spill.
+// (G = false) carry no test of g, which frees registers; zero acceleration
+// enters ctoprim_cell either way, the same operations on the same values.
+// With G the test stays: loading g unconditionally made the FP64 kernels
+// spill.
 template <typename R, bool G>
 struct RowCtx {
   const double* u;     // group base + lane
@@ -121,10 +120,8 @@ __device__ __forceinline__ void store_face(double* flux, double* tmp, size_t fba
 // With ZR, ok points at the batch's refinement flags (+ lane) and a face
 // with a flagged cell on either side stores a zero flux: the value the
 // reference's reset leaves there (hydro/godunov_fine.f90:720-749).
-// Ctx supplies prim(i,j,k) and nv: RowCtx evaluates the primitives from
-// uin, and the staged kernel of unsplit.hip reads them from LDS (the 27-point
-// slopes need RowCtx).  ST: the 7-point slope type fixed at compile time, or
-// -1 (see slope1).
+// Ctx supplies prim(i,j,k) and nv (RowCtx).  ST: the 7-point slope type
+// fixed at compile time, or -1 (see slope1).
 template <typename R, int D, int RS, bool S27, bool ZR, int ST, typename Ctx>
 __device__ __forceinline__ void row_faces(const Ctx& c, const SolverConsts<R>& sc, int a1, int b1,
                                           R dtdx, double* flux, double* tmp, size_t fvs, const FluxScale fs,
