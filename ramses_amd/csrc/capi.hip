@@ -31,6 +31,7 @@ hipError_t launch_uniform_godunov(const double* u, double* unew, int n, double d
                                   double* partials = nullptr, double* d_sums = nullptr);
 hipError_t launch_level_batch(double* const* buf0, double* const* buf1, double* const* state, const int* n,
                               const double* dx, int nslots, const HydroParams& hp, bool fp32, hipStream_t s);
+long level_batch_blocks(const int* n, int nslots);
 hipError_t launch_init_slot(double* state, double t_end, double start, hipStream_t s);
 hipError_t launch_amr_godunov(const AmrLevelArgs& a, double dx, const double* d_dt, double* tmp, bool fp32,
                               hipStream_t s);
@@ -1138,7 +1139,6 @@ int ramses_level_batch_step(const ramses_level_slot* slots, int nslots, void* st
   double* st[RAMSES_MAX_SLOTS];
   int n[RAMSES_MAX_SLOTS];
   double dx[RAMSES_MAX_SLOTS];
-  long blocks = 0;
   for (int i = 0; i < nslots; ++i) {
     const ramses_level_slot& s = slots[i];
     if (!s.buf[0] || !s.buf[1] || !s.state) return fail(-1, "null slot pointer");
@@ -1148,10 +1148,8 @@ int ramses_level_batch_step(const ramses_level_slot* slots, int nslots, void* st
     st[i] = s.state;
     n[i] = s.n;
     dx[i] = s.dx;
-    const int tz = ramses::batch_tz(s.n);
-    blocks += (long)(s.n / 16) * (s.n / 8) * (s.n / tz);
   }
-  if (blocks > 2147483647L) return fail(-1, "batch too large");
+  if (ramses::level_batch_blocks(n, nslots) > 2147483647L) return fail(-1, "batch too large");
   hipError_t e = ramses::launch_level_batch(b0, b1, st, n, dx, nslots, c.hp, c.precision == RAMSES_FP32_MIXED,
                                            (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "level batch launch");

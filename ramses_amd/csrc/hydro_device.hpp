@@ -59,6 +59,17 @@ inline unsigned persist_blocks() { return tuning().persist_blocks > 0 ? (unsigne
 // Levels of at most this many octs run the AMR unsplit one face per thread.
 inline int amr_face_octs() { return tuning().amr_face_octs > 0 ? tuning().amr_face_octs : (tuning().amr_face_octs < 0 ? 0 : 8192); }
 
+// The dispatcher hands workgroup b to XCD b % 8, and each XCD has its own
+// L2.  Workgroup b is given the logical index that makes every XCD run one
+// contiguous range of logical workgroups (a bijection of [0, G)), so
+// workgroups that share cells or cache lines run on the same XCD and find
+// them in its L2.
+__device__ __forceinline__ unsigned xcd_contiguous(unsigned b, unsigned G) {
+  constexpr unsigned X = 8;
+  const unsigned x = b % X, q = G / X, r = G % X;
+  return x * q + (x < r ? x : r) + b / X;
+}
+
 // Fortran MAX/MIN of two reals.  The hardware min/max (IEEE maxNum/minNum)
 // returns the same value as the reference for every non-NaN pair; the only
 // possible difference, the sign of a zero result when +0 and -0 tie, cannot
@@ -949,10 +960,6 @@ __device__ __forceinline__ void cons_block_store(ConsSums s, double* partials, l
     partials[3 * block + 2] = ei;
   }
 }
-
-// z planes per workgroup of a batched level slot (n a multiple of 16): a
-// divisor of n, at most 32.
-__host__ __device__ inline int batch_tz(int n) { return n <= 32 ? n : (n % 32 == 0 ? 32 : 16); }
 
 // Positive doubles order like their bit patterns, so a min-reduction of dt
 // can use an integer atomic.

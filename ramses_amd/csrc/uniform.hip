@@ -71,7 +71,10 @@ constexpr int tile_threads() { return (TX * TY + 2 * (TX + TY) + 63) / 64 * 64; 
 
 // One workgroup's tile of a level: columns [x0, x0+TX) x [y0, y0+TY),
 // planes [z0, z0+TZ).  Shared by the single-level and the batched kernels.
-// ST: the slope type fixed at compile time, or -1 (see slope1).
+// A tile may reach past the level's last column or row (n >= TX, TY): the
+// periodic wrap makes the threads there repeat cells of the other side, and
+// they store nothing.  ST: the slope type fixed at compile time, or -1 (see
+// slope1).
 template <typename R, int TX, int TY, int RS, bool SUMS = false, int ST = -1>
 __device__ __forceinline__ void level_tile(const double* __restrict__ u, double* __restrict__ unew, int n, double dx,
                                            double dt, double* d_dt_next, const HydroParams& hp, int x0, int y0,
@@ -122,6 +125,25 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
   const int e = ey * EX + ex;  // own slot in the exchange area
   const int xg = wrapi(x0 - 1 + ex, n), yg = wrapi(y0 - 1 + ey, n);
   const int qo = (ey + 1) * QX + (ex + 1);  // own cell in the primitive plane
+  const bool inside = x0 + ex <= n && y0 + ey <= n;  // (interior threads) the cell is not a repeated one
+
+  // A plane of one variable is addressed from a scalar base by a 32-bit byte
+  // offset that a thread keeps for the whole march (its own cell, and the
+  // one or two cells it converts to primitives), so that a load or store
+  // takes no vector instruction for its address.
+  auto at = [&](const double* base, unsigned off) {
+    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off);
+  };
+  const unsigned own = 8u * (unsigned)(yg * n + xg);
+  // cell t for every thread; the cells beyond NT go to the last threads (the
+  // ring's wave, which solves fewer faces), in reverse order
+  static_assert(NQ <= 2 * NT, "a plane is at most two cells per thread");
+  unsigned ld[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int c = k == 0 ? t : 2 * NT - 1 - t;
+    ld[k] = 8u * (unsigned)(wrapi(y0 - 2 + c / QX, n) * n + wrapi(x0 - 2 + c % QX, n));
+  }
 
   const SolverConsts<R> sc = make_consts<R>(hp);
   const double dtxhalf = dt * 0.5;
@@ -131,18 +153,14 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
 
   // cooperative ctoprim of plane zp (periodic) into slot s
   auto load_plane = [&](int zp, int s) {
-    const int zg = wrapi(zp, n);
-    static_assert(NQ <= 2 * NT, "a plane is at most two cells per thread");
-    // cell t for every thread; the cells beyond NT go to the last threads
-    // (the ring's wave, which solves fewer faces), in reverse order
+    const double* up = u + (long)wrapi(zp, n) * plane;
+#pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int c = k == 0 ? t : 2 * NT - 1 - t;
       if (c >= NQ) continue;
-      const int qx = c % QX, qy = c / QX;
-      const int gx = wrapi(x0 - 2 + qx, n), gy = wrapi(y0 - 2 + qy, n);
-      const long o = (long)zg * plane + (long)gy * n + gx;
-      const Prim<R> q = ctoprim_cell<R>(u[o], u[o + vstride], u[o + 2 * vstride], u[o + 3 * vstride],
-                                        u[o + 4 * vstride], 0.0, 0.0, 0.0, dtxhalf, smalle, hp);
+      const Prim<R> q = ctoprim_cell<R>(at(up, ld[k]), at(up + vstride, ld[k]), at(up + 2 * vstride, ld[k]),
+                                        at(up + 3 * vstride, ld[k]), at(up + 4 * vstride, ld[k]), 0.0, 0.0, 0.0,
+                                        dtxhalf, smalle, hp);
       qs[s][0][c] = q.r;
       qs[s][1][c] = q.u;
       qs[s][2][c] = q.v;
@@ -193,9 +211,9 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
     double upre[5] = {0, 0, 0, 0, 0};
     if constexpr (sizeof(R) == 4) {
       if (interior && faces_xy) {
-        const long o = (long)wrapi(p, n) * plane + (long)yg * n + xg;
+        const double* up = u + (long)wrapi(p, n) * plane;
 #pragma unroll
-        for (int v = 0; v < 5; ++v) upre[v] = u[o + v * vstride];
+        for (int v = 0; v < 5; ++v) upre[v] = at(up + v * vstride, own);
       }
     }
     __syncthreads();
@@ -268,10 +286,10 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
         __syncthreads();
         if (interior) {
           // hydro/godunov_fine.f90:770-772: unew = uold + (flux(i) - flux(i+1)), idim=1 then 2
-          const long o = (long)wrapi(p, n) * plane + (long)yg * n + xg;
+          const double* up = u + (long)wrapi(p, n) * plane;
 #pragma unroll
           for (int v = 0; v < 5; ++v)
-            part[v] = u[o + v * vstride] + (fx_sh[v * FSTRIDE + e] - fx_sh[v * FSTRIDE + e + 1]);
+            part[v] = at(up + v * vstride, own) + (fx_sh[v * FSTRIDE + e] - fx_sh[v * FSTRIDE + e + 1]);
 #pragma unroll
           for (int v = 0; v < 5; ++v) part[v] = part[v] + (fy_sh[v * FSTRIDE + e] - fy_sh[v * FSTRIDE + e + EX]);
         }
@@ -308,20 +326,20 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
     }
     // plane p-1 is complete: hydro/godunov_fine.f90:751-792 in idim order x, y, z
     if (interior && p >= z0 + 1) {
-      const int zg = wrapi(p - 1, n);
-      const long o = (long)zg * plane + (long)yg * n + xg;
       double un[5];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const double s = part_prev[v] + (fz_prev[v] - fz[v]);  // idim=3
-        un[v] = s;
-        unew[o + v * vstride] = s;
+      for (int v = 0; v < 5; ++v) un[v] = part_prev[v] + (fz_prev[v] - fz[v]);  // idim=3
+      if (inside) {
+        double* np = unew + (long)(p - 1) * plane;
+#pragma unroll
+        for (int v = 0; v < 5; ++v)
+          *reinterpret_cast<double*>(reinterpret_cast<char*>(np + v * vstride) + own) = un[v];
       }
       if (d_dt_next) {
         if constexpr (sizeof(R) == 8) wmax = fmax_f(wmax, cmpdt_w(un[0], un[1], un[2], un[3], un[4], hp));
         else wmax = fmax_f(wmax, cmpdt_w_fast(un[0], un[1], un[2], un[3], un[4], hp));
       }
-      if constexpr (SUMS) cons_add(cs, un[0], un[1], un[2], un[3], un[4], vol, hp.smallr);
+      if (SUMS && inside) cons_add(cs, un[0], un[1], un[2], un[3], un[4], vol, hp.smallr);
     }
     // carry to the next plane
     fz_left = rotate(qm_z, 2);
@@ -371,24 +389,17 @@ template <typename R, int TX, int TY, int RS, bool SUMS, int ST>
 // The register budget: 3 waves per SIMD in FP64 (166 VGPRs), 4 in FP32-mixed
 // (at most 128).
 __global__ __launch_bounds__((tile_threads<TX, TY>()))
-__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3, 8))) void uniform_godunov_kernel(UniformArgs a, int TZ,
-                                                                                           int y0, int boff) {
-  // XCD-aware tile order: the hardware deals workgroups round-robin to the
-  // 8 XCDs, so workgroup b runs on XCD b%8.  Giving each XCD a contiguous
-  // range of tiles (x fastest, then y, then z chunk) keeps the tiles that run
-  // side by side on one XCD spatial neighbours, and their shared halo
-  // columns are served by that XCD's L2 instead of HBM.  The launch covers
-  // rows [y0, y0 + TY * gridDim.y); its workgroups' courant sums go to
-  // partials[boff + block].
-  const int ntx = gridDim.x, nty = gridDim.y;
-  const int nb = ntx * nty * gridDim.z;
-  const int b = blockIdx.x + ntx * (blockIdx.y + nty * blockIdx.z);
-  const int per_xcd = (nb + 7) / 8;
-  int logical = (b & 7) * per_xcd + (b >> 3);
-  if ((nb & 7) != 0) logical = b;  // ragged grids keep the plain order
-  const int tx = logical % ntx, ty = (logical / ntx) % nty, tzc = logical / (ntx * nty);
-  level_tile<R, TX, TY, RS, SUMS, ST>(a.u, a.unew, a.n, a.dx, *a.d_dt, a.d_dt_next, a.hp, tx * TX, y0 + ty * TY,
-                                  tzc * TZ, TZ, a.partials, boff + b);
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3, 8))) void uniform_godunov_kernel(UniformArgs a, int ntx,
+                                                                                           int nty, int TZ) {
+  // Workgroup b runs on XCD b % 8 (the hardware deals them out in turn).
+  // Giving each XCD a contiguous range of tiles (x fastest, then y, then z
+  // chunk; xcd_contiguous) keeps the tiles that run side by side on one XCD
+  // spatial neighbours, and their shared halo columns are served by that
+  // XCD's L2 instead of HBM.  The last chunk may be shorter.
+  const int logical = (int)xcd_contiguous(blockIdx.x, gridDim.x);
+  const int tx = logical % ntx, ty = (logical / ntx) % nty, z0 = logical / (ntx * nty) * TZ;
+  level_tile<R, TX, TY, RS, SUMS, ST>(a.u, a.unew, a.n, a.dx, *a.d_dt, a.d_dt_next, a.hp, tx * TX, ty * TY, z0,
+                                     min(TZ, a.n - z0), a.partials, blockIdx.x);
 }
 
 // Many independent levels advanced by one launch (continuous batching).
@@ -407,11 +418,11 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3, 8))) void batch_godun
   const double* u = sl.buf[par];
   double* unew = sl.buf[par ^ 1];
   const int n = sl.n;
-  const int ntx = n / TX, nty = n / TY;
+  const int ntx = (n + TX - 1) / TX, nty = (n + TY - 1) / TY;
   const int local = b - a.blk0[s];
-  const int tx = local % ntx, ty = (local / ntx) % nty, tzc = local / (ntx * nty);
-  level_tile<R, TX, TY, RS, false, ST>(u, unew, n, sl.dx, st[kDtUse], st + kDtNext, a.hp, tx * TX, ty * TY,
-                                      tzc * sl.tz, sl.tz);
+  const int tx = local % ntx, ty = (local / ntx) % nty, z0 = local / (ntx * nty) * sl.tz;
+  level_tile<R, TX, TY, RS, false, ST>(u, unew, n, sl.dx, st[kDtUse], st + kDtNext, a.hp, tx * TX, ty * TY, z0,
+                                      min(sl.tz, n - z0));
 }
 
 // Per-slot bookkeeping before each batched step (one thread per slot):
@@ -543,84 +554,119 @@ __global__ void cmpdt_group(const double* uu, const double* gg, int nv, int ncel
   }
 }
 
-// Tiles of rows [y0, y0 + ny), ny a multiple of TY; returns the number of
-// workgroups launched.
 template <typename R, int TX, int TY, bool SUMS, int ST>
-long launch_band_st(const UniformArgs& a, int TZ, int y0, int ny, int boff, hipStream_t s) {
-  constexpr int NT = tile_threads<TX, TY>();
-  const dim3 grid(a.n / TX, ny / TY, a.n / TZ);
+void launch_tile_st(const UniformArgs& a, int ntx, int nty, int TZ, dim3 grid, hipStream_t s) {
+  const dim3 block(tile_threads<TX, TY>());
   switch (a.hp.riemann) {
     case kHLLC:
-      hipLaunchKernelGGL((uniform_godunov_kernel<R, TX, TY, kHLLC, SUMS, ST>), grid, dim3(NT), 0, s, a, TZ, y0, boff);
+      hipLaunchKernelGGL((uniform_godunov_kernel<R, TX, TY, kHLLC, SUMS, ST>), grid, block, 0, s, a, ntx, nty, TZ);
       break;
     case kHLL:
-      hipLaunchKernelGGL((uniform_godunov_kernel<R, TX, TY, kHLL, SUMS, ST>), grid, dim3(NT), 0, s, a, TZ, y0, boff);
+      hipLaunchKernelGGL((uniform_godunov_kernel<R, TX, TY, kHLL, SUMS, ST>), grid, block, 0, s, a, ntx, nty, TZ);
       break;
     case kACOUSTIC:
     case kEXACT:
-      hipLaunchKernelGGL((uniform_godunov_kernel<R, TX, TY, kDynamicRiemann, SUMS, ST>), grid, dim3(NT), 0, s, a, TZ,
-                         y0, boff);
+      hipLaunchKernelGGL((uniform_godunov_kernel<R, TX, TY, kDynamicRiemann, SUMS, ST>), grid, block, 0, s, a, ntx, nty,
+                         TZ);
       break;
     default:
-      hipLaunchKernelGGL((uniform_godunov_kernel<R, TX, TY, kLLF, SUMS, ST>), grid, dim3(NT), 0, s, a, TZ, y0, boff);
+      hipLaunchKernelGGL((uniform_godunov_kernel<R, TX, TY, kLLF, SUMS, ST>), grid, block, 0, s, a, ntx, nty, TZ);
       break;
   }
-  return (long)grid.x * grid.y * grid.z;
 }
 
-// Minmod, the reference's default slope (hydro/hydro_parameters.f90:76),
-// has kernels of its own with the limiter fixed at compile time: without
-// the branches on the slope type the compiler schedules the traces across
-// what were separate blocks, which measured 8% faster at 512^3 in both
-// precisions.  Other slope types take it at run time.
-template <typename R, int TX, int TY, bool SUMS>
-long launch_band(const UniformArgs& a, int TZ, int y0, int ny, int boff, hipStream_t s) {
-  return a.hp.slope_type == 1 ? launch_band_st<R, TX, TY, SUMS, 1>(a, TZ, y0, ny, boff, s)
-                              : launch_band_st<R, TX, TY, SUMS, -1>(a, TZ, y0, ny, boff, s);
-}
-
-// Rows [0, ny12) in 16x12 tiles, the rest in 16x8 tiles: ny12 is the
-// largest multiple of 12 that leaves a multiple of 8, or -1 if there is
-// none (n must be a multiple of 16).
-inline int rows_in_16x12(int n) {
-  for (int ny = n / 12 * 12; ny >= 12; ny -= 12)
-    if ((n - ny) % 8 == 0) return ny;
-  return -1;
-}
-
-// Launch the level kernel (16x12 tiles: two bands, see rows_in_16x12); with
-// sums, then add the workgroups' conservation sums into d_sums[0..2] in
-// block order.
-template <typename R, int TX, int TY, bool SUMS>
-hipError_t launch_tile_s(const UniformArgs& a, int TZ, double* d_sums, hipStream_t s) {
-  long nblocks;
-  if constexpr (TY == 12) {
-    const int ny = rows_in_16x12(a.n);
-    nblocks = launch_band<R, 16, 12, SUMS>(a, TZ, 0, ny, 0, s);
-    if (ny < a.n) nblocks += launch_band<R, 16, 8, SUMS>(a, TZ, ny, a.n - ny, (int)nblocks, s);
+// Launch the level kernel; with sums, then add the workgroups' conservation
+// sums into d_sums[0..2] in block order.  Minmod, the reference's default
+// slope (hydro/hydro_parameters.f90:76), has kernels of its own with the
+// limiter fixed at compile time; other slope types take it at run time.
+template <typename R, int TX, int TY>
+hipError_t launch_tile(const UniformArgs& a, int TZ, double* d_sums, hipStream_t s) {
+  const int ntx = (a.n + TX - 1) / TX, nty = (a.n + TY - 1) / TY;
+  const dim3 grid((unsigned)(ntx * nty * ((a.n + TZ - 1) / TZ)));
+  const bool st1 = a.hp.slope_type == 1;
+  if (a.partials) {
+    st1 ? launch_tile_st<R, TX, TY, true, 1>(a, ntx, nty, TZ, grid, s)
+        : launch_tile_st<R, TX, TY, true, -1>(a, ntx, nty, TZ, grid, s);
+    hipLaunchKernelGGL(cons_finish, dim3(1), dim3(256), 0, s, (const double*)a.partials, (long)grid.x, d_sums, 0);
   } else {
-    nblocks = launch_band<R, TX, TY, SUMS>(a, TZ, 0, a.n, 0, s);
+    st1 ? launch_tile_st<R, TX, TY, false, 1>(a, ntx, nty, TZ, grid, s)
+        : launch_tile_st<R, TX, TY, false, -1>(a, ntx, nty, TZ, grid, s);
   }
-  if constexpr (SUMS)
-    hipLaunchKernelGGL(cons_finish, dim3(1), dim3(256), 0, s, (const double*)a.partials, nblocks, d_sums, 0);
   return hipGetLastError();
 }
 
-template <typename R, int TX, int TY>
-hipError_t launch_tile(const UniformArgs& a, int TZ, double* d_sums, hipStream_t s) {
-  return a.partials ? launch_tile_s<R, TX, TY, true>(a, TZ, d_sums, s) : launch_tile_s<R, TX, TY, false>(a, TZ, d_sums, s);
+// Time estimate of W workgroups of TZ planes on the 256 CUs, in us: m of
+// them on the fullest CU, TZ + 2 planes each (two are marched for their
+// traced states only).  A CU takes its m workgroups' planes side by side
+// while they fit, then one after the other at full throughput.  The plane
+// times are those measured with 16x12 tiles (hllc, minmod): one workgroup
+// alone 3.9 us a plane in FP64 and 3.1 in FP32-mixed, three FP64 ones 7.2,
+// four FP32-mixed ones 5.6.  The estimate is within 10% of the measured time
+// for n = 16..512 and z chunks of 2..128 planes.
+inline double level_estimate(long W, int TZ, bool fp32) {
+  const double m = (double)((W + 255) / 256);
+  const double plane = fp32 ? (m <= 4 ? 2.3 + 0.82 * m : 1.48 * m) : (m <= 3 ? 2.2 + 1.7 * m : 2.4 * m);
+  return (TZ + 2) * plane;
 }
+
+// The z chunk with the least estimate, at least 2 planes and at most
+// max_blocks workgroups.  Long chunks repeat fewer planes, short ones fill
+// the chip: 2 planes at n <= 64, 6 at 96, 16 at 128, 32 at 256 and 64 at 512
+// in FP64 (with max_blocks out of the way), the fastest or within 3% of it
+// among those measured.
+inline int best_tz(int n, long tiles, bool fp32, long max_blocks) {
+  int best = n;
+  double least = 1e300;
+  for (int tz = n < 2 ? n : 2; tz <= n; ++tz) {
+    const long W = tiles * ((n + tz - 1) / tz);
+    if (W > max_blocks && tz < n) continue;
+    const double t = level_estimate(W, tz, fp32);
+    if (t < least) {
+      least = t;
+      best = tz;
+    }
+  }
+  return best;
+}
+
+constexpr int kBatchTX = 16, kBatchTY = 12;
+inline long batch_tiles(int n) { return (long)((n + kBatchTX - 1) / kBatchTX) * ((n + kBatchTY - 1) / kBatchTY); }
 
 template <typename R, int RS>
 void launch_batch_t(const BatchArgs& a, int nblocks, hipStream_t s) {
-  constexpr int TX = 16, TY = 8, NT = tile_threads<TX, TY>();
-  if (a.hp.slope_type == 1)  // minmod: see launch_band
+  constexpr int TX = kBatchTX, TY = kBatchTY, NT = tile_threads<TX, TY>();
+  if (a.hp.slope_type == 1)  // minmod: see launch_tile
     hipLaunchKernelGGL((batch_godunov_kernel<R, TX, TY, RS, 1>), dim3(nblocks), dim3(NT), 0, s, a);
   else
     hipLaunchKernelGGL((batch_godunov_kernel<R, TX, TY, RS, -1>), dim3(nblocks), dim3(NT), 0, s, a);
 }
 
 }  // namespace
+
+// One z chunk for every slot of a batch: the least estimate for all their
+// workgroups together (a slot that is done exits at once and is not known
+// here).
+static int batch_tz(const int* n, int nslots, bool fp32) {
+  int best = 32;
+  double least = 1e300;
+  for (int tz : {2, 4, 6, 8, 12, 16, 24, 32}) {
+    long W = 0;
+    for (int i = 0; i < nslots; ++i) W += batch_tiles(n[i]) * ((n[i] + tz - 1) / tz);
+    const double t = level_estimate(W, tz, fp32);
+    if (t < least) {
+      least = t;
+      best = tz;
+    }
+  }
+  return best;
+}
+
+// The workgroups of a batch at its shortest z chunk.
+long level_batch_blocks(const int* n, int nslots) {
+  long W = 0;
+  for (int i = 0; i < nslots; ++i) W += batch_tiles(n[i]) * ((n[i] + 1) / 2);
+  return W;
+}
 
 // Continuous batching: one bookkeeping launch and one update launch advance
 // every slot of `slots` by one step of its own dt.
@@ -629,6 +675,7 @@ hipError_t launch_level_batch(double* const* buf0, double* const* buf1, double* 
   BatchArgs a{};
   a.nslots = nslots;
   a.hp = hp;
+  const int tz = batch_tz(n, nslots, fp32);
   int blocks = 0;
   for (int i = 0; i < nslots; ++i) {
     BatchSlot& sl = a.slot[i];
@@ -637,9 +684,9 @@ hipError_t launch_level_batch(double* const* buf0, double* const* buf1, double* 
     sl.state = state[i];
     sl.n = n[i];
     sl.dx = dx[i];
-    sl.tz = batch_tz(n[i]);
+    sl.tz = tz;
     a.blk0[i] = blocks;
-    blocks += (n[i] / 16) * (n[i] / 8) * (n[i] / sl.tz);
+    blocks += (int)(batch_tiles(n[i]) * ((n[i] + tz - 1) / tz));
   }
   a.blk0[nslots] = blocks;
   hipLaunchKernelGGL(batch_advance_kernel, dim3(1), dim3(64), 0, s, a);
@@ -697,37 +744,33 @@ hipError_t launch_courant(const double* u, int n, double dx, const HydroParams& 
   return hipGetLastError();
 }
 
-// Workgroups of the largest level launch (8x8 tiles of 4 planes; the
-// courant reduction uses at most as many), 3 doubles of sums each.
-size_t uniform_sums_work_bytes(int n) {
+// Workgroups of the largest level launch with sums (8x8 tiles of 4 planes;
+// the courant reduction uses at most as many), 3 doubles each.
+long sums_blocks(int n) {
   const long blocks = (long)n * n * n / 256;
-  return (size_t)(blocks > 1 ? blocks : 1) * 3 * sizeof(double);
+  return blocks > 1 ? blocks : 1;
 }
+size_t uniform_sums_work_bytes(int n) { return (size_t)sums_blocks(n) * 3 * sizeof(double); }
 
-// Tile choice: the launch-shape knob when it fits n, else 16x12 where n
-// allows it (three interior waves and one ring wave: the ring's work is a
-// third of a tile's, against a half for 16x8), else the largest tile
-// dividing n; and a z chunk that leaves enough workgroups to fill the chip.
+// Tile choice: the launch-shape knob when it divides n, else 16x12 (three
+// interior waves and one ring wave: the ring's work is a third of a tile's,
+// against a half for 16x8), whose last tiles may reach past the level, or
+// 16x8 for n <= 24, where a third of a 16x12 tile's rows would.
 hipError_t launch_uniform_godunov(const double* u, double* unew, int n, double dx, const double* d_dt,
                                   double* d_dt_next, const HydroParams& hp, bool fp32, hipStream_t s,
                                   double* partials, double* d_sums) {
   UniformArgs a{u, unew, d_dt, d_dt_next, partials, n, dx, hp};
-  int TX, TY;
+  int TX = 16, TY = 12;
   const int tile = tuning().level_tile;
-  const bool fits12 = n % 16 == 0 && rows_in_16x12(n) > 0;
   if (tile == 1 && n % 32 == 0) { TX = 32; TY = 8; }
-  else if (tile == 2 && n % 16 == 0) { TX = 16; TY = 8; }
-  else if (tile == 3) { TX = 8; TY = 8; }
+  else if (tile == 3 || n < 16) { TX = 8; TY = 8; }
   else if (tile == 4 && n % 32 == 0) { TX = 32; TY = 16; }
-  else if (fits12) { TX = 16; TY = 12; }  // tile 5, and the default
-  else if (n % 32 == 0) { TX = 32; TY = 8; }
-  else if (n % 16 == 0) { TX = 16; TY = 8; }
-  else { TX = 8; TY = 8; }
-  const long tiles = (long)(n / TX) * (n / TY);
-  int TZ = n;
-  while (TZ > 4 && TZ % 2 == 0 && tiles * (n / TZ) < 2048) TZ /= 2;
-  const int tz = tuning().level_tz;
-  if (tz >= 4 && tz <= n && n % tz == 0) TZ = tz;
+  else if ((tile == 2 && n % 16 == 0) || (tile == 0 && n <= 24)) { TX = 16; TY = 8; }
+  const long tiles = (long)((n + TX - 1) / TX) * ((n + TY - 1) / TY);
+  // with sums, three doubles per workgroup have to fit the caller's buffer
+  const long max_blocks = partials ? sums_blocks(n) : 0x7fffffffL;
+  int TZ = tuning().level_tz;
+  if (TZ < 4 || TZ > n || n % TZ != 0 || tiles * (n / TZ) > max_blocks) TZ = best_tz(n, tiles, fp32, max_blocks);
   if (fp32) {
     if (TY == 12) return launch_tile<float, 16, 12>(a, TZ, d_sums, s);
     if (TX == 32 && TY == 16) return launch_tile<float, 32, 16>(a, TZ, d_sums, s);

@@ -36,17 +36,6 @@ namespace {
 
 using unsplit_dev::unsplit_task;
 
-// The dispatcher hands workgroup b to XCD b % 8, and each XCD has its own
-// L2.  Workgroup b is given the logical index that makes every XCD run one
-// contiguous range of logical workgroups (a bijection of [0, G)), so the
-// workgroups that share a batch's cells or their cache lines run on the same
-// XCD and find them in its L2.
-__device__ __forceinline__ unsigned xcd_contiguous(unsigned b, unsigned G) {
-  constexpr unsigned X = 8;
-  const unsigned x = b % X, q = G / X, r = G % X;
-  return x * q + (x < r ? x : r) + b / X;
-}
-
 // One thread per (group, row, lane) task of the 27-point slopes; G: a.grav is
 // non-null.
 template <typename R, int RS, bool G>
