@@ -401,24 +401,19 @@ void with_solver(int riemann, F f) {
   }
 }
 
+constexpr unsigned kRefluxSplit = 1u << 16;
+__host__ __device__ inline bool reflux_from_coarse(unsigned nf, unsigned nc) { return 8ULL * nc <= 6ULL * nf; }
+
 // Conservative correction of the coarser leaf cells next to the level's
-// octs.  Thread = (one cell of a coarse-level oct, one variable): the tree
-// walk is repeated per variable, which keeps five times more threads in
-// flight on the small coarse levels where this kernel is latency-bound.  A
-// coarse leaf c receives from each fine oct o that sits across one of its
-// faces the four (reset) fluxes of o's boundary faces on c's side, times
-// -1/8 (c left of o) or +1/8 (c right of o).  The reference adds them in
-// loop order: batch of o, then dimension, then side, then face (k3, j3, i3);
-// the same order is rebuilt here from the position of o in the level's
-// active list.
-__device__ __forceinline__ void reflux_task(const AmrLevelArgs& a, long tix) {
-  const long cidx = tix / 5;
-  const int v = (int)(tix % 5);
+// octs.  A coarse leaf c receives from each fine oct o that sits across one
+// of its faces the four (reset) fluxes of o's boundary faces on c's side,
+// times -1/8 (c left of o) or +1/8 (c right of o).  The reference adds them
+// in loop order: batch of o, then dimension, then side, then face (k3, j3,
+// i3); the same order is rebuilt here from the position of o in the level's
+// active list.  Variables [v0, v1); first: the key of the contributor through
+// which c was found, or -1 where c is visited once.
+__device__ __forceinline__ void reflux_cell(const AmrLevelArgs& a, int g, int ind, long c, int v0, int v1, int first) {
   const AmrTreeView& t = a.t;
-  const int g = a.active_coarse[cidx >> 3];
-  const int ind = (int)(cidx & 7) + 1;
-  const long c = cell_of(t, ind, g);
-  if (t.son[c] != 0) return;  // only leaves receive the correction (:811,863)
   const int p[3] = {(ind - 1) & 1, ((ind - 1) >> 1) & 1, (ind - 1) >> 2};
   // the six neighbour cells first (independent loads), then their sons
   long nc[6];
@@ -437,77 +432,131 @@ __device__ __forceinline__ void reflux_task(const AmrLevelArgs& a, long tix) {
   int pz[6];
 #pragma unroll
   for (int k = 0; k < 6; ++k) pz[k] = so[k] > 0 ? a.pos[so[k]] : 0;
-  // up to 6 contributing octs: key = batch*6 + 2*d + side
-  int keys[6], posn[6], ne = 0;
+  // up to 6 contributing octs: key = batch*6 + 2*d + side in the upper half,
+  // the oct's position below; a fixed network sorts them (as an array indexed
+  // by their number they would live in scratch memory)
+  constexpr long long kNone = 0x7fffffffffffffffLL;
+  long long kp[6];
 #pragma unroll
   for (int in = 1; in <= 6; ++in) {
-    if (so[in - 1] <= 0) continue;
     const int ax = (in - 1) >> 1, plus = (in - 1) & 1;
     // c is on o's minus side when n is c's plus neighbour
-    const int side = plus ? 0 : 1;
-    keys[ne] = (pz[in - 1] / a.nv) * 6 + 2 * ax + side;
-    posn[ne] = pz[in - 1];
-    ++ne;
+    const long long key = (long long)(pz[in - 1] / a.nv) * 6 + 2 * ax + (plus ? 0 : 1);
+    kp[in - 1] = so[in - 1] > 0 ? key << 32 | (long long)pz[in - 1] : kNone;
   }
-  if (ne == 0) return;
-  for (int i = 1; i < ne; ++i)  // insertion sort, at most 6 entries
-    for (int k = i; k > 0 && keys[k - 1] > keys[k]; --k) {
-      const int tk = keys[k]; keys[k] = keys[k - 1]; keys[k - 1] = tk;
-      const int tp = posn[k]; posn[k] = posn[k - 1]; posn[k - 1] = tp;
-    }
+  auto order = [&](int i, int k) {
+    const long long lo = kp[i] < kp[k] ? kp[i] : kp[k], hi = kp[i] < kp[k] ? kp[k] : kp[i];
+    kp[i] = lo;
+    kp[k] = hi;
+  };
+  order(1, 2); order(4, 5); order(0, 2); order(3, 5); order(0, 1); order(3, 4);
+  order(2, 5); order(0, 3); order(1, 4); order(2, 4); order(1, 3); order(2, 3);
+  if (kp[0] == kNone) return;
+  if (first >= 0 && (int)(kp[0] >> 32) != first) return;  // the first contributor takes the cell
   const int nv = a.nv;
   const size_t fvs = (size_t)nv * 27;
   const double oneontwotondim = 1.0 / 8.0;
   // All contributions are loaded first (independent loads, issued together),
   // then summed in the reference's order: contributor e by key, and within
   // it the 4 faces of the oct side in (k3, j3, i3) loop order.
-  double fv[6][4];
+  for (int v = v0; v < v1; ++v) {
+    double fv[6][4];
 #pragma unroll
-  for (int e = 0; e < 6; ++e) {
-    if (e >= ne) break;
-    const int d = (keys[e] % 6) >> 1, side = keys[e] & 1;
-    const int b = posn[e] / nv, lane = posn[e] % nv;
-    const double* flux = a.flux + (size_t)b * fvs * 15 + lane + (size_t)27 * (v + 5 * d) * nv;
-    // the side's 2x2 faces: the transverse coordinates run over {1,2} and the
-    // normal one is 1 (side 0, the oct's minus face) or 3 (side 1)
+    for (int e = 0; e < 6; ++e) {
+      if (kp[e] == kNone) break;
+      const int key = (int)(kp[e] >> 32), pos = (int)kp[e];
+      const int d = (key % 6) >> 1, side = key & 1;
+      const int b = pos / nv, lane = pos % nv;
+      const double* flux = a.flux + (size_t)b * fvs * 15 + lane + (size_t)27 * (v + 5 * d) * nv;
+      // the side's 2x2 faces: the transverse coordinates run over {1,2} and the
+      // normal one is 1 (side 0, the oct's minus face) or 3 (side 1)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int t1 = 1 + (q & 1), t2 = 1 + (q >> 1);  // inner loop first
-      int i3, j3, k3;
-      if (d == 0) { i3 = side ? 3 : 1; j3 = t1; k3 = t2; }
-      else if (d == 1) { i3 = t1; j3 = side ? 3 : 1; k3 = t2; }
-      else { i3 = t1; j3 = t2; k3 = side ? 3 : 1; }
-      fv[e][q] = flux[fslot(i3, j3, k3) * nv];
-    }
+      for (int q = 0; q < 4; ++q) {
+        const int t1 = 1 + (q & 1), t2 = 1 + (q >> 1);  // inner loop first
+        int i3, j3, k3;
+        if (d == 0) { i3 = side ? 3 : 1; j3 = t1; k3 = t2; }
+        else if (d == 1) { i3 = t1; j3 = side ? 3 : 1; k3 = t2; }
+        else { i3 = t1; j3 = t2; k3 = side ? 3 : 1; }
+        fv[e][q] = flux[fslot(i3, j3, k3) * nv];
+      }
   }
   double s = a.unew[(long)v * a.ustride + c];
 #pragma unroll
   for (int e = 0; e < 6; ++e) {
-    if (e >= ne) break;
-    const int side = keys[e] & 1;
+    if (kp[e] == kNone) break;
+    const int side = (int)(kp[e] >> 32) & 1;
 #pragma unroll
     for (int q = 0; q < 4; ++q) s = side ? s + fv[e][q] * oneontwotondim : s - fv[e][q] * oneontwotondim;
   }
   a.unew[(long)v * a.ustride + c] = s;
+  }
 }
 
-__global__ void amr_reflux(AmrLevelArgs a) {
-  const long n = 40L * level_count(a.noct_coarse, a.dnoct_coarse);
-  const long stride = (long)gridDim.x * blockDim.x;
-  for (long tix = (long)blockIdx.x * blockDim.x + threadIdx.x; tix < n; tix += stride) reflux_task(a, tix);
+// The leaves are found from the side with fewer octs: every cell of the
+// coarser level, or every side of the level's own octs where the neighbour
+// oct is missing (its cell is the leaf), of which the first in the
+// reference's order takes the cell.  Behind 1,000 octs on a level of 32,768
+// the first way took 28 us, the second 7.  Where that is few tasks, each
+// variable is a task of its own: the walk is repeated, but the kernel is
+// bound by latency then.  blk of nblk workgroups.
+__device__ __forceinline__ void reflux_tasks(const AmrLevelArgs& a, unsigned blk, unsigned nblk) {
+  const AmrTreeView& t = a.t;
+  const unsigned nf = (unsigned)level_count(a.noct, a.dnoct), nc = (unsigned)level_count(a.noct_coarse, a.dnoct_coarse);
+  if (nf == 0 || nc == 0) return;
+  const unsigned stride = nblk * blockDim.x, id = blk * blockDim.x + threadIdx.x;
+  const bool coarse = reflux_from_coarse(nf, nc);
+  const unsigned per = coarse ? 8 * nc : 6 * nf;  // below 2^31, as cell indices are
+  const unsigned split = per < kRefluxSplit ? 5 : 1;
+  for (unsigned i = id; i < per * split; i += stride) {
+    const unsigned v0 = split == 1 ? 0 : i / per, r = split == 1 ? i : i - v0 * per;
+    const int v1 = split == 1 ? 5 : (int)v0 + 1;
+    if (coarse) {  // (cell, oct), the oct fastest
+      const unsigned ind = r / nc;
+      const int g = a.active_coarse[r - ind * nc];
+      const long c = cell_of(t, (int)ind + 1, g);
+      if (t.son[c] == 0) reflux_cell(a, g, (int)ind + 1, c, (int)v0, v1, -1);  // only leaves (:811,863)
+    } else {  // (side, oct)
+      const unsigned side = r / nf, o = r - side * nf;
+      const int c = nbor_of(t, a.active[o], (int)side + 1);
+      if (c <= t.ncoarse || t.son[c] != 0) continue;
+      const unsigned q = (unsigned)(c - t.ncoarse - 1), ind = q / (unsigned)t.ngridmax;
+      // c lies on the oct's side `side`: the same key as reflux_cell's
+      reflux_cell(a, (int)(q - ind * (unsigned)t.ngridmax) + 1, (int)ind + 1, c, (int)v0, v1,
+                  (int)(o / a.nv) * 6 + (int)side);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void amr_reflux(AmrLevelArgs a) { reflux_tasks(a, blockIdx.x, gridDim.x); }
+
+// The cells of a level, 32 octs x 8 cells per 256 threads and turn: 32
+// consecutive octs per cell, so that a variable is read in runs of 256 bytes
+// where the octs are (cell by cell of each oct it is runs of 64), and no
+// division finds the cell.  The oct count is the host value or, with dn set,
+// the one in device memory; f(igrid, ind); blk of nblk workgroups of a
+// multiple of 256 threads.
+template <typename F>
+__device__ __forceinline__ void for_level_cells(const int* active, int noct, int blk, int nblk, F f) {
+  const int ind = (int)(threadIdx.x >> 5 & 7) + 1, per = (int)(blockDim.x >> 8);
+  const int first = (blk * per + (int)(threadIdx.x >> 8)) * 32 + (int)(threadIdx.x & 31);
+  for (int o = first; o < noct; o += nblk * per * 32) f(active[o], ind);
+}
+template <typename F>
+__device__ __forceinline__ void for_level_cells(const int* active, int noct, F f) {
+  for_level_cells(active, noct, (int)blockIdx.x, (int)gridDim.x, f);
 }
 
 // set_unew / set_uold over the level's active cells (hydro/godunov_fine.f90:58-65, 193-197).
-// The per-cell kernels below take the oct count as a host value or, with
-// dn set, from device memory (grid-stride loops over a persistent grid).
-__global__ void amr_copy_level(const int* active, int noct_h, const int* dn, AmrTreeView t, const double* src,
-                               double* dst, long ustride) {
-  const int noct = level_count(noct_h, dn);
-  const long n = 8L * noct, stride = (long)gridDim.x * blockDim.x;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const long c = cell_of(t, (int)(i / noct) + 1, active[i % noct]);
-    for (int v = 0; v < 5; ++v) dst[(long)v * ustride + c] = src[(long)v * ustride + c];
-  }
+__global__ __launch_bounds__(256) void amr_copy_level(const int* active, int noct_h, const int* dn, AmrTreeView t,
+                                                     const double* src, double* dst, long ustride) {
+  for_level_cells(active, level_count(noct_h, dn), [&](int g, int ind) {
+    const long c = cell_of(t, ind, g);
+    double q[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = src[(long)v * ustride + c];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) dst[(long)v * ustride + c] = q[v];
+  });
 }
 
 // upl for one refined cell c with son oct s: the average of its children
@@ -547,136 +596,154 @@ __device__ inline void upl_cell(const AmrTreeView& t, double* u, long ustride, l
 }
 
 // upload_fine: refined cells of the level get the average of their children
-// (hydro/interpol_hydro.f90:5-67).
-__global__ void amr_upload(const int* active, int noct_h, const int* dn, AmrTreeView t, double* u, long ustride,
-                           double smallr, int ivar_mode) {
-  const long n = 8L * level_count(noct_h, dn), stride = (long)gridDim.x * blockDim.x;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const long c = cell_of(t, (int)(i % 8) + 1, active[i / 8]);
+// (hydro/interpol_hydro.f90:5-67).  flag1 (or null): flag every cell too, all
+// that flag_fine does below levelmin (init_flag, amr/flag_utils.f90:150-157).
+__global__ __launch_bounds__(256) void amr_upload(const int* active, int noct_h, const int* dn, AmrTreeView t,
+                                                 double* u, long ustride, double smallr, int ivar_mode, int* flag1) {
+  for_level_cells(active, level_count(noct_h, dn), [&](int g, int ind) {
+    const long c = cell_of(t, ind, g);
     const int s = t.son[c];
+    if (flag1) flag1[c] = 1;
     if (s > 0) upl_cell(t, u, ustride, c, s, smallr, ivar_mode);
-  }
+  });
 }
 
 // set_uold followed by upload_fine of the level in one pass
 // (hydro/godunov_fine.f90:135-232, hydro/interpol_hydro.f90:5-263): a leaf
 // takes unew, a refined cell the average of its children's uold (set_uold
 // writes every cell and upload_fine then rewrites the refined ones, so the
-// result is the same).
-__global__ void amr_finish(const int* active, int noct_h, const int* dn, AmrTreeView t, const double* unew, double* u,
-                           long ustride, double smallr, int ivar_mode) {
-  const long n = 8L * level_count(noct_h, dn), stride = (long)gridDim.x * blockDim.x;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const long c = cell_of(t, (int)(i % 8) + 1, active[i / 8]);
+// result is the same).  The first thread also ends the level step's time
+// bookkeeping: dtnew(l-1) = dtnew(l) if nsubcycle(l-1) == 1, or dtold(l) +
+// dtnew(l) after the second substep (amr/amr_step.f90:573-576); nsub_coarser
+// 0: level l is levelmin.  The first `refluxers` workgroups do the level's
+// reflux instead (reflux_tasks), which reads its fluxes and adds to the
+// coarser level's unew: neither touches what the other reads.
+__global__ __launch_bounds__(256) void amr_finish(AmrLevelArgs a, double* u, int ivar_mode, double* dt,
+                                                 const double* dtold, int nsub_coarser, int icount, int refluxers) {
+  if ((int)blockIdx.x < refluxers) {
+    reflux_tasks(a, blockIdx.x, (unsigned)refluxers);
+    return;
+  }
+  const AmrTreeView& t = a.t;
+  const double* unew = a.unew;
+  const long ustride = a.ustride;
+  const double smallr = a.hp.smallr;
+  const int l = a.ilevel;
+  const int noct = level_count(a.noct, a.dnoct);
+  if ((int)blockIdx.x == refluxers && threadIdx.x == 0 && noct > 0 && nsub_coarser > 0) {
+    if (nsub_coarser == 1) dt[l - 1] = dt[l];
+    if (icount == 2) dt[l - 1] = dtold[l] + dt[l];
+  }
+  for_level_cells(a.active, noct, (int)blockIdx.x - refluxers, (int)gridDim.x - refluxers, [&](int g, int ind) {
+    const long c = cell_of(t, ind, g);
     const int s = t.son[c];
     if (s <= 0) {
+      double q[5];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) u[(long)v * ustride + c] = unew[(long)v * ustride + c];
+      for (int v = 0; v < 5; ++v) q[v] = unew[(long)v * ustride + c];
+#pragma unroll
+      for (int v = 0; v < 5; ++v) u[(long)v * ustride + c] = q[v];
     } else {
       upl_cell(t, u, ustride, c, s, smallr, ivar_mode);
     }
-  }
+  });
+}
+
+// The workgroup's largest w, in thread 0.
+__device__ __forceinline__ double block_max(double w) {
+  __shared__ double red[16];
+  for (int off = 32; off > 0; off >>= 1) w = fmax_f(w, __shfl_xor(w, off, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) w = fmax_f(w, red[k]);
+  return w;
 }
 
 // courant_fine over the level's leaf cells (hydro/courant_fine.f90:44-131):
 // block max of the cmpdt wave speed, block dt limit min-combined (exact,
 // see cmpdt_w).
-__global__ void amr_courant(const int* active, int noct_h, const int* dn, AmrTreeView t, const double* u,
-                            long ustride, double dx, HydroParams hp, double* d_dt) {
-  const long n = 8L * level_count(noct_h, dn), stride = (long)gridDim.x * blockDim.x;
+__global__ __launch_bounds__(256) void amr_courant(const int* active, int noct_h, const int* dn, AmrTreeView t,
+                                                  const double* u, long ustride, double dx, HydroParams hp,
+                                                  double* d_dt) {
   double w = 0.0;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const long c = cell_of(t, (int)(i % 8) + 1, active[i / 8]);
+  for_level_cells(active, level_count(noct_h, dn), [&](int g, int ind) {
+    const long c = cell_of(t, ind, g);
     if (t.son[c] == 0)
       w = fmax_f(w, cmpdt_w(u[c], u[ustride + c], u[2 * ustride + c], u[3 * ustride + c], u[4 * ustride + c], hp));
-  }
-  for (int off = 32; off > 0; off >>= 1) w = fmax_f(w, __shfl_xor(w, off, 64));
-  __shared__ double red[4];
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double m = red[0];
-    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) m = fmax_f(m, red[k]);
-    if (m > 0.0) atomicMin(reinterpret_cast<unsigned long long*>(d_dt), dt_bits(cmpdt_from_w(m, dx, hp)));
-  }
+  });
+  w = block_max(w);
+  if (threadIdx.x == 0 && w > 0.0)
+    atomicMin(reinterpret_cast<unsigned long long*>(d_dt), dt_bits(cmpdt_from_w(w, dx, hp)));
 }
 
-// set_unew and courant_fine of a level in one pass over its cells
-// (hydro/godunov_fine.f90:40-130, hydro/courant_fine.f90:44-131): every
-// cell copies uold to unew, every leaf joins the block max of the cmpdt wave
-// speed, and the block's dt limit is min-combined into *d_dt (exact: the dt
-// limit is non-increasing in the wave speed).
-__global__ void amr_begin(const int* active, int noct_h, const int* dn, AmrTreeView t, const double* u, double* unew,
-                          long ustride, double dx, HydroParams hp, double* d_dt, double* partials) {
+// set_unew, newdt_fine and courant_fine of a level in one pass over its
+// cells (hydro/godunov_fine.f90:40-130, pm/newdt_fine.f90:51,177,
+// hydro/courant_fine.f90:44-131): every cell copies uold to unew and every
+// leaf joins the max of the cmpdt wave speed in d.wmax.  The workgroup that
+// finishes last does the level's time-step bookkeeping (amr/amr_step.f90):
+//   dtold(l) = dtnew(l); dtnew(l) = min(start, dtnew(l-1)/nsubcycle(l-1)
+//   below levelmin, the limit of the largest wave speed) (:327-330; the dt
+//   limit is non-increasing in the wave speed and min is exact, so the order
+//   of the minima does not matter), and where no finer level has octs
+//   dtold(l+1) = dtnew(l+1) = dtnew(l)/nsubcycle(l), t += dtnew(l) (:353-362,
+//   amr/update_time.f90:217,331); cnt counts update_time calls (nstep) and
+//   cell updates.
+// As kernels of one thread before and after the pass these took 2.6 us each,
+// twice a level step.  At most 256 workgroups of 1024: their two atomics meet
+// at one address each (3,600 workgroups of 256 took 78 us for a level of
+// 115k octs, 36 of them for these).
+constexpr int kBeginThreads = 1024;
+__global__ __launch_bounds__(kBeginThreads) void amr_begin(const int* active, int noct_h, const int* dn, AmrTreeView t,
+                                                const double* u, double* unew, long ustride, double dx,
+                                                HydroParams hp, AmrStepDt d, double* partials) {
   const int noct = level_count(noct_h, dn);
-  const long n = 8L * noct, stride = (long)gridDim.x * blockDim.x;
   double w = 0.0;
   ConsSums cs{0.0, 0.0, 0.0};  // courant_fine's sums over the leaves (partials set)
   const double vol = dx * dx * dx;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const long c = cell_of(t, (int)(i / noct) + 1, active[i % noct]);
+  for_level_cells(active, noct, [&](int g, int ind) {
+    const long c = cell_of(t, ind, g);
+    const int s = t.son[c];
     double q[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) q[v] = u[(long)v * ustride + c];
 #pragma unroll
     for (int v = 0; v < 5; ++v) unew[(long)v * ustride + c] = q[v];
-    if (t.son[c] == 0) {
+    if (s == 0) {
       w = fmax_f(w, cmpdt_w(q[0], q[1], q[2], q[3], q[4], hp));
       if (partials) cons_add(cs, q[0], q[1], q[2], q[3], q[4], vol, hp.smallr);
     }
-  }
+  });
   if (partials) {
-    __shared__ double cred[3 * 4];
+    __shared__ double cred[3 * (kBeginThreads / 64)];
     cons_block_store(cs, partials, blockIdx.x, cred);
   }
-  for (int off = 32; off > 0; off >>= 1) w = fmax_f(w, __shfl_xor(w, off, 64));
-  __shared__ double red[4];
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double m = red[0];
-    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) m = fmax_f(m, red[k]);
-    if (m > 0.0) atomicMin(reinterpret_cast<unsigned long long*>(d_dt), dt_bits(cmpdt_from_w(m, dx, hp)));
+  const unsigned working = min((unsigned)((noct + kBeginThreads / 8 - 1) / (kBeginThreads / 8)), gridDim.x);
+  if (blockIdx.x >= working) return;
+  w = block_max(w);
+  if (threadIdx.x != 0) return;
+  // The count depends on what the maximum returned, so it cannot be seen
+  // before the maximum; a fence in its place would write back and drop the
+  // XCD's whole L2 for every workgroup (0.13 ms of a level of 10^5 octs).
+  unsigned dep = (unsigned)atomicMax(d.wmax, w > 0.0 ? dt_bits(w) : 0ULL);
+  asm volatile("v_and_b32 %0, 0, %0" : "+v"(dep));
+  if (atomicAdd(d.done, 1u + dep) != working - 1) return;
+  const double wm = __longlong_as_double((long long)atomicExch(d.wmax, 0ULL));
+  *d.done = 0;
+  const int l = d.l;
+  double v = d.start;
+  if (d.nsub_coarser > 0) v = fmin_f(d.dt[l - 1] / (double)d.nsub_coarser, v);
+  if (wm > 0.0) v = fmin_f(v, cmpdt_from_w(wm, dx, hp));
+  d.dtold[l] = d.dt[l];
+  d.dt[l] = v;
+  if (d.cnt) d.cnt[1] += 8LL * noct;
+  if (d.has_finer && (dn ? dn[1] > 0 : d.finer_octs > 0)) return;
+  if (d.has_finer) {
+    d.dtold[l + 1] = v / (double)d.nsub;
+    d.dt[l + 1] = v / (double)d.nsub;
   }
-}
-
-// The level time-step bookkeeping of amr_step (amr/amr_step.f90), one
-// thread, so a coarse step keeps every dt on the device:
-//   op 0  newdt_fine prologue: dtold(l) = dtnew(l); dtnew(l) = start, capped
-//         by dtnew(l-1)/nsubcycle(l-1) below levelmin (:327-330; the courant
-//         reduction then min-combines into it -- min is exact, so the order
-//         of the three minima does not matter)
-//   op 1  no finer level: dtold(l+1) = dtnew(l+1) = dtnew(l)/nsubcycle(l),
-//         t += dtnew(l) (:353-362, amr/update_time.f90:217,331)
-//   op 2  end of the step: dtnew(l-1) = dtnew(l) if nsubcycle(l-1) == 1, or
-//         dtold(l) + dtnew(l) after the second substep (:573-576)
-// With dn (the device oct counts, indexed by level) the operations are those
-// of a level step that runs only when level l has octs, and op 1 only when
-// no finer level does (amr/amr_step.f90:345-365); cnt, if set, counts
-// update_time calls (cnt[0], nstep) and cell updates (cnt[1]).
-__global__ void amr_dt_kernel(int op, double* dt, double* dtold, double* time, int l, int coarser, int nsub,
-                              int icount, double start, const int* dn, long long* cnt) {
-  if (dn) {
-    if (dn[l] == 0) return;
-    if (op == 1 && coarser && dn[l + 1] > 0) return;
-    if (cnt && op == 0) cnt[1] += 8LL * dn[l];
-    if (cnt && op == 1) cnt[0] += 1;
-  }
-  if (op == 0) {
-    dtold[l] = dt[l];
-    double v = start;
-    if (coarser) v = fmin_f(dt[l - 1] / (double)nsub, v);
-    dt[l] = v;
-  } else if (op == 1) {
-    if (coarser) {  // here: a finer level index exists
-      dtold[l + 1] = dt[l] / (double)nsub;
-      dt[l + 1] = dt[l] / (double)nsub;
-    }
-    time[0] = time[0] + dt[l];
-  } else {
-    if (nsub == 1) dt[l - 1] = dt[l];
-    if (icount == 2) dt[l - 1] = dtold[l] + dt[l];
-  }
+  d.time[0] = d.time[0] + v;
+  if (d.cnt) d.cnt[0] += 1;
 }
 
 // update_time's conservation baselines (amr/update_time.f90:229-246) at
@@ -791,16 +858,26 @@ __global__ void set_ints(int* p, int n, int v) {
 
 }  // namespace
 
-// Grid of a per-cell launch over n items: sized to n for a host count, a
-// fixed persistent grid for a count read from device memory.
-inline unsigned cell_grid(long n, const int* dn) {
-  return dn ? persist_blocks() : (unsigned)((n + 255) / 256);
+// Grid of a launch over the cells of noct octs (for_level_cells): sized to a
+// host count, a fixed persistent grid for a count read from device memory.
+inline unsigned cell_grid(int noct, const int* dn) {
+  return dn ? persist_blocks() : (unsigned)((noct + 31) / 32);
 }
 
-// gather + unsplit + update + reflux of one level; dt is read from d_dt.
-// With a.dnoct / a.dnoct_coarse the counts are read from device memory and
-// the grids are persistent (batch loops), so the launches can be captured.
-hipError_t launch_amr_godunov(const AmrLevelArgs& a, double dx, const double* d_dt, double* tmp, bool fp32,
+// Workgroups of a level's reflux, 0 without a coarser level.
+static unsigned reflux_grid(const AmrLevelArgs& a) {
+  if (!a.active_coarse || (!a.dnoct_coarse && a.noct_coarse <= 0)) return 0;
+  if (a.dnoct) return persist_blocks();
+  const unsigned nf = (unsigned)a.noct, nc = (unsigned)a.noct_coarse;
+  const long per = reflux_from_coarse(nf, nc) ? 8L * nc : 6L * nf;
+  return (unsigned)(((per < (long)kRefluxSplit ? 5 * per : per) + 255) / 256);
+}
+
+// gather + unsplit + update of one level (godunov_fine without its reflux);
+// dt is read from d_dt.  With a.dnoct / a.dnoct_coarse the counts are read
+// from device memory and the grids are persistent (batch loops), so the
+// launches can be captured.
+hipError_t launch_amr_sweep(const AmrLevelArgs& a, double dx, const double* d_dt, double* tmp, bool fp32,
                               hipStream_t s) {
   const bool dev = a.dnoct != nullptr;
   if (!dev && a.noct <= 0) return hipSuccess;
@@ -849,68 +926,71 @@ hipError_t launch_amr_godunov(const AmrLevelArgs& a, double dx, const double* d_
     hipLaunchKernelGGL(amr_update, dim3(ugrid), dim3(256), 0, s, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  if (a.active_coarse && (a.dnoct_coarse || a.noct_coarse > 0)) {
-    const long n = 40L * a.noct_coarse;
-    hipLaunchKernelGGL(amr_reflux, dim3(cell_grid(n, a.dnoct_coarse)), dim3(256), 0, s, a);
-  }
+  return hipGetLastError();
+}
+
+hipError_t launch_amr_reflux(const AmrLevelArgs& a, hipStream_t s) {
+  const unsigned grid = reflux_grid(a);
+  if (grid == 0 || (!a.dnoct && a.noct <= 0)) return hipSuccess;
+  hipLaunchKernelGGL(amr_reflux, dim3(grid), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_amr_copy(const int* active, int noct, const AmrTreeView& t, const double* src, double* dst,
                            long ustride, hipStream_t s, const int* dn) {
   if (!dn && noct <= 0) return hipSuccess;
-  hipLaunchKernelGGL(amr_copy_level, dim3(cell_grid(8L * noct, dn)), dim3(256), 0, s, active, noct, dn, t, src, dst,
+  hipLaunchKernelGGL(amr_copy_level, dim3(cell_grid(noct, dn)), dim3(256), 0, s, active, noct, dn, t, src, dst,
                      ustride);
   return hipGetLastError();
 }
 
 hipError_t launch_amr_upload(const int* active, int noct, const AmrTreeView& t, double* u, long ustride,
-                             double smallr, int ivar_mode, hipStream_t s, const int* dn) {
+                             double smallr, int ivar_mode, hipStream_t s, const int* dn, int* flag1) {
   if (!dn && noct <= 0) return hipSuccess;
-  hipLaunchKernelGGL(amr_upload, dim3(cell_grid(8L * noct, dn)), dim3(256), 0, s, active, noct, dn, t, u, ustride,
-                     smallr, ivar_mode);
+  hipLaunchKernelGGL(amr_upload, dim3(cell_grid(noct, dn)), dim3(256), 0, s, active, noct, dn, t, u, ustride,
+                     smallr, ivar_mode, flag1);
   return hipGetLastError();
 }
 
 hipError_t launch_amr_courant(const int* active, int noct, const AmrTreeView& t, const double* u, long ustride,
                               double dx, const HydroParams& hp, double* d_dt, hipStream_t s, const int* dn) {
   if (!dn && noct <= 0) return hipSuccess;
-  hipLaunchKernelGGL(amr_courant, dim3(cell_grid(8L * noct, dn)), dim3(256), 0, s, active, noct, dn, t, u, ustride,
+  hipLaunchKernelGGL(amr_courant, dim3(cell_grid(noct, dn)), dim3(256), 0, s, active, noct, dn, t, u, ustride,
                      dx, hp, d_dt);
   return hipGetLastError();
 }
 
-// With partials (room for amr_begin_blocks(noct, dn) workgroups) the
-// level's conservation sums are added into sums[0..2] after the pass.
+static unsigned begin_grid(int noct, bool persistent) {
+  const unsigned nb = (unsigned)((noct + kBeginThreads / 8 - 1) / (kBeginThreads / 8));
+  return persistent || nb > 256 ? 256 : nb;
+}
+
+// With partials (amr_begin_partials_bytes) the level's conservation sums are
+// added into sums[0..2] after the pass.
 hipError_t launch_amr_begin(const int* active, int noct, const AmrTreeView& t, const double* u, double* unew,
-                            long ustride, double dx, const HydroParams& hp, double* d_dt, hipStream_t s,
+                            long ustride, double dx, const HydroParams& hp, const AmrStepDt& d, hipStream_t s,
                             const int* dn, double* partials, double* sums) {
   if (!dn && noct <= 0) return hipSuccess;
-  const unsigned nb = cell_grid(8L * noct, dn);
-  hipLaunchKernelGGL(amr_begin, dim3(nb), dim3(256), 0, s, active, noct, dn, t, u, unew, ustride, dx, hp, d_dt,
-                     partials);
+  const unsigned nb = begin_grid(noct, dn != nullptr);
+  hipLaunchKernelGGL(amr_begin, dim3(nb), dim3(kBeginThreads), 0, s, active, noct, dn, t, u, unew, ustride, dx, hp, d, partials);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !partials) return e;
   return launch_cons_finish(partials, nb, sums, 1, s);
 }
 
 size_t amr_begin_partials_bytes(int noct, bool persistent) {
-  const size_t nb = persistent ? persist_blocks() : (size_t)((8L * noct + 255) / 256);
+  const size_t nb = begin_grid(noct, persistent);
   return (nb > 0 ? nb : 1) * 3 * sizeof(double);
 }
 
-hipError_t launch_amr_finish(const int* active, int noct, const AmrTreeView& t, const double* unew, double* u,
-                             long ustride, double smallr, int ivar_mode, hipStream_t s, const int* dn) {
-  if (!dn && noct <= 0) return hipSuccess;
-  hipLaunchKernelGGL(amr_finish, dim3(cell_grid(8L * noct, dn)), dim3(256), 0, s, active, noct, dn, t, unew, u,
-                     ustride, smallr, ivar_mode);
-  return hipGetLastError();
-}
-
-hipError_t launch_amr_dt(int op, double* dt, double* dtold, double* time, int l, int coarser, int nsub, int icount,
-                         double start, hipStream_t s, const int* dn, long long* cnt) {
-  hipLaunchKernelGGL(amr_dt_kernel, dim3(1), dim3(1), 0, s, op, dt, dtold, time, l, coarser, nsub, icount, start, dn,
-                     cnt);
+// set_uold, upload_fine, the reflux into the coarser level and the end of the
+// level step's time bookkeeping, in one launch.
+hipError_t launch_amr_finish(const AmrLevelArgs& a, double* u, double* dt, const double* dtold, int nsub_coarser,
+                             int icount, hipStream_t s) {
+  if (!a.dnoct && a.noct <= 0) return hipSuccess;
+  const unsigned refluxers = reflux_grid(a);
+  hipLaunchKernelGGL(amr_finish, dim3(refluxers + cell_grid(a.noct, a.dnoct)), dim3(256), 0, s, a, u, a.interpol_var, dt,
+                     dtold, nsub_coarser, icount, (int)refluxers);
   return hipGetLastError();
 }
 

@@ -41,6 +41,22 @@ struct AmrLevelArgs {
   int* error;                // set nonzero if the tree violates the refinement rule
 };
 
+// The time-step bookkeeping that amr_begin does for level l of a coarse step.
+struct AmrStepDt {
+  double* dt;      // dtnew(l) at index l
+  double* dtold;
+  double* time;
+  int l;
+  int nsub_coarser;  // nsubcycle(l-1), or 0 at levelmin
+  int nsub;          // nsubcycle(l)
+  int has_finer;     // l < nlevelmax
+  int finer_octs;    // octs of level l+1 (with device counts dn[l+1] is read instead)
+  double start;      // newdt_fine's starting value capped by cmpdt's
+  long long* cnt;    // update_time calls and cell updates, or null
+  unsigned long long* wmax;  // zero between launches, as is
+  unsigned* done;            // the count of finished workgroups
+};
+
 // Every level's grid list and host oct count (index = level), for a kernel
 // that walks several levels.
 constexpr int kConsMaxLevels = 33;  // RAMSES_MAX_LEVELS + 1

@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <atomic>
+#include <new>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -33,27 +34,26 @@ hipError_t launch_level_batch(double* const* buf0, double* const* buf1, double* 
                               const double* dx, int nslots, const HydroParams& hp, bool fp32, hipStream_t s);
 long level_batch_blocks(const int* n, int nslots);
 hipError_t launch_init_slot(double* state, double t_end, double start, hipStream_t s);
-hipError_t launch_amr_godunov(const AmrLevelArgs& a, double dx, const double* d_dt, double* tmp, bool fp32,
-                              hipStream_t s);
+hipError_t launch_amr_sweep(const AmrLevelArgs& a, double dx, const double* d_dt, double* tmp, bool fp32,
+                            hipStream_t s);
+hipError_t launch_amr_reflux(const AmrLevelArgs& a, hipStream_t s);
 hipError_t launch_amr_copy(const int* active, int noct, const AmrTreeView& t, const double* src, double* dst,
                            long ustride, hipStream_t s, const int* dn = nullptr);
 hipError_t launch_amr_upload(const int* active, int noct, const AmrTreeView& t, double* u, long ustride,
-                             double smallr, int ivar_mode, hipStream_t s, const int* dn = nullptr);
+                             double smallr, int ivar_mode, hipStream_t s, const int* dn = nullptr,
+                             int* flag1 = nullptr);
 hipError_t launch_amr_courant(const int* active, int noct, const AmrTreeView& t, const double* u, long ustride,
                               double dx, const HydroParams& hp, double* d_dt, hipStream_t s, const int* dn = nullptr);
-hipError_t launch_amr_dt(int op, double* dt, double* dtold, double* time, int l, int coarser, int nsub, int icount,
-                         double start, hipStream_t s, const int* dn = nullptr, long long* cnt = nullptr);
 hipError_t launch_set_ints(int* p, int n, int v, hipStream_t s);
 hipError_t launch_amr_cons0(const ConsLevels& lv, const int* dn, const AmrTreeView& t, const double* u, long ustride,
                             int levelmin, int nlevelmax, double boxlen, int nv, const int* armed, double* cons0,
                             hipStream_t s);
 hipError_t launch_clear_bits(int* p, int mask, hipStream_t s);
 hipError_t launch_amr_begin(const int* active, int noct, const AmrTreeView& t, const double* u, double* unew,
-                            long ustride, double dx, const HydroParams& hp, double* d_dt, hipStream_t s,
-                            const int* dn = nullptr, double* partials = nullptr,
-                            double* sums = nullptr);
-hipError_t launch_amr_finish(const int* active, int noct, const AmrTreeView& t, const double* unew, double* u,
-                             long ustride, double smallr, int ivar_mode, hipStream_t s, const int* dn = nullptr);
+                            long ustride, double dx, const HydroParams& hp, const AmrStepDt& d, hipStream_t s,
+                            const int* dn = nullptr, double* partials = nullptr, double* sums = nullptr);
+hipError_t launch_amr_finish(const AmrLevelArgs& a, double* u, double* dt, const double* dtold, int nsub_coarser,
+                             int icount, hipStream_t s);
 struct RefineParams {
   double err_grad_d, err_grad_u, err_grad_p;
   double floor_d, floor_u, floor_p;
@@ -70,7 +70,7 @@ hipError_t launch_flag_fine(const int* active, int noct, const AmrTreeView& t, i
 size_t refine_work_bytes(int noct, int noct_fine);
 hipError_t launch_refine_fine_dev(const int* active, const int* dn_l, int ilevel, const AmrTreeView& t,
                                   const TreeMut& m, int* active_fine, int* dn_f, int* pos, int* ring, int* dfree,
-                                  int* ctrl, int* flag1, int* flag2, double* xg, double* uold, double* unew,
+                                  unsigned* done, int* flag1, int* flag2, double* xg, double* uold, double* unew,
                                   int interpol_type, int interpol_var, double smallr, void* work, int* d_error,
                                   int capacity, hipStream_t s);
 hipError_t launch_refine_fine(const int* active, int noct, int ilevel, const AmrTreeView& t, const TreeMut& m,
@@ -437,8 +437,36 @@ int ramses_amr_config(int interpol_type, int interpol_var) {
 
 unsigned long ramses_amr_work_bytes(int noct) { return (unsigned long)amr_work(noct < 0 ? 0 : noct, current().nvector); }
 
-int ramses_amr_godunov(const ramses_amr_tree* t, const ramses_amr_level* lv, const double* uold, double* unew,
-                       const double* d_dt, void* work, unsigned long work_bytes, int* d_error, void* stream) {
+namespace {
+// The arguments of a level's sweep; the workspace (ramses_amr_work_bytes) is
+// laid out for nb batches.  Returns the sweep's tmp array.
+double* sweep_args(ramses::AmrLevelArgs& a, const ramses::AmrTreeView& v, const Config& c, const double* uold,
+                   double* unew, int ilevel, const int* pos, void* work, size_t nb, int* error) {
+  const size_t nv = (size_t)c.nvector;
+  a.t = v;
+  a.uold = uold;
+  a.unew = unew;
+  a.ustride = v.ncell + 1;
+  a.ilevel = ilevel;
+  a.pos = pos;
+  char* w = (char*)(((uintptr_t)work + 255) & ~(uintptr_t)255);
+  a.uin = (double*)w;
+  a.flux = a.uin + nb * nv * 216 * 5;
+  double* tmp = a.flux + nb * nv * 27 * 15;
+  a.ok = (unsigned char*)(tmp + nb * nv * 27 * 6);
+  a.nv = c.nvector;
+  a.interpol_type = c.interpol_type;
+  a.interpol_var = c.interpol_var;
+  a.hp = c.hp;
+  a.error = error;
+  return tmp;
+}
+
+// godunov_fine of a level with the counts on the host, without its reflux;
+// a: the sweep's arguments, for the launch that does the reflux.
+int godunov_level(const ramses_amr_tree* t, const ramses_amr_level* lv, const double* uold, double* unew,
+                  const double* d_dt, void* work, unsigned long work_bytes, int* d_error, hipStream_t s,
+                  ramses::AmrLevelArgs& a) {
   const Config c = current();
   ramses::AmrTreeView v;
   int rc = amr_view(t, v);
@@ -451,34 +479,27 @@ int ramses_amr_godunov(const ramses_amr_tree* t, const ramses_amr_level* lv, con
   if (c.nvector * 27 > 1024) return fail(-8, "nvector too large for the AMR gather (max 37)");
   const size_t need = amr_work(lv->noct, c.nvector);
   if (!work || work_bytes < need) return fail(-1, "work buffer too small (see ramses_amr_work_bytes)");
-  ramses::AmrLevelArgs a;
-  a.t = v;
-  a.uold = uold;
-  a.unew = unew;
-  a.ustride = v.ncell + 1;
+  double* tmp = sweep_args(a, v, c, uold, unew, lv->ilevel, lv->pos, work,
+                           (size_t)((lv->noct + c.nvector - 1) / c.nvector), d_error);
   a.active = lv->active;
   a.noct = lv->noct;
   a.dnoct = nullptr;
   a.dnoct_coarse = nullptr;
-  a.ilevel = lv->ilevel;
-  a.pos = lv->pos;
-  const int nv = c.nvector;
-  const size_t nb = (size_t)((lv->noct + nv - 1) / nv);
-  char* w = (char*)(((uintptr_t)work + 255) & ~(uintptr_t)255);
-  a.uin = (double*)w;
-  a.flux = a.uin + nb * nv * 216 * 5;
-  double* tmp = a.flux + nb * nv * 27 * 15;
-  a.ok = (unsigned char*)(tmp + nb * nv * 27 * 6);
-  a.nv = nv;
-  a.interpol_type = c.interpol_type;
-  a.interpol_var = c.interpol_var;
-  a.hp = c.hp;
   a.active_coarse = lv->active_coarse;
   a.noct_coarse = lv->active_coarse ? lv->noct_coarse : 0;
-  a.error = d_error;
-  hipError_t e = ramses::launch_amr_godunov(a, lv->dx, d_dt, tmp, c.precision == RAMSES_FP32_MIXED,
-                                            (hipStream_t)stream);
+  hipError_t e = ramses::launch_amr_sweep(a, lv->dx, d_dt, tmp, c.precision == RAMSES_FP32_MIXED, s);
   if (e != hipSuccess) return hip_fail(e, "amr godunov launch");
+  return 0;
+}
+}  // namespace
+
+int ramses_amr_godunov(const ramses_amr_tree* t, const ramses_amr_level* lv, const double* uold, double* unew,
+                       const double* d_dt, void* work, unsigned long work_bytes, int* d_error, void* stream) {
+  ramses::AmrLevelArgs a;
+  int rc = godunov_level(t, lv, uold, unew, d_dt, work, work_bytes, d_error, (hipStream_t)stream, a);
+  if (rc) return rc;
+  hipError_t e = ramses::launch_amr_reflux(a, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "amr reflux launch");
   return 0;
 }
 
@@ -603,6 +624,8 @@ struct StepCtx {
   Config cfg;
   bool cons_armed;  // nstep_coarse changed since the last update_time
   bool cons_done;   // the step's first update_time has been passed
+  unsigned long long* wmax;  // zeroed device words of amr_begin
+  unsigned* done;
 };
 
 // The grid lists and host counts of every level.
@@ -665,22 +688,20 @@ int amr_step_rec(StepCtx& c, int l, int icount) {
   double start = c.cfg.hp.courant_factor * lv.dx / c.cfg.hp.smallc;
   const double cap = m->boxlen / c.cfg.hp.smallc;
   if (cap < start) start = cap;
-  const int coarser = l > m->levelmin;
-  hipError_t e = ramses::launch_amr_dt(0, m->dt, m->dtold, m->time, l, coarser, coarser ? m->nsubcycle[l - 1] : 1,
-                                       0, start, c.s);
-  if (e != hipSuccess) return hip_fail(e, "dt launch");
-  // courant_fine and set_unew in one pass (with the conservation sums:
-  // mass_tot = mass_tot + mass_all etc., hydro/courant_fine.f90:152-154)
+  // courant_fine and set_unew in one pass, with newdt_fine's and, where no
+  // finer level has octs, update_time's bookkeeping (and the conservation
+  // sums: mass_tot = mass_tot + mass_all etc., hydro/courant_fine.f90:152-154)
+  const int nsub_coarser = l > m->levelmin ? m->nsubcycle[l - 1] : 0;
+  const ramses::AmrStepDt d{m->dt, m->dtold, m->time, l, nsub_coarser, m->nsubcycle[l], l < m->nlevelmax,
+                            l < m->nlevelmax ? m->noct[l + 1] : 0, start, nullptr, c.wmax, c.done};
   if (m->sums && (rc = ensure_work(m, ramses::amr_begin_partials_bytes(lv.noct, false), c.s))) return rc;
-  e = ramses::launch_amr_begin(lv.active, lv.noct, v, m->uold, m->unew, v.ncell + 1, lv.dx, c.cfg.hp, m->dt + l, c.s,
-                               nullptr, m->sums ? (double*)m->work : nullptr, m->sums);
+  hipError_t e = ramses::launch_amr_begin(lv.active, lv.noct, v, m->uold, m->unew, v.ncell + 1, lv.dx, c.cfg.hp, d, c.s,
+                                          nullptr, m->sums ? (double*)m->work : nullptr, m->sums);
   if (e != hipSuccess) return hip_fail(e, "courant / set_unew launch");
   if (l < m->nlevelmax && m->noct[l + 1] > 0) {
     if ((rc = amr_step_rec(c, l + 1, 1))) return rc;
     if (m->nsubcycle[l] == 2 && (rc = amr_step_rec(c, l + 1, 2))) return rc;
   } else {
-    e = ramses::launch_amr_dt(1, m->dt, m->dtold, m->time, l, l < m->nlevelmax, m->nsubcycle[l], 0, 0.0, c.s);
-    if (e != hipSuccess) return hip_fail(e, "dt launch");
     m->nstep += 1;
     // update_time's conservation baselines (amr/update_time.f90:229-246)
     if (m->cons0 && !c.cons_done && c.cons_armed) {
@@ -692,21 +713,18 @@ int amr_step_rec(StepCtx& c, int l, int icount) {
   }
   lv = level_of(m, l);  // the finer levels' refinements changed noct(l+1) only
   if ((rc = ensure_work(m, amr_work(lv.noct, current().nvector), c.s))) return rc;
-  rc = ramses_amr_godunov(&m->tree, &lv, m->uold, m->unew, m->dt + l, m->work, m->work_bytes, m->error, c.s);
+  ramses::AmrLevelArgs a;
+  rc = godunov_level(&m->tree, &lv, m->uold, m->unew, m->dt + l, m->work, m->work_bytes, m->error, c.s, a);
   if (rc) return rc;
   m->cell_updates += 8LL * lv.noct;
-  e = ramses::launch_amr_finish(lv.active, lv.noct, v, m->unew, m->uold, v.ncell + 1, c.cfg.hp.smallr, c.cfg.interpol_var,
-                                c.s);
-  if (e != hipSuccess) return hip_fail(e, "set_uold/upload launch");
+  // the reflux with set_uold and upload_fine
+  e = ramses::launch_amr_finish(a, m->uold, m->dt, m->dtold, nsub_coarser, icount, c.s);
+  if (e != hipSuccess) return hip_fail(e, "reflux/set_uold/upload launch");
   if (m->adaptive) {
     // ensure_ref_rules runs for icount < nsubcycle(l-1) (amr/flag_utils.f90:94-98)
     const int ic = (l <= m->levelmin || m->nsubcycle[l - 1] == 2) ? icount : 2;
     rc = ramses_amr_flag_fine(&m->tree, &lv, ic, m->levelmin, m->nlevelmax, m->uold, m->flag1, m->flag2, c.s);
     if (rc) return rc;
-  }
-  if (l > m->levelmin) {
-    e = ramses::launch_amr_dt(2, m->dt, m->dtold, m->time, l, 1, m->nsubcycle[l - 1], icount, 0.0, c.s);
-    if (e != hipSuccess) return hip_fail(e, "dt launch");
   }
   return 0;
 }
@@ -719,10 +737,12 @@ int amr_step_rec(StepCtx& c, int l, int icount) {
 struct AmrDevState {
   int noct[RAMSES_MAX_LEVELS + 2];
   int free[4];       // head, numbf, used_mem
-  int ctrl[4];       // refine decision: ncreate, nkill, ok
   int error;         // *m->error after the step
   int cons_armed;    // nstep_coarse changed since the last update_time
   long long cnt[2];  // nstep, cell_updates
+  // zero between the kernels that use them
+  unsigned long long wmax;  // amr_begin's largest wave speed
+  unsigned done;            // workgroups that have finished
 };
 
 struct GraphState {
@@ -753,6 +773,25 @@ struct GraphState {
     cap = nullptr;
   }
 };
+
+// The mesh's library-owned state with its device part, zeroed on stream s.
+int ensure_state(ramses_amr_mesh* m, hipStream_t s, GraphState*& gs) {
+  gs = static_cast<GraphState*>(m->graph_state);
+  if (!gs) {
+    gs = new (std::nothrow) GraphState();
+    if (!gs) return fail(-1, "out of host memory");
+    m->graph_state = gs;
+  }
+  if (gs->dev) return 0;
+  hipError_t e = hipMalloc(&gs->dev, sizeof(AmrDevState));
+  if (e != hipSuccess) {
+    gs->dev = nullptr;
+    return hip_fail(e, "step state");
+  }
+  e = ramses::launch_set_ints(reinterpret_cast<int*>(gs->dev), (int)(sizeof(AmrDevState) / sizeof(int)), 0, s);
+  if (e != hipSuccess) return hip_fail(e, "step state");
+  return 0;
+}
 
 void graph_key(const ramses_amr_mesh* m, int capacity, std::vector<long>& k) {
   k.clear();
@@ -803,7 +842,7 @@ hipError_t gstep(GCtx& g, int l, int icount) {
   if (m->adaptive && m->levelmin < m->nlevelmax && (l == m->levelmin || icount > 1)) {
     for (int i = l; i < m->nlevelmax; ++i) {
       e = ramses::launch_refine_fine_dev(m->active[i], dn + i, i, g.v, g.tm, m->active[i + 1], dn + i + 1, m->pos,
-                                         m->free.ring, g.dev->free, g.dev->ctrl, m->flag1, m->flag2, m->xg, m->uold,
+                                         m->free.ring, g.dev->free, &g.dev->done, m->flag1, m->flag2, m->xg, m->uold,
                                          m->unew, g.c.interpol_type, g.c.interpol_var, g.c.hp.smallr, g.work, m->error,
                                          g.capacity, g.s);
       if (e != hipSuccess) return e;
@@ -813,21 +852,17 @@ hipError_t gstep(GCtx& g, int l, int icount) {
   double start = g.c.hp.courant_factor * dx / g.c.hp.smallc;
   const double capdt = m->boxlen / g.c.hp.smallc;
   if (capdt < start) start = capdt;
-  const int coarser = l > m->levelmin;
-  e = ramses::launch_amr_dt(0, m->dt, m->dtold, m->time, l, coarser, coarser ? m->nsubcycle[l - 1] : 1, 0, start, g.s,
-                            dn, g.dev->cnt);
-  if (e != hipSuccess) return e;
+  const int nsub_coarser = l > m->levelmin ? m->nsubcycle[l - 1] : 0;
+  const ramses::AmrStepDt d{m->dt, m->dtold, m->time, l, nsub_coarser, m->nsubcycle[l], l < m->nlevelmax, 0, start,
+                            g.dev->cnt, &g.dev->wmax, &g.dev->done};
   double* partials = m->sums ? (double*)(((uintptr_t)g.work + 255) & ~(uintptr_t)255) : nullptr;
-  e = ramses::launch_amr_begin(m->active[l], 0, g.v, m->uold, m->unew, us, dx, g.c.hp, m->dt + l, g.s, dn + l,
-                               partials, m->sums);
-  if (e != hipSuccess) return e;  // courant_fine + set_unew
+  e = ramses::launch_amr_begin(m->active[l], 0, g.v, m->uold, m->unew, us, dx, g.c.hp, d, g.s, dn + l, partials,
+                               m->sums);
+  if (e != hipSuccess) return e;  // newdt_fine, courant_fine and set_unew
   if (l < m->nlevelmax) {
     if ((e = gstep(g, l + 1, 1)) != hipSuccess) return e;
     if (m->nsubcycle[l] == 2 && (e = gstep(g, l + 1, 2)) != hipSuccess) return e;
   }
-  e = ramses::launch_amr_dt(1, m->dt, m->dtold, m->time, l, l < m->nlevelmax, m->nsubcycle[l], 0, 0.0, g.s, dn,
-                            g.dev->cnt);
-  if (e != hipSuccess) return e;
   // update_time's conservation baselines: emitted after the first update_time
   // of the capture order (the deepest level's).  At run time the step's
   // first update_time may come at a shallower level, but every launch
@@ -840,44 +875,22 @@ hipError_t gstep(GCtx& g, int l, int icount) {
     if (e != hipSuccess) return e;
   }
   ramses::AmrLevelArgs a;
-  a.t = g.v;
-  a.uold = m->uold;
-  a.unew = m->unew;
-  a.ustride = us;
+  double* tmp = sweep_args(a, g.v, g.c, m->uold, m->unew, l, m->pos, g.work,
+                           (size_t)((g.capacity + g.c.nvector - 1) / g.c.nvector), m->error);
   a.active = m->active[l];
   a.noct = 0;
   a.dnoct = dn + l;
   a.dnoct_coarse = l > 1 ? dn + l - 1 : nullptr;
-  a.ilevel = l;
-  a.pos = m->pos;
-  const int nv = g.c.nvector;
-  const size_t nb = (size_t)((g.capacity + nv - 1) / nv);
-  char* w = (char*)(((uintptr_t)g.work + 255) & ~(uintptr_t)255);
-  a.uin = (double*)w;
-  a.flux = a.uin + nb * nv * 216 * 5;
-  double* tmp = a.flux + nb * nv * 27 * 15;
-  a.ok = (unsigned char*)(tmp + nb * nv * 27 * 6);
-  a.nv = nv;
-  a.interpol_type = g.c.interpol_type;
-  a.interpol_var = g.c.interpol_var;
-  a.hp = g.c.hp;
   a.active_coarse = l > 1 ? m->active[l - 1] : nullptr;
   a.noct_coarse = 0;
-  a.error = m->error;
-  e = ramses::launch_amr_godunov(a, dx, m->dt + l, tmp, g.c.precision == RAMSES_FP32_MIXED, g.s);
+  e = ramses::launch_amr_sweep(a, dx, m->dt + l, tmp, g.c.precision == RAMSES_FP32_MIXED, g.s);
   if (e != hipSuccess) return e;
-  e = ramses::launch_amr_finish(m->active[l], 0, g.v, m->unew, m->uold, us, g.c.hp.smallr, g.c.interpol_var, g.s,
-                                dn + l);
+  e = ramses::launch_amr_finish(a, m->uold, m->dt, m->dtold, nsub_coarser, icount, g.s);
   if (e != hipSuccess) return e;
   if (m->adaptive) {
     const int ic = (l <= m->levelmin || m->nsubcycle[l - 1] == 2) ? icount : 2;
     e = ramses::launch_flag_fine(m->active[l], 0, g.v, l, ic, m->levelmin, m->nlevelmax, m->uold, us, m->flag1,
                                  m->flag2, g.c.rp, g.c.hp, g.s, dn + l);
-    if (e != hipSuccess) return e;
-  }
-  if (l > m->levelmin) {
-    e = ramses::launch_amr_dt(2, m->dt, m->dtold, m->time, l, 1, m->nsubcycle[l - 1], icount, 0.0, g.s, dn,
-                              g.dev->cnt);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -898,11 +911,7 @@ hipError_t gcoarse(GCtx& g) {
     const long us = g.v.ncell + 1;
     for (int l = m->levelmin - 1; l >= 1; --l)
       if ((e = ramses::launch_amr_upload(m->active[l], 0, g.v, m->uold, us, g.c.hp.smallr, g.c.interpol_var, g.s,
-                                         g.dev->noct + l)) != hipSuccess)
-        return e;
-    for (int l = m->levelmin - 1; l >= 1; --l)
-      if ((e = ramses::launch_flag_fine(m->active[l], 0, g.v, l, 2, m->levelmin, m->nlevelmax, m->uold, us, m->flag1,
-                                        m->flag2, g.c.rp, g.c.hp, g.s, g.dev->noct + l)) != hipSuccess)
+                                         g.dev->noct + l, m->flag1)) != hipSuccess)  // upload_fine, flag_fine
         return e;
     if ((e = ramses::launch_set_ints(m->flag1 + 1, m->tree.ncoarse, 1, g.s)) != hipSuccess) return e;
   }
@@ -934,15 +943,12 @@ int coarse_step_graph(ramses_amr_mesh* m, hipStream_t s) {
   ramses::AmrTreeView v;
   int rc = amr_view(&m->tree, v);
   if (rc) return rc;
-  GraphState* gs = static_cast<GraphState*>(m->graph_state);
+  GraphState* gs = nullptr;
+  if ((rc = ensure_state(m, s, gs))) return rc;
   hipError_t e;
-  if (!gs) {
-    gs = new GraphState();
-    m->graph_state = gs;
-    if ((e = hipStreamCreate(&gs->cap)) != hipSuccess) return hip_fail(e, "capture stream");
-    if ((e = hipMalloc(&gs->dev, sizeof(AmrDevState))) != hipSuccess) return hip_fail(e, "graph state");
-    if ((e = hipHostMalloc(&gs->host, sizeof(AmrDevState))) != hipSuccess) return hip_fail(e, "graph staging");
-  }
+  if (!gs->cap && (e = hipStreamCreate(&gs->cap)) != hipSuccess) return hip_fail(e, "capture stream");
+  if (!gs->host && (e = hipHostMalloc(&gs->host, sizeof(AmrDevState))) != hipSuccess)
+    return hip_fail(e, "graph staging");
   if (gs->capacity != capacity || !gs->work) {
     if (gs->work) {
       if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "graph workspace sync");
@@ -1028,25 +1034,27 @@ int ramses_amr_coarse_step(ramses_amr_mesh* m, void* stream) {
       return fail(-1, "free list head/numbf out of range");
   }
   if (m->graph) return coarse_step_graph(m, (hipStream_t)stream);
-  StepCtx c{m, (hipStream_t)stream, current(), m->nstep_coarse != m->nstep_coarse_old, false};
+  GraphState* gs = nullptr;
+  int rc = ensure_state(m, (hipStream_t)stream, gs);
+  if (rc) return rc;
+  StepCtx c{m,     (hipStream_t)stream, current(),    m->nstep_coarse != m->nstep_coarse_old,
+            false, &gs->dev->wmax,      &gs->dev->done};
   // adaptive_loop resets the totals at every coarse step (amr/adaptive_loop.f90:89-91)
   if (m->sums) {
     hipError_t e = ramses::launch_set_doubles(m->sums, 3, 0.0, c.s);
     if (e != hipSuccess) return hip_fail(e, "sums reset launch");
   }
-  int rc = amr_step_rec(c, m->levelmin, 1);
+  rc = amr_step_rec(c, m->levelmin, 1);
   if (rc) return rc;
   m->nstep_coarse_old = m->nstep_coarse;  // update_time's bookkeeping (amr/update_time.f90:310)
   m->nstep_coarse += 1;
   if (m->adaptive && m->levelmin < m->nlevelmax) {
-    for (int l = m->levelmin - 1; l >= 1; --l) {
-      ramses_amr_level lv = level_of(m, l);
-      if ((rc = ramses_amr_upload(&m->tree, &lv, m->uold, c.s))) return rc;
-    }
-    for (int l = m->levelmin - 1; l >= 1; --l) {
-      ramses_amr_level lv = level_of(m, l);
-      rc = ramses_amr_flag_fine(&m->tree, &lv, 2, m->levelmin, m->nlevelmax, m->uold, m->flag1, m->flag2, c.s);
-      if (rc) return rc;
+    ramses::AmrTreeView v;
+    if ((rc = amr_view(&m->tree, v))) return rc;
+    for (int l = m->levelmin - 1; l >= 1; --l) {  // upload_fine, flag_fine
+      hipError_t e = ramses::launch_amr_upload(m->active[l], m->noct[l], v, m->uold, v.ncell + 1, c.cfg.hp.smallr,
+                                               c.cfg.interpol_var, c.s, nullptr, m->flag1);
+      if (e != hipSuccess) return hip_fail(e, "upload launch");
     }
     hipError_t e = ramses::launch_set_ints(m->flag1 + 1, m->tree.ncoarse, 1, c.s);  // flag_coarse
     if (e != hipSuccess) return hip_fail(e, "flag_coarse launch");
