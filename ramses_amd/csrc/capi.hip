@@ -86,6 +86,11 @@ Tuning& tuning() {
 
 #include "unsplit_args.hpp"
 #include "amr_args.hpp"
+#include "oct_tile.hpp"
+
+namespace ramses {
+const oct_tile::Tables& tile_tables();
+}
 
 namespace {
 
@@ -125,9 +130,11 @@ Config current() {
   return g_cfg;
 }
 
-// Device staging for the host-memory entry points, with a pinned host
-// mirror: the caller's arrays are copied into it on the host and cross PCIe
-// in two DMA transfers each way instead of six pageable ones.  The
+// Staging for the host-memory entry points: pinned host memory that the
+// kernel reads and writes itself (unsplit_direct), and for the 27-point
+// slopes and cmpdt device memory with a pinned host mirror: the caller's
+// arrays are copied into it on the host and cross PCIe in one DMA transfer
+// each way.  The
 // reference's unsplit is not reentrant (its `save` scratch arrays,
 // hydro/umuscl.f90:41-53); the host-memory form is likewise serialised on
 // one library-owned stream.
@@ -137,11 +144,30 @@ struct Staging {
   double* buf = nullptr;   // device
   double* host = nullptr;  // pinned host memory of the same size
   size_t cap = 0;          // doubles
-  int ensure(size_t n) {
-    if (!stream) {
-      hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
-      if (e != hipSuccess) return hip_fail(e, "hipStreamCreate");
+  double* direct = nullptr;  // pinned host memory that the kernel itself reads and writes
+  size_t direct_cap = 0;     // doubles
+  int ensure_stream() {
+    if (stream) return 0;
+    hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
+    return e == hipSuccess ? 0 : hip_fail(e, "hipStreamCreate");
+  }
+  int ensure_direct(size_t n) {
+    int rc = ensure_stream();
+    if (rc || n <= direct_cap) return rc;
+    if (direct) (void)hipHostFree(direct);
+    direct = nullptr;
+    direct_cap = 0;
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&direct), n * sizeof(double), hipHostMallocDefault);
+    if (e != hipSuccess) {
+      direct = nullptr;
+      return hip_fail(e, "hipHostMalloc");
     }
+    direct_cap = n;
+    return 0;
+  }
+  int ensure(size_t n) {
+    int rc = ensure_stream();
+    if (rc) return rc;
     if (n <= cap) return 0;
     // every call synchronises its stream before returning, so nothing is in
     // flight on the old buffers
@@ -234,12 +260,86 @@ int ramses_unsplit_device(const double* uin, const double* gravin, double* flux,
   return 0;
 }
 
+}  // extern "C"
+
+namespace {
+
+// One batch from and to host memory with the 7-point slopes.  The kernel
+// itself reads the 80 cells per oct that a face depends on from pinned host
+// memory and writes the 36 faces there, 5.2 KB per oct, so the host copies a
+// quarter of the arrays and no transfer is set up: 40 us a call of 32 octs,
+// 69 with DMA transfers of the whole arrays, most of it the launch and the
+// wait.  Entries of flux and tmp that the reference never writes are not
+// touched.  A gravity array of +0.0
+// words in those cells gives the bits of none.
+int unsplit_direct(const Config& c, const double* uin, const double* gravin, double* flux, double* tmp, double dx,
+                   double dy, double dz, double dt, int ngrid) {
+  using namespace ramses;
+  if (!(dx > 0) || !(dy > 0) || !(dz > 0)) return fail(-1, "dx, dy, dz must be > 0");
+  const oct_tile::Tables& tab = tile_tables();
+  const size_t nv = (size_t)c.nvector, run = (size_t)ngrid * sizeof(double);
+  std::lock_guard<std::mutex> lk(g_stage.mu);
+  int rc = g_stage.ensure_direct(nv * (oct_tile::kCells * 8 + oct_tile::kFaces * 7));
+  if (rc) return rc;
+  double* h_u = g_stage.direct;
+  double* h_g = h_u + nv * oct_tile::kCells * 5;
+  double* h_f = h_g + nv * oct_tile::kCells * 3;
+  for (int k = 0; k < oct_tile::kCells; ++k)
+    for (int v = 0; v < 5; ++v)
+      std::memcpy(h_u + (size_t)(k * 5 + v) * nv, uin + ((size_t)v * 216 + tab.cell[k]) * nv, run);
+  bool gravity = false;
+  if (gravin) {
+    uint64_t any = 0;
+    for (int k = 0; k < oct_tile::kCells; ++k)
+      for (int v = 0; v < 3; ++v) {
+        const double* g = gravin + ((size_t)v * 216 + tab.cell[k]) * nv;
+        std::memcpy(h_g + (size_t)(k * 3 + v) * nv, g, run);
+        for (int l = 0; l < ngrid; ++l) {
+          uint64_t w;
+          std::memcpy(&w, g + l, sizeof w);
+          any |= w;
+        }
+      }
+    gravity = any != 0;
+  }
+  UnsplitArgs a;
+  a.uin = h_u;
+  a.grav = gravity ? h_g : nullptr;
+  a.flux = h_f;
+  a.tmp = nullptr;
+  a.dx[0] = dx;
+  a.dx[1] = dy;
+  a.dx[2] = dz;
+  a.dt = dt;
+  a.d_dt = nullptr;
+  a.ngroups = 1;
+  a.ngrid_last = ngrid;
+  a.nv = c.nvector;
+  a.hp = c.hp;
+  a.compact = 1;
+  hipError_t e = launch_unsplit(a, c.precision == RAMSES_FP32_MIXED, g_stage.stream);
+  if (e != hipSuccess) return hip_fail(e, "unsplit launch");
+  if ((e = hipStreamSynchronize(g_stage.stream)) != hipSuccess) return hip_fail(e, "unsplit sync");
+  for (int f = 0; f < oct_tile::kFaces; ++f) {
+    const double* o = h_f + (size_t)(7 * f) * nv;
+    const size_t d = (size_t)f / 12, at = tab.out[f];
+    for (size_t v = 0; v < 5; ++v) std::memcpy(flux + (at + 27 * (v + 5 * d)) * nv, o + v * nv, run);
+    for (size_t v = 0; v < 2; ++v) std::memcpy(tmp + (at + 27 * (v + 2 * d)) * nv, o + (5 + v) * nv, run);
+  }
+  return 0;
+}
+
+}  // namespace
+
+extern "C" {
+
 int ramses_unsplit(const double* uin, const double* gravin, double* flux, double* tmp, double dx, double dy,
                    double dz, double dt, int ngrid) {
   const Config c = current();
   if (!uin || !flux || !tmp) return fail(-1, "null array");
   if (ngrid < 0 || ngrid > c.nvector) return fail(-1, "ngrid out of [0, nvector]");
   if (ngrid == 0) return 0;
+  if (c.hp.slope_type != 3) return unsplit_direct(c, uin, gravin, flux, tmp, dx, dy, dz, dt, ngrid);
   const size_t nv = (size_t)c.nvector;
   const size_t nu = nv * 216 * 5, ng = nv * 216 * 3, nf = nv * 27 * 5 * 3, nt = nv * 27 * 2 * 3;
   std::lock_guard<std::mutex> lk(g_stage.mu);
@@ -357,8 +457,9 @@ void unsplit_(const double* uin, const double* gravin, const double* pin, double
   // so it is not copied and the gravity-free kernels run; a -0.0 or any
   // other word keeps the array.
   const double* g = gravin;
-  if (g) {
-    const size_t n = (size_t)current().nvector * 216 * 3;
+  const Config c = current();
+  if (g && c.hp.slope_type == 3) {  // else only the words that are read count (unsplit_direct)
+    const size_t n = (size_t)c.nvector * 216 * 3;
     size_t i = 0;
     for (; i < n; ++i) {
       uint64_t w;

@@ -74,19 +74,21 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void unsplit_tile(UnsplitArgs a, long
   const SolverConsts<R> sc = make_consts<R>(hp);
   const double dtxhalf = dt * 0.5;
   const double smalle = hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0);  // hydro/umuscl.f90:884
-  const size_t vs = (size_t)nv * 216;
-  const double* u = a.uin + g * vs * 5 + lane;
-  const double* gr = G ? a.grav + g * vs * 3 + lane : nullptr;
+  // strides between cells and between variables
+  const size_t cs = a.compact ? (size_t)nv * 5 : (size_t)nv, vs = a.compact ? (size_t)nv : (size_t)nv * 216;
+  const size_t gcs = a.compact ? (size_t)nv * 3 : (size_t)nv;
+  const double* u = a.uin + g * ((size_t)nv * 216 * 5) + lane;
+  const double* gr = G ? a.grav + g * ((size_t)nv * 216 * 3) + lane : nullptr;
   double w[kLoads][5], acc[kLoads][3];
 #pragma unroll
   for (int k = 0; k < kLoads; ++k) {
     const int e = t + k * kThreads;
     if (e < kPairs) {
-      const size_t o = (size_t)kTab.cell[e / kOcts] * nv;
+      const size_t cell = a.compact ? (size_t)(e / kOcts) : (size_t)kTab.cell[e / kOcts];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) w[k][v] = u[o + v * vs];
+      for (int v = 0; v < 5; ++v) w[k][v] = u[cell * cs + v * vs];
 #pragma unroll
-      for (int v = 0; v < 3; ++v) acc[k][v] = G ? gr[o + v * vs] : 0.0;
+      for (int v = 0; v < 3; ++v) acc[k][v] = G ? gr[cell * gcs + v * vs] : 0.0;
     }
   }
 #pragma unroll
@@ -111,15 +113,24 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void unsplit_tile(UnsplitArgs a, long
     double out[7];
     scale_flux<7>(val, fs, out);  // :106,111,129,153
     if (o0 + l < nocts) {
-      double* flux = a.flux + g * fvs * 15 + (size_t)(kTab.out[f] + 27 * 5 * d) * nv + lane;
+      double *flux, *tmp;
+      size_t st;
+      if (a.compact) {
+        st = (size_t)nv;
+        flux = a.flux + (size_t)(7 * f) * nv + lane;
+        tmp = flux + 5 * st;
+      } else {
+        st = fvs;
+        flux = a.flux + g * fvs * 15 + (size_t)(kTab.out[f] + 27 * 5 * d) * nv + lane;
+        tmp = a.tmp + g * fvs * 6 + (size_t)(kTab.out[f] + 27 * 2 * d) * nv + lane;
+      }
       flux[0] = out[0];
-      flux[(size_t)(1 + d) * fvs] = out[1];  // the momenta in their own order (:809-842)
-      flux[(size_t)(d == 0 ? 2 : 1) * fvs] = out[2];
-      flux[(size_t)(d == 2 ? 2 : 3) * fvs] = out[3];
-      flux[4 * fvs] = out[4];
-      double* tmp = a.tmp + g * fvs * 6 + (size_t)(kTab.out[f] + 27 * 2 * d) * nv + lane;
+      flux[(size_t)(1 + d) * st] = out[1];  // the momenta in their own order (:809-842)
+      flux[(size_t)(d == 0 ? 2 : 1) * st] = out[2];
+      flux[(size_t)(d == 2 ? 2 : 3) * st] = out[3];
+      flux[4 * st] = out[4];
       tmp[0] = out[5];
-      tmp[fvs] = out[6];
+      tmp[st] = out[6];
     }
   }
 }
@@ -172,6 +183,11 @@ static void launch_r(const UnsplitArgs& a, long grid, int block, hipStream_t str
       break;
     default: s27 ? launch_t<R, kLLF, true>(a, grid, block, stream) : launch_t<R, kLLF, false>(a, grid, block, stream); break;
   }
+}
+
+const oct_tile::Tables& tile_tables() {
+  static constexpr oct_tile::Tables t = oct_tile::make_tables();
+  return t;
 }
 
 hipError_t launch_unsplit(const UnsplitArgs& a, bool fp32, hipStream_t stream) {

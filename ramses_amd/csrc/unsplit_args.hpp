@@ -25,6 +25,10 @@ struct UnsplitArgs {
   // Oct-tree sweeps only: at or below this many octs the level's unsplit
   // runs one face per thread instead of one row of faces per thread.
   int face_octs = 0;
+  // One batch in the layout of the host-memory calls (7-point slopes): uin
+  // (and grav) hold the 80 cells a face depends on, [slot][variable][nv], and
+  // flux holds the 36 faces, [face][5 fluxes, 2 tmp][nv]; tmp is not used.
+  int compact = 0;
 };
 
 }  // namespace ramses

@@ -60,3 +60,39 @@ def test_level_sweep_ragged_tiles(gpu, oracle_lib, level, octs, riemann, slope):
     want = np.where(swept, ref[(slice(None),) + at], grid[(slice(None),) + at])
     assert np.array_equal(s.state("new")[:, cells - 1], want)
     ra.configure()
+
+
+@pytest.mark.parametrize("slope", [1, 2, 3])
+@pytest.mark.parametrize("gravity", ["none", "zero", "negative zero", "full", "unread"])
+@pytest.mark.parametrize("nv,ngrid", [(32, 32), (32, 5), (7, 7), (37, 36), (130, 129)])
+def test_host_call_same_bits_as_device_call(gpu, nv, ngrid, gravity, slope):
+    """unsplit on host arrays against the resident form, to the bit and to the
+    sign of a zero: lanes past ngrid and entries outside the faces keep the
+    caller's values, and gravity in cells that no face depends on (the 6^3
+    corners) changes nothing."""
+    import torch
+    rng = np.random.default_rng(13)
+    shape = (1, 6, 6, 6, nv)
+    u = np.ascontiguousarray(np.moveaxis(conserved(rng.lognormal(0.0, 1.0, shape), rng.normal(0.0, 1.0, (3,) + shape),
+                                                   rng.lognormal(-0.5, 0.5, shape), 5 / 3), 0, 1))
+    u[:, 1, 2:4] = -0.0  # momenta whose zero's sign a +0.0 acceleration drops
+    g = {"none": None, "zero": np.zeros(ra.grav_shape(nv)), "negative zero": np.full(ra.grav_shape(nv), -0.0),
+         "full": rng.normal(0.0, 1.0, ra.grav_shape(nv)), "unread": np.zeros(ra.grav_shape(nv))}[gravity]
+    if gravity == "unread":
+        if slope == 3:
+            pytest.skip("the 27-point slopes read every cell")
+        g[:, [0, 0, 5], [0, 5, 5], [5, 0, 5]] = 7.0
+    ra.configure(gamma=5 / 3, riemann="hllc", slope_type=slope, nvector=nv)
+    flux, tmp = np.full(ra.flux_shape(nv), 3.0), np.full(ra.tmp_shape(nv), 3.0)
+    d = [None if a is None else torch.from_numpy(np.ascontiguousarray(a[None])).cuda() for a in (u[0], g, flux, tmp)]
+    for call in ("c", "fortran"):
+        flux[:], tmp[:] = 3.0, 3.0
+        if call == "c":
+            ra.unsplit(u[0], g, flux, tmp, 0.01, 0.02, 0.04, 1e-4, ngrid)
+        else:
+            ra.unsplit_fortran(u[0], g, np.zeros((6, 6, 6, nv)), flux, tmp, 0.01, 0.02, 0.04, 1e-4, ngrid)
+        ra.unsplit_device(d[0], d[1], d[2], d[3], 0.01, 1e-4, ngrid_last=ngrid, dy=0.02, dz=0.04)
+        torch.cuda.synchronize()
+        for h, r in ((flux, d[2]), (tmp, d[3])):
+            assert np.array_equal(h.view(np.uint64), r[0].cpu().numpy().view(np.uint64)), call
+    ra.configure()
