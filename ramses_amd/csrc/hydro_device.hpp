@@ -81,6 +81,41 @@ __device__ __forceinline__ double fmin_f(double a, double b) { return __builtin_
 __device__ __forceinline__ float fmax_f(float a, float b) { return __builtin_fmaxf(a, b); }
 __device__ __forceinline__ float fmin_f(float a, float b) { return __builtin_fminf(a, b); }
 
+// The same for results of arithmetic, which are never signalling NaNs: for
+// operands from memory (shared memory, kernel arguments) the compiler puts a
+// v_max in front of the intrinsics that would quiet one, six for a face of
+// the level kernel.  floor_at: the bound is the same for all lanes.
+__device__ __forceinline__ double max_q(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double min_q(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double floor_at(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "s"(b));
+  return r;
+}
+__device__ __forceinline__ float max_q(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ float min_q(float a, float b) {
+  float r;
+  asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ float floor_at(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "s"(b), "v"(a));
+  return r;
+}
+
 // Division / square root in the working precision.  FP64 keeps IEEE
 // correctly rounded division and sqrt (the reference's semantics); the FP32
 // path uses the hardware reciprocal / sqrt (about 1 ulp), which is what makes
@@ -131,8 +166,13 @@ __device__ __forceinline__ unsigned hi_word(double x) {
   return (unsigned)((unsigned long long)__builtin_bit_cast(long long, x) >> 32);
 }
 __device__ __forceinline__ unsigned max_u(unsigned a, unsigned b) { return a > b ? a : b; }
-// Whether any active lane's flag is clear: a scalar branch.
-__device__ __forceinline__ bool any_not(bool ok) { return __builtin_expect(__ballot(!ok) != 0, 0); }
+// Whether any active lane has a flag clear: a scalar branch.  The lanes'
+// masks are combined rather than their flags: a compare alone is its mask,
+// and a combination would first become 0 or 1 in a vector register.
+template <typename... B>
+__device__ __forceinline__ bool any_not(B... ok) {
+  return __builtin_expect((__builtin_amdgcn_ballot_w64(!ok) | ...) != 0, 0);
+}
 
 // Primitive state of one cell: rho, vx, vy, vz, p.
 template <typename R>
@@ -184,6 +224,16 @@ __device__ __forceinline__ Prim<R> ctoprim_cell(double u0, double u1, double u2,
   return q;
 }
 
+// Both selects as selects: written with an early `return zero`, each of the
+// 15 slopes of a cell is an exec-mask branch that cuts the trace into small
+// blocks.
+template <typename R>
+__device__ __forceinline__ R minmod(R dlft, R drgt) {
+  const R zero = (R)0;
+  const R lim = (dlft > zero) ? fmin_f(dlft, drgt) : fmax_f(dlft, drgt);
+  return (dlft * drgt) <= zero ? zero : lim;
+}
+
 // One-dimensional slope of the 3D uslope branches with axial stencils
 // (hydro/umuscl.f90:1241-1285 minmod, :1286-1327 moncen, :1393-1431 van
 // Leer, :1432-1473 generalised moncen).
@@ -194,13 +244,7 @@ __device__ __forceinline__ R slope1(R qm1, R q0, R qp1, int st_run, R theta) {
   const int st = ST >= 0 ? ST : st_run;
   const R zero = (R)0;
   if (st == 1) {
-    const R dlft = q0 - qm1;
-    const R drgt = qp1 - q0;
-    // Both selects as selects: written with an early `return zero`, each of
-    // the 15 slopes of a cell is an exec-mask branch that cuts the trace into
-    // small blocks.
-    const R lim = (dlft > zero) ? fmin_f(dlft, drgt) : fmax_f(dlft, drgt);
-    return (dlft * drgt) <= zero ? zero : lim;
+    return minmod(q0 - qm1, qp1 - q0);
   } else if (st == 2) {
     const R two = (R)2;
     const R dlft = two * (q0 - qm1);
@@ -238,6 +282,16 @@ __device__ __forceinline__ Prim<R> slope_prim(const Prim<R>& a, const Prim<R>& b
   d.w = slope1<R, ST>(a.w, b.w, c.w, st, theta);
   d.p = slope1<R, ST>(a.p, b.p, c.p, st, theta);
   return d;
+}
+
+// Minmod of the primitives' differences.
+template <typename R>
+__device__ __forceinline__ Prim<R> minmod(const Prim<R>& a, const Prim<R>& b) {
+  return {minmod(a.r, b.r), minmod(a.u, b.u), minmod(a.v, b.v), minmod(a.w, b.w), minmod(a.p, b.p)};
+}
+template <typename R>
+__device__ __forceinline__ Prim<R> operator-(const Prim<R>& a, const Prim<R>& b) {
+  return {a.r - b.r, a.u - b.u, a.v - b.v, a.w - b.w, a.p - b.p};
 }
 
 // Source terms of the Hancock predictor (hydro/umuscl.f90:576-580).
@@ -335,11 +389,10 @@ __device__ __forceinline__ Face<R> rotate(const Prim<R>& q, int d) {
 // where the divisor lies in [2^-120, 2^120) in magnitude and every numerator
 // is zero, infinite, a NaN (v_frexp gives them exponent 0, and the fixup
 // their quotients) or in [2^-800, 2^800): a wavefront with a lane outside
-// divides in full.
+// divides in full.  y = rcp_newton(d) (FP64).
 template <int N, typename R>
-__device__ __forceinline__ void quotients(const R* n, R d, R* out) {
+__device__ __forceinline__ void quotients(const R* n, R d, R y, R* out) {
   if constexpr (sizeof(R) == 8) {
-    const double y = rcp_newton(d);
     int lo = 0, hi = 0;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
@@ -349,7 +402,7 @@ __device__ __forceinline__ void quotients(const R* n, R d, R* out) {
       out[k] = __builtin_amdgcn_div_fixup(quot(n[k], d, y), d, n[k]);
     }
     const unsigned dh = (hi_word(d) & 0x7fffffffu) - ((1023u - 120u) << 20);
-    if (!any_not(dh < (240u << 20) && lo > -800 && hi < 800)) return;
+    if (!any_not(dh < (240u << 20), lo > -800, hi < 800)) return;
   }
 #pragma unroll
   for (int k = 0; k < N; ++k) out[k] = div_w(n[k], d);
@@ -373,6 +426,17 @@ __device__ __forceinline__ void sound_speeds(R rl, R pl, R rr, R pr, R gamma, un
   }
   cl = sqrt_w(div_w(nl, rl));
   cr = sqrt_w(div_w(nr, rr));
+}
+
+// The larger of the two, with one root in FP64 (see riemann_hllc).
+template <typename R>
+__device__ __forceinline__ R larger_sound_speed(R rl, R pl, R rr, R pr, R gamma, unsigned div_hi) {
+  const R nl = gamma * pl, nr = gamma * pr;
+  if constexpr (sizeof(R) == 8) {
+    const R c = sqrt_normal(fmax_f(quot(nl, rl, rcp_newton(rl)), quot(nr, rr, rcp_newton(rr))));
+    if (!any_not(max_u(max_u(hi_word(rl), hi_word(rr)), max_u(hi_word(pl), hi_word(pr))) < div_hi)) return c;
+  }
+  return fmax_f(sqrt_w(div_w(nl, rl)), sqrt_w(div_w(nr, rr)));
 }
 
 // riemann_llf: hydro/godunov_utils.f90:660-820
@@ -426,10 +490,9 @@ __device__ __forceinline__ Flux6<R> riemann_hll(const Face<R>& L, const Face<R>&
   const R half = (R)0.5, zero = (R)0;
   const R rl = fmax_f(L.r, smallr), ul = L.un, pl = fmax_f(L.p, rl * smallp);
   const R rr = fmax_f(Rt.r, smallr), ur = Rt.un, pr = fmax_f(Rt.p, rr * smallp);
-  R cl, cr;
-  sound_speeds(rl, pl, rr, pr, gamma, div_hi, cl, cr);
-  const R SL = fmin_f(fmin_f(ul, ur) - fmax_f(cl, cr), zero);
-  const R SR = fmax_f(fmax_f(ul, ur) + fmax_f(cl, cr), zero);
+  const R c = larger_sound_speed(rl, pl, rr, pr, gamma, div_hi);
+  const R SL = fmin_f(fmin_f(ul, ur) - c, zero);
+  const R SR = fmax_f(fmax_f(ul, ur) + c, zero);
   R uL[6], uR[6], fL[6], fR[6];
   uL[0] = L.r;
   uR[0] = Rt.r;
@@ -463,7 +526,9 @@ __device__ __forceinline__ Flux6<R> riemann_hll(const Face<R>& L, const Face<R>&
   R num[6];
 #pragma unroll
   for (int n = 0; n < 6; ++n) num[n] = SR * fL[n] - SL * fR[n] + SR * SL * (uR[n] - uL[n]);
-  quotients<6>(num, den, g.f);
+  R y{};
+  if constexpr (sizeof(R) == 8) y = rcp_newton(den);
+  quotients<6>(num, den, y, g.f);
   return g;
 }
 
@@ -485,86 +550,76 @@ template <typename R>
 __device__ __forceinline__ Flux6<R> riemann_hllc(const Face<R>& L, const Face<R>& Rt, R gamma, R smallr,
                                                  R smallp, R entho, R smallc2, unsigned div_hi) {
   const R half = (R)0.5, zero = (R)0;
-  const R rl = fmax_f(L.r, smallr);
-  const R Pl = fmax_f(L.p, rl * smallp);
-  const R ul = L.un;
-  const R el = Pl * entho;
-  R ecinl = half * rl * ul * ul;
-  ecinl = ecinl + half * rl * (L.ut1 * L.ut1);
-  ecinl = ecinl + half * rl * (L.ut2 * L.ut2);
-  const R etotl = el + ecinl;
-  const R Ptotl = Pl;
-  const R rr = fmax_f(Rt.r, smallr);
-  const R Pr = fmax_f(Rt.p, rr * smallp);
-  const R ur = Rt.un;
-  const R er = Pr * entho;
-  R ecinr = half * rr * ur * ur;
-  ecinr = ecinr + half * rr * (Rt.ut1 * Rt.ut1);
-  ecinr = ecinr + half * rr * (Rt.ut2 * Rt.ut2);
-  const R etotr = er + ecinr;
-  const R Ptotr = Pr;
-  R SL = zero, SR = zero, rcl = zero, rcr = zero, ustar = zero, Ptotstar = zero;
-  // the waves from the two sound speeds, and the numerators and the divisor
+  const R rl = floor_at(L.r, smallr), ul = L.un;
+  const R Pl = max_q(L.p, rl * smallp);
+  const R rr = floor_at(Rt.r, smallr), ur = Rt.un;
+  const R Pr = max_q(Rt.p, rr * smallp);
+  R SL = zero, SR = zero, ustar = zero, Ptotstar = zero;
+  // the waves from the larger sound speed, and the numerators and the divisor
   // of the star velocity and pressure
   R nu = zero, np = zero, den = zero;
-  auto waves = [&](R cfastl, R cfastr) {
-    SL = fmin_f(ul, ur) - fmax_f(cfastl, cfastr);
-    SR = fmax_f(ul, ur) + fmax_f(cfastl, cfastr);
-    rcl = rl * (ul - SL);
-    rcr = rr * (SR - ur);
-    nu = rcr * ur + rcl * ul + (Ptotl - Ptotr);
-    np = rcr * Ptotl + rcl * Ptotr + rcl * rcr * (ul - ur);
+  auto waves = [&](R cfast) {
+    SL = min_q(ul, ur) - cfast;
+    SR = max_q(ul, ur) + cfast;
+    const R rcl = rl * (ul - SL);
+    const R rcr = rr * (SR - ur);
+    nu = rcr * ur + rcl * ul + (Pl - Pr);
+    np = rcr * Pl + rcl * Pr + rcl * rcr * (ul - ur);
     den = rcr + rcl;
   };
   bool full = true;
   if constexpr (sizeof(R) == 8) {
-    waves(sqrt_normal(fmax_f(quot(gamma * Pl, rl, rcp_newton(rl)), smallc2)),
-          sqrt_normal(fmax_f(quot(gamma * Pr, rr, rcp_newton(rr)), smallc2)));
+    // max(sqrt(a), sqrt(b)) is sqrt(max(a, b)): a correctly rounded root is
+    // monotonic
+    const R cl2 = floor_at(quot(gamma * Pl, rl, rcp_newton(rl)), smallc2);
+    const R cr2 = floor_at(quot(gamma * Pr, rr, rcp_newton(rr)), smallc2);
+    waves(sqrt_normal(max_q(cl2, cr2)));
     const double y = rcp_newton(den);
     ustar = quot(nu, den, y);
     Ptotstar = quot(np, den, y);
     const unsigned m = max_u(max_u(hi_word(rl), hi_word(rr)), max_u(hi_word(Pl), hi_word(Pr)));
     const unsigned dh = hi_word(den) - ((1023u - 100u) << 20);
-    full = any_not(m < div_hi && dh < (210u << 20) && __builtin_amdgcn_frexp_exp(nu) > -200);
+    full = any_not(m < div_hi, dh < (210u << 20), __builtin_amdgcn_frexp_exp(nu) > -200);
   }
   if (full) {
-    waves(sqrt_w(fmax_f(div_w(gamma * Pl, rl), smallc2)), sqrt_w(fmax_f(div_w(gamma * Pr, rr), smallc2)));
+    waves(fmax_f(sqrt_w(floor_at(div_w(gamma * Pl, rl), smallc2)), sqrt_w(floor_at(div_w(gamma * Pr, rr), smallc2))));
     ustar = div_w(nu, den);
     Ptotstar = div_w(np, den);
   }
-  R ro, uo, Ptoto, etoto, eo;
-  if (SL > zero) {
-    ro = rl; uo = ul; Ptoto = Ptotl; etoto = etotl; eo = el;
-  } else if (SR > zero || ustar > zero) {
-    // left star state when ustar>0, right star state otherwise (SR>0)
-    const bool left = ustar > zero;
-    const R S = left ? SL : SR;
-    const R us = left ? ul : ur;
-    const R rs = left ? rl : rr;
-    const R es = left ? el : er;
-    const R ets = left ? etotl : etotr;
-    const R Pts = left ? Ptotl : Ptotr;
-    const R dS = S - ustar;
-    const R nr = rs * (S - us), ne = (S - us) * ets - Pts * us + Ptotstar * ustar, ni = es * (S - us);
-    ro = etoto = eo = zero;
-    bool fulls = true;
-    if constexpr (sizeof(R) == 8) {
-      const double y = rcp_newton(dS);
-      ro = quot(nr, dS, y);
-      etoto = quot(ne, dS, y);
-      eo = quot(ni, dS, y);
-      fulls = full || any_not(abs_w(dS) >= 0x1p-90 && ets < 0x1p800);
-    }
-    if (fulls) {
-      ro = div_w(nr, dS);
-      etoto = div_w(ne, dS);
-      eo = div_w(ni, dS);
-    }
-    uo = ustar;
-    Ptoto = Ptotstar;
-  } else {
-    ro = rr; uo = ur; Ptoto = Ptotr; etoto = etotr; eo = er;
+  // The state upwind, left or right, and inside the outer waves its star
+  // state.  Its energy is formed once, for the side taken, and every choice
+  // is a select (the level kernel at 256^3, FP64: 828 us, 851 with both
+  // sides' energies, two roots and a branch for each region).
+  const bool star = !(SL > zero) && (SR > zero || ustar > zero);
+  const bool left = SL > zero || ustar > zero;
+  const R r0 = left ? rl : rr, u0 = left ? ul : ur, P0 = left ? Pl : Pr;
+  const R t1 = left ? L.ut1 : Rt.ut1, t2 = left ? L.ut2 : Rt.ut2;
+  const R e0 = P0 * entho;
+  R ecin = half * r0 * u0 * u0;
+  ecin = ecin + half * r0 * (t1 * t1);
+  ecin = ecin + half * r0 * (t2 * t2);
+  const R et0 = e0 + ecin;
+  const R S = left ? SL : SR;
+  const R dS = S - ustar;
+  const R nr = r0 * (S - u0), ne = (S - u0) * et0 - P0 * u0 + Ptotstar * ustar, ni = e0 * (S - u0);
+  R rs = zero, ets = zero, es = zero;
+  bool fulls = true;
+  if constexpr (sizeof(R) == 8) {
+    const double y = rcp_newton(dS);
+    rs = quot(nr, dS, y);
+    ets = quot(ne, dS, y);
+    es = quot(ni, dS, y);
+    auto mask = [](bool c) { return __builtin_amdgcn_ballot_w64(c); };  // (see any_not)
+    fulls = full || __builtin_expect((~mask(SL > zero) & (mask(SR > zero) | mask(ustar > zero)) &
+                                      (mask(!(abs_w(dS) >= 0x1p-90)) | mask(!(et0 < 0x1p800)))) != 0, 0);
   }
+  if (fulls) {
+    rs = div_w(nr, dS);
+    ets = div_w(ne, dS);
+    es = div_w(ni, dS);
+  }
+  const R ro = star ? rs : r0, uo = star ? ustar : u0, Ptoto = star ? Ptotstar : P0, etoto = star ? ets : et0;
+  const R eo = star ? es : e0;
   Flux6<R> g;
   g.f[0] = ro * uo;
   g.f[1] = ro * uo * uo + Ptoto;
@@ -710,10 +765,10 @@ __device__ __forceinline__ Flux6<R> riemann_exact(const Face<R>& L, const Face<R
 // to stay bitwise while avoiding a divide; the FP32-mixed path multiplies by
 // dt/dx in FP64.
 struct FluxScale {
-  double dt, dx, inv_dx, dtdx;
+  double dt, dx, inv_dx, dtdx, rcp_dx;
 };
 
-__host__ __device__ inline FluxScale make_scale(double dt, double dx) {
+__device__ inline FluxScale make_scale(double dt, double dx) {
   FluxScale s;
   s.dt = dt;
   s.dx = dx;
@@ -721,6 +776,7 @@ __host__ __device__ inline FluxScale make_scale(double dt, double dx) {
   int e = 0;
   const double m = __builtin_frexp(dx, &e);
   s.inv_dx = (m == 0.5) ? 1.0 / dx : 0.0;
+  s.rcp_dx = rcp_newton(dx);
   return s;
 }
 
@@ -736,7 +792,7 @@ __device__ __forceinline__ void scale_flux(const R* f, const FluxScale& s, doubl
 #pragma unroll
       for (int k = 0; k < N; ++k) out[k] = fd[k] * s.inv_dx;
     } else {
-      quotients<N>(fd, s.dx, out);
+      quotients<N>(fd, s.dx, s.rcp_dx, out);
     }
   } else {
 #pragma unroll
@@ -776,6 +832,38 @@ __device__ __forceinline__ Flux6<R> riemann_solve(const Face<R>& L, const Face<R
   if (c.riemann == kACOUSTIC) return riemann_acoustic(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc);
   if (c.riemann == kEXACT) return riemann_exact(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc, c.niter);
   return riemann_llf(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
+}
+
+// A value that all lanes of a wavefront share, held in scalar registers: a
+// constant computed by vector instructions otherwise keeps a vector register
+// (or two) for as long as it is used.
+__device__ __forceinline__ float scalar(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+}
+__device__ __forceinline__ double scalar(double x) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+template <typename R>
+__device__ __forceinline__ SolverConsts<R> scalar(SolverConsts<R> c) {
+  c.gamma = scalar(c.gamma);
+  c.smallr = scalar(c.smallr);
+  c.smallp = scalar(c.smallp);
+  c.entho = scalar(c.entho);
+  c.smallc2 = scalar(c.smallc2);
+  c.theta = scalar(c.theta);
+  c.smallc = scalar(c.smallc);
+  return c;
+}
+__device__ __forceinline__ FluxScale scalar(FluxScale s) {
+  s.dt = scalar(s.dt);
+  s.dx = scalar(s.dx);
+  s.inv_dx = scalar(s.inv_dx);
+  s.dtdx = scalar(s.dtdx);
+  s.rcp_dx = scalar(s.rcp_dx);
+  return s;
 }
 
 template <typename R, int RS>
@@ -840,9 +928,8 @@ __device__ __forceinline__ double cmpdt_cell(double u0, double u1, double u2, do
 // leaves w no such number).  A momentum too small for an exact remainder
 // changes nothing: its velocity is added to c >= 2^-60.
 __device__ __forceinline__ double cmpdt_w(double u0, double u1, double u2, double u3, double u4,
-                                          const HydroParams& hp) {
+                                          const HydroParams& hp, double smallp) {
   const double gamma = hp.gamma;
-  const double smallp = hp.smallc * hp.smallc / gamma;
   const double rho = fmax_f(u0, hp.smallr);
   auto wave = [&](double vx, double vy, double vz, auto speed) {
     double e = u4;
@@ -859,9 +946,14 @@ __device__ __forceinline__ double cmpdt_w(double u0, double u1, double u2, doubl
   const double y = rcp_newton(rho);
   double w = wave(quot(u1, rho, y), quot(u2, rho, y), quot(u3, rho, y),
                   [&](double c) { return sqrt_normal(quot(c, rho, y)); });
-  if (any_not(hi_word(rho) < hp.div_hi && w < 0x1p400))
+  if (any_not(hi_word(rho) < hp.div_hi, w < 0x1p400))
     w = wave(u1 / rho, u2 / rho, u3 / rho, [&](double c) { return __builtin_sqrt(c / rho); });
   return w;
+}
+
+__device__ __forceinline__ double cmpdt_w(double u0, double u1, double u2, double u3, double u4,
+                                          const HydroParams& hp) {
+  return cmpdt_w(u0, u1, u2, u3, u4, hp, hp.smallc * hp.smallc / hp.gamma);
 }
 
 // cmpdt_w of the FP32-mixed path: the same FP64 expression with the

@@ -10,15 +10,28 @@
 // threads cover the tile and the ring of cells next to its four sides (the
 // corners excluded), so the traced states of the halo cells that face the
 // tile are computed by a thread like any other.  Per plane:
-//   1. primitives of the next plane (tile + 2 cells of halo) -> LDS,
-//   2. each thread computes slopes and traced states of its own cell from
-//      its column (registers) and its x/y neighbours (LDS),
-//   3. left states are exchanged through LDS and x/y face fluxes solved,
-//   4. the z face below the cell is solved from the previous plane's traced
-//      state kept in registers, completing the update of the plane below,
-//   5. the new state is written and its cmpdt limit min-reduced (wavefront
-//      shuffles, then LDS across waves, then one 64-bit atomic min on the
-//      bit pattern of the positive double).
+//   1. each thread computes slopes and traced states of its own cell from
+//      its column (registers) and its x/y neighbours (LDS), and leaves the
+//      left states in LDS,
+//   2. the z face below the cell is solved from the previous plane's traced
+//      state kept in registers; with the x/y fluxes of that plane (LDS) it
+//      completes the plane below, whose new state is written and its cmpdt
+//      limit min-reduced (wavefront shuffles, then LDS across waves, then one
+//      64-bit atomic min on the bit pattern of the positive double),
+//   3. x/y faces are solved from the exchanged left states, their fluxes and
+//      the next plane's primitives (own cell and the tile's surroundings)
+//      left in LDS.
+// Two barriers a plane part these (the fluxes have LDS of their own, which
+// still lets three FP64 or four FP32-mixed workgroups share a CU); with the
+// primitives of two planes and one area for states and fluxes there were
+// five in FP64 and seven in FP32-mixed.
+//
+// What bounds it: vector issue (75% of the cycles, at the 2.0 GHz that this
+// load leaves of 2.4).  At 256^3 a pass takes 816 us in FP64 and 520 us in
+// FP32-mixed (918 and 578 with five and seven barriers, energies of both
+// sides of a face and two roots a face), at 512^3 6.3 ms.  Four FP64 waves a
+// SIMD (128 VGPRs, one LDS area more shared and a third barrier) ran 3%
+// slower.
 // Each primitive is computed by one ctoprim per cell per workgroup, each
 // face flux once, and every value keeps the reference's operation order, so
 // the FP64 path reproduces godfine1+unsplit on a uniform grid bit for bit.
@@ -87,8 +100,9 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
   constexpr int NT = tile_threads<TX, TY>();
   static_assert(NI % 64 == 0, "interior cells fill whole wavefronts");
 
-  __shared__ R qs[2][5][NQ];   // primitive planes (ring of 2)
-  __shared__ __align__(16) R xch[10][NE];  // exchange: traced left states, then fluxes
+  __shared__ R qs[5][NQ];                   // primitives of the plane whose states are traced
+  __shared__ __align__(16) R qm[10][NE];    // its traced left states: x, then y
+  __shared__ __align__(16) double fl[10][NE];  // fluxes (scaled): x, then y
   __shared__ double red[NT / 64];
 
   const long plane = (long)n * n;
@@ -103,7 +117,7 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
   // courant epilogue.
   // (ex, ey) are coordinates in the tile with its ring, interior 1..TX, 1..TY.
   enum { kNone = -1, kInterior = 0, kLeft, kRight, kBottom, kTop };
-  int ex = 0, ey = 0, kind = kNone;
+  int ex = 1, ey = 1, kind = kNone;
   if (t < NI) {
     ex = 1 + t % TX;
     ey = 1 + t / TX;
@@ -121,249 +135,239 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
       kind = h < TX ? kBottom : kTop;
     }
   }
-  const bool active = kind != kNone;
-  const int e = ey * EX + ex;  // own slot in the exchange area
-  const int xg = wrapi(x0 - 1 + ex, n), yg = wrapi(y0 - 1 + ey, n);
+  const int e = ey * EX + ex;  // own slot in the exchange areas
   const int qo = (ey + 1) * QX + (ex + 1);  // own cell in the primitive plane
   const bool inside = x0 + ex <= n && y0 + ey <= n;  // (interior threads) the cell is not a repeated one
 
+  // The ring's waves also convert the cells around the ring that its slopes
+  // read: a column or row outside each side and the ring's four corners.
+  constexpr int kOuter = 2 * (TX + TY) + 4;
+  static_assert(kOuter <= NT - NI, "one outer cell per thread of the ring's waves");
+  int ox = 1, oy = 1;
+  const bool outer = t >= NI && t < NI + kOuter;
+  if (outer) {
+    int h = t - NI;
+    if (h < 2 * TY) {
+      ox = h < TY ? -1 : TX + 2;
+      oy = 1 + h % TY;
+    } else if (h < 2 * (TX + TY)) {
+      h -= 2 * TY;
+      ox = 1 + h % TX;
+      oy = h < TX ? -1 : TY + 2;
+    } else {
+      h -= 2 * (TX + TY);
+      ox = h % 2 ? TX + 1 : 0;
+      oy = h / 2 ? TY + 1 : 0;
+    }
+  }
+  const int qx = (oy + 1) * QX + (ox + 1);
+
   // A plane of one variable is addressed from a scalar base by a 32-bit byte
   // offset that a thread keeps for the whole march (its own cell, and the
-  // one or two cells it converts to primitives), so that a load or store
-  // takes no vector instruction for its address.
+  // outer cell it converts), so that a load or store takes no vector
+  // instruction for its address.
   auto at = [&](const double* base, unsigned off) {
     return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off);
   };
-  const unsigned own = 8u * (unsigned)(yg * n + xg);
-  // cell t for every thread; the cells beyond NT go to the last threads (the
-  // ring's wave, which solves fewer faces), in reverse order
-  static_assert(NQ <= 2 * NT, "a plane is at most two cells per thread");
-  unsigned ld[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int c = k == 0 ? t : 2 * NT - 1 - t;
-    ld[k] = 8u * (unsigned)(wrapi(y0 - 2 + c / QX, n) * n + wrapi(x0 - 2 + c % QX, n));
-  }
+  auto offset = [&](int cx, int cy) { return 8u * (unsigned)(wrapi(y0 - 1 + cy, n) * n + wrapi(x0 - 1 + cx, n)); };
+  const unsigned own = offset(ex, ey), own2 = offset(ox, oy);
 
-  const SolverConsts<R> sc = make_consts<R>(hp);
-  const double dtxhalf = dt * 0.5;
-  const double smalle = hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0);
-  const R dtdx = (R)(dt / dx);
-  const FluxScale fs = make_scale(dt, dx);
+  const SolverConsts<R> sc = scalar(make_consts<R>(hp));
+  const double dtxhalf = scalar(dt * 0.5);
+  const double smalle = scalar(hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0));
+  const R dtdx = scalar((R)(dt / dx));
+  const FluxScale fs = scalar(make_scale(dt, dx));
 
-  // cooperative ctoprim of plane zp (periodic) into slot s
-  auto load_plane = [&](int zp, int s) {
+  struct Raw {
+    double v[5];
+  };
+  // keeps the compiler from forming 64-bit vector addresses ahead of the march
+  auto fixed = [](unsigned off) {
+    asm("" : "+v"(off));
+    return off;
+  };
+  auto load = [&](int zp, unsigned off) {
     const double* up = u + (long)wrapi(zp, n) * plane;
+    Raw r;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int c = k == 0 ? t : 2 * NT - 1 - t;
-      if (c >= NQ) continue;
-      const Prim<R> q = ctoprim_cell<R>(at(up, ld[k]), at(up + vstride, ld[k]), at(up + 2 * vstride, ld[k]),
-                                        at(up + 3 * vstride, ld[k]), at(up + 4 * vstride, ld[k]), 0.0, 0.0, 0.0,
-                                        dtxhalf, smalle, hp);
-      qs[s][0][c] = q.r;
-      qs[s][1][c] = q.u;
-      qs[s][2][c] = q.v;
-      qs[s][3][c] = q.w;
-      qs[s][4][c] = q.p;
-    }
+    for (int v = 0; v < 5; ++v) r.v[v] = at(up + v * vstride, fixed(off));
+    return r;
   };
-  auto read_q = [&](int s, int c) {
-    return Prim<R>{qs[s][0][c], qs[s][1][c], qs[s][2][c], qs[s][3][c], qs[s][4][c]};
+  auto prim = [&](const Raw& r) {
+    return ctoprim_cell<R>(r.v[0], r.v[1], r.v[2], r.v[3], r.v[4], 0.0, 0.0, 0.0, dtxhalf, smalle, hp);
+  };
+  auto put_q = [&](const Prim<R>& q, int c) {
+    qs[0][c] = q.r;
+    qs[1][c] = q.u;
+    qs[2][c] = q.v;
+    qs[3][c] = q.w;
+    qs[4][c] = q.p;
+  };
+  auto read_q = [&](int c) { return Prim<R>{qs[0][c], qs[1][c], qs[2][c], qs[3][c], qs[4][c]}; };
+  auto put_qm = [&](const Prim<R>& q, int row) {
+    qm[row][e] = q.r;
+    qm[row + 1][e] = q.u;
+    qm[row + 2][e] = q.v;
+    qm[row + 3][e] = q.w;
+    qm[row + 4][e] = q.p;
+  };
+  auto read_qm = [&](int row, int c) {
+    return Prim<R>{qm[row][c], qm[row + 1][c], qm[row + 2][c], qm[row + 3][c], qm[row + 4][c]};
   };
 
-  // own-column primitives at p-1 and p
-  Prim<R> qprev{}, qcur{};
+  // own-column primitives at p-1 and p; for minmod their difference in place
+  // of those at p-1 (every difference along z serves two planes)
+  Prim<R> qprev = prim(load(z0 - 2, own)), qcur = prim(load(z0 - 1, own));
+  if constexpr (ST == 1) qprev = qcur - qprev;
   // values carried from the previous plane
   Face<R> fz_left{};          // rotated qm_z of plane p-1
   double fz_prev[5] = {0, 0, 0, 0, 0};  // flux through the z face below plane p-1 (scaled)
-  double part_prev[5] = {0, 0, 0, 0, 0};  // (u + dFx) + dFy of plane p-1
   double wmax = 0.0;  // largest cmpdt wave speed of the new state
   ConsSums cs{0.0, 0.0, 0.0};  // courant_fine's sums of the new state (SUMS)
   const double vol = dx * dx * dx;
 
-  // prologue: planes z0-2 and z0-1
-  load_plane(z0 - 2, 0);
-  __syncthreads();
-  if (active) qprev = read_q(0, qo);
-  __syncthreads();
-  load_plane(z0 - 1, 1);
-  __syncthreads();
-  if (active) qcur = read_q(1, qo);
-
-  // One plane of the march.  kWaves: 0 for a wave of interior cells, 1 for
-  // the ring's wave; the cell kinds of a wave are then known at compile time
-  // (the cells of a wave are all interior or all ring, NI being a multiple
-  // of 64).
-  const bool active_run = active;
-  const int kind_run = kind;
-  auto plane_step = [&](auto waves_tag, int p) {
-    constexpr int kWaves = decltype(waves_tag)::value;
-    const bool interior = kWaves == 0;
-    const bool active = kWaves == 0 ? true : active_run;
-    const int kind = kWaves == 0 ? (int)kInterior : kind_run;
-    const int scur = (p - z0 + 2) & 1;  // slot of plane p (z0-2 -> 0, z0-1 -> 1)
-    const int snext = scur ^ 1;
-    const bool faces_xy = (p >= z0) && (p < z0 + TZ);
-    // FP32-mixed: the own cell's conserved state for the x/y update is
-    // loaded before the next plane, so its latency hides behind the plane's
-    // work (in FP64 the 10 more live registers would spill)
-    double upre[5] = {0, 0, 0, 0, 0};
-    if constexpr (sizeof(R) == 4) {
-      if (interior && faces_xy) {
-        const double* up = u + (long)wrapi(p, n) * plane;
-#pragma unroll
-        for (int v = 0; v < 5; ++v) upre[v] = at(up + v * vstride, own);
+  // The march over the planes z0-1 .. z0+TZ.  kWaves: 0 for a wave of
+  // interior cells, 1 for the ring's waves; the cell kinds of a wave are then
+  // known at compile time (the cells of a wave are all interior or all ring,
+  // NI being a multiple of 64).  A plane takes two barriers:
+  //   A: the primitives of plane p and the x and y fluxes of plane p-1 are
+  //      there.  Trace plane p, leave the left states; solve the z face
+  //      between p-1 and p and finish plane p-1.
+  //   B: the left states of plane p are there, and every reader of the
+  //      primitives and of the fluxes of p-1 is done.  Solve the x and y
+  //      faces of plane p, leave their fluxes and the primitives of p+1.
+  auto march = [&](auto waves_tag) {
+    constexpr bool interior = decltype(waves_tag)::value == 0;
+    // FP32-mixed has the registers to keep the own column's conserved state
+    // for its update two planes later (541 us at 256^3, 590 with it loaded
+    // again); in FP64 it is loaded again
+    constexpr bool kKeep = interior && sizeof(R) == 4;
+    const bool ring = kind > kInterior;
+    const bool xdir = kind == kLeft || kind == kRight;
+    if (interior || ring) put_q(qcur, qo);
+    if (!interior && outer) put_q(prim(load(z0 - 1, own2)), qx);
+    Raw next = load(z0, own);
+    Raw u0{}, uc{};
+    for (int p = z0 - 1;; ++p) {
+      const bool faces_xy = p >= z0 && p < z0 + TZ;
+      __syncthreads();  // A
+      const Prim<R> qnext = prim(next);
+      const Raw u1 = u0;  // conserved state of plane p-1 (kKeep)
+      if constexpr (kKeep) {
+        u0 = uc;
+        uc = next;
       }
+      Prim<R> qp_x{}, qp_y{};
+      {
+        const Prim<R> xm = read_q(qo - 1), xp = read_q(qo + 1);
+        const Prim<R> ym = read_q(qo - QX), yp = read_q(qo + QX);
+        const Prim<R> dqx = slope_prim<R, ST>(xm, qcur, xp, sc.slope_type, sc.theta);
+        const Prim<R> dqy = slope_prim<R, ST>(ym, qcur, yp, sc.slope_type, sc.theta);
+        Prim<R> dqz;
+        if constexpr (ST == 1) {
+          const Prim<R> drgt = qnext - qcur;
+          dqz = minmod(qprev, drgt);
+          qprev = drgt;
+        } else {
+          dqz = slope_prim<R, ST>(qprev, qcur, qnext, sc.slope_type, sc.theta);
+          qprev = qcur;
+        }
+        const Source<R> src = trace_sources<R, ST>(qcur, dqx, dqy, dqz, sc.gamma, sc.div_hi);
+        if constexpr (interior) {
+          Prim<R> q_x, q_y, qp_z, qm_z;
+          trace_dir(qcur, dqx, src, dtdx, sc.smallr, qp_x, q_x);
+          trace_dir(qcur, dqy, src, dtdx, sc.smallr, qp_y, q_y);
+          trace_dir(qcur, dqz, src, dtdx, sc.smallr, qp_z, qm_z);
+          if (faces_xy) {
+            put_qm(q_x, 0);
+            put_qm(q_y, 5);
+          }
+          // z face below plane p (between p-1 and p)
+          double fz[5] = {0, 0, 0, 0, 0};
+          if (p >= z0) {
+            const Flux6<R> g = riemann_fixed<R, RS>(fz_left, rotate(qp_z, 2), sc);
+            R fc[5];
+            unrotate(g, 2, fc);
+            scale_flux<5>(fc, fs, fz);  // hydro/umuscl.f90:153
+          }
+          // plane p-1 is complete: hydro/godunov_fine.f90:751-792 in idim
+          // order, unew = ((uold + dFx) + dFy) + dFz
+          if (p >= z0 + 1) {
+            const Raw old = kKeep ? u1 : load(p - 1, own);
+            double un[5];
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+              const double ux = old.v[v] + (fl[v][e] - fl[v][e + 1]);
+              const double uy = ux + (fl[5 + v][e] - fl[5 + v][e + EX]);
+              un[v] = uy + (fz_prev[v] - fz[v]);
+            }
+            if (inside) {
+              double* np = unew + (long)(p - 1) * plane;
+#pragma unroll
+              for (int v = 0; v < 5; ++v)
+                *reinterpret_cast<double*>(reinterpret_cast<char*>(np + v * vstride) + fixed(own)) = un[v];
+            }
+            if (d_dt_next) {
+              if constexpr (sizeof(R) == 8) wmax = fmax_f(wmax, cmpdt_w(un[0], un[1], un[2], un[3], un[4], hp, sc.smallp));
+              else wmax = fmax_f(wmax, cmpdt_w_fast(un[0], un[1], un[2], un[3], un[4], hp));
+            }
+            if (SUMS && inside) cons_add(cs, un[0], un[1], un[2], un[3], un[4], vol, hp.smallr);
+          }
+          fz_left = rotate(qm_z, 2);
+#pragma unroll
+          for (int v = 0; v < 5; ++v) fz_prev[v] = fz[v];
+        } else {
+          // a left or right ring cell feeds only an x face, a bottom or top
+          // one only a y face, and none a z face
+          Prim<R> q;
+          trace_dir(qcur, xdir ? dqx : dqy, src, dtdx, sc.smallr, qp_x, q);
+          if (ring && faces_xy) put_qm(q, xdir ? 0 : 5);
+        }
+      }
+      qcur = qnext;
+      if (p == z0 + TZ) break;
+      __syncthreads();  // B
+      if (faces_xy) {
+        if constexpr (interior) {
+          R fc[5];
+          double f[5];
+          unrotate(riemann_fixed<R, RS>(rotate(read_qm(0, e - 1), 0), rotate(qp_x, 0), sc), 0, fc);  // x-1/2
+          scale_flux<5>(fc, fs, f);  // hydro/umuscl.f90:106
+#pragma unroll
+          for (int v = 0; v < 5; ++v) fl[v][e] = f[v];
+          unrotate(riemann_fixed<R, RS>(rotate(read_qm(5, e - EX), 1), rotate(qp_y, 1), sc), 1, fc);  // y-1/2
+          scale_flux<5>(fc, fs, f);  // :129
+#pragma unroll
+          for (int v = 0; v < 5; ++v) fl[5 + v][e] = f[v];
+        } else if (kind == kRight || kind == kTop) {
+          // the right column's x faces and the top row's y faces in one pass
+          const Prim<R> l = read_qm(xdir ? 0 : 5, xdir ? e - 1 : e - EX);
+          auto face = [&](const Prim<R>& q) {
+            const Face<R> fx = rotate(q, 0), fy = rotate(q, 1);
+            return xdir ? fx : fy;
+          };
+          const Flux6<R> g = riemann_fixed<R, RS>(face(l), face(qp_x), sc);
+          R fcx[5], fcy[5], fc[5];
+          double f[5];
+          unrotate(g, 0, fcx);
+          unrotate(g, 1, fcy);
+#pragma unroll
+          for (int v = 0; v < 5; ++v) fc[v] = xdir ? fcx[v] : fcy[v];
+          scale_flux<5>(fc, fs, f);
+#pragma unroll
+          for (int v = 0; v < 5; ++v) fl[(xdir ? 0 : 5) + v][e] = f[v];
+        }
+      }
+      next = load(p + 2, own);
+      if (interior || ring) put_q(qcur, qo);
+      if (!interior && outer) put_q(prim(load(p + 1, own2)), qx);
     }
-    __syncthreads();
-    load_plane(p + 1, snext);
-    __syncthreads();
-    Prim<R> qnext{};
-    Prim<R> qp_x{}, qm_x{}, qp_y{}, qm_y{}, qp_z{}, qm_z{};
-    if (active) {
-      qnext = read_q(snext, qo);
-      const Prim<R> xm = read_q(scur, qo - 1), xp = read_q(scur, qo + 1);
-      const Prim<R> ym = read_q(scur, qo - QX), yp = read_q(scur, qo + QX);
-      const Prim<R> dqx = slope_prim<R, ST>(xm, qcur, xp, sc.slope_type, sc.theta);
-      const Prim<R> dqy = slope_prim<R, ST>(ym, qcur, yp, sc.slope_type, sc.theta);
-      const Prim<R> dqz = slope_prim<R, ST>(qprev, qcur, qnext, sc.slope_type, sc.theta);
-      const Source<R> src = trace_sources<R, ST>(qcur, dqx, dqy, dqz, sc.gamma, sc.div_hi);
-      if constexpr (kWaves == 0) {
-        trace_dir(qcur, dqx, src, dtdx, sc.smallr, qp_x, qm_x);
-        trace_dir(qcur, dqy, src, dtdx, sc.smallr, qp_y, qm_y);
-        trace_dir(qcur, dqz, src, dtdx, sc.smallr, qp_z, qm_z);
-      } else {
-        // a left or right ring cell feeds only an x face, a bottom or top one
-        // only a y face, and none a z face
-        const bool xdir = kind == kLeft || kind == kRight;
-        trace_dir(qcur, xdir ? dqx : dqy, src, dtdx, sc.smallr, qp_x, qm_x);
-        qp_y = qp_x;
-        qm_y = qm_x;
-      }
-    }
-    double part[5] = {0, 0, 0, 0, 0};
-    if (faces_xy) {
-      if (active) {
-        xch[0][e] = qm_x.r; xch[1][e] = qm_x.u; xch[2][e] = qm_x.v; xch[3][e] = qm_x.w; xch[4][e] = qm_x.p;
-        xch[5][e] = qm_y.r; xch[6][e] = qm_y.u; xch[7][e] = qm_y.v; xch[8][e] = qm_y.w; xch[9][e] = qm_y.p;
-      }
-      __syncthreads();
-      double fxs[5] = {0, 0, 0, 0, 0}, fys[5] = {0, 0, 0, 0, 0};
-      if (interior || kind == kRight) {  // x face at x-1/2
-        const int lo = e - 1;
-        const Prim<R> l{xch[0][lo], xch[1][lo], xch[2][lo], xch[3][lo], xch[4][lo]};
-        const Flux6<R> g = riemann_fixed<R, RS>(rotate(l, 0), rotate(qp_x, 0), sc);
-        R fc[5];
-        unrotate(g, 0, fc);
-        scale_flux<5>(fc, fs, fxs);  // hydro/umuscl.f90:106
-      }
-      if (interior || kind == kTop) {  // y face at y-1/2
-        const int lo = e - EX;
-        const Prim<R> l{xch[5][lo], xch[6][lo], xch[7][lo], xch[8][lo], xch[9][lo]};
-        const Flux6<R> g = riemann_fixed<R, RS>(rotate(l, 1), rotate(qp_y, 1), sc);
-        R fc[5];
-        unrotate(g, 1, fc);
-        scale_flux<5>(fc, fs, fys);  // :129
-      }
-      __syncthreads();
-      // The fluxes, in double, go through the exchange area reinterpreted:
-      // in FP64 it holds the x and the y fluxes side by side (one exchange),
-      // in FP32 one direction at a time.
-      double* fx_sh = reinterpret_cast<double*>(&xch[0][0]);
-      constexpr int FSTRIDE = NE;  // doubles per variable
-      static_assert(sizeof(R) * 10 * NE >= sizeof(double) * 5 * NE, "exchange area too small");
-      if constexpr (sizeof(R) == 8) {
-        double* fy_sh = fx_sh + 5 * FSTRIDE;
-        if (interior || kind == kRight) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) fx_sh[v * FSTRIDE + e] = fxs[v];
-        }
-        if (interior || kind == kTop) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) fy_sh[v * FSTRIDE + e] = fys[v];
-        }
-        __syncthreads();
-        if (interior) {
-          // hydro/godunov_fine.f90:770-772: unew = uold + (flux(i) - flux(i+1)), idim=1 then 2
-          const double* up = u + (long)wrapi(p, n) * plane;
-#pragma unroll
-          for (int v = 0; v < 5; ++v)
-            part[v] = at(up + v * vstride, own) + (fx_sh[v * FSTRIDE + e] - fx_sh[v * FSTRIDE + e + 1]);
-#pragma unroll
-          for (int v = 0; v < 5; ++v) part[v] = part[v] + (fy_sh[v * FSTRIDE + e] - fy_sh[v * FSTRIDE + e + EX]);
-        }
-      } else {
-        if (interior || kind == kRight) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) fx_sh[v * FSTRIDE + e] = fxs[v];
-        }
-        __syncthreads();
-        if (interior) {
-          // hydro/godunov_fine.f90:770-772, idim=1: unew = uold + (flux(i) - flux(i+1))
-#pragma unroll
-          for (int v = 0; v < 5; ++v) part[v] = upre[v] + (fx_sh[v * FSTRIDE + e] - fx_sh[v * FSTRIDE + e + 1]);
-        }
-        __syncthreads();
-        if (interior || kind == kTop) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) fx_sh[v * FSTRIDE + e] = fys[v];
-        }
-        __syncthreads();
-        if (interior) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) part[v] = part[v] + (fx_sh[v * FSTRIDE + e] - fx_sh[v * FSTRIDE + e + EX]);  // idim=2
-        }
-      }
-    }
-    // z face below plane p (between p-1 and p)
-    double fz[5] = {0, 0, 0, 0, 0};
-    if (interior && p >= z0) {
-      const Flux6<R> g = riemann_fixed<R, RS>(fz_left, rotate(qp_z, 2), sc);
-      R fc[5];
-      unrotate(g, 2, fc);
-      scale_flux<5>(fc, fs, fz);  // :153
-    }
-    // plane p-1 is complete: hydro/godunov_fine.f90:751-792 in idim order x, y, z
-    if (interior && p >= z0 + 1) {
-      double un[5];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) un[v] = part_prev[v] + (fz_prev[v] - fz[v]);  // idim=3
-      if (inside) {
-        double* np = unew + (long)(p - 1) * plane;
-#pragma unroll
-        for (int v = 0; v < 5; ++v)
-          *reinterpret_cast<double*>(reinterpret_cast<char*>(np + v * vstride) + own) = un[v];
-      }
-      if (d_dt_next) {
-        if constexpr (sizeof(R) == 8) wmax = fmax_f(wmax, cmpdt_w(un[0], un[1], un[2], un[3], un[4], hp));
-        else wmax = fmax_f(wmax, cmpdt_w_fast(un[0], un[1], un[2], un[3], un[4], hp));
-      }
-      if (SUMS && inside) cons_add(cs, un[0], un[1], un[2], un[3], un[4], vol, hp.smallr);
-    }
-    // carry to the next plane
-    fz_left = rotate(qm_z, 2);
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      fz_prev[v] = fz[v];
-      part_prev[v] = part[v];
-    }
-    qprev = qcur;
-    qcur = qnext;
   };
-  // The interior waves and the ring's wave run copies of the march with
+  // The interior waves and the ring's waves run copies of the march with
   // their cell kinds fixed, both meeting the same barriers in the same order
-  // (at 512^3: FP64 5.5% faster, FP32-mixed 3.5% once held to 128 VGPRs,
-  // where it takes 117).  A further copy for the planes between the first
-  // two and the last, with their tests folded, spilled 48 B in FP64 and ran
-  // 9% slower.
-  using kInteriorWaves = std::integral_constant<int, 0>;
-  using kRingWave = std::integral_constant<int, 1>;
-  if (t >= NI) {
-    for (int p = z0 - 1; p <= z0 + TZ; ++p) plane_step(kRingWave{}, p);
-  } else {
-    for (int p = z0 - 1; p <= z0 + TZ; ++p) plane_step(kInteriorWaves{}, p);
-  }
+  // (at 512^3: FP64 5.5% faster, FP32-mixed 3.5% once held to 128 VGPRs).
+  if (t >= NI) march(std::integral_constant<int, 1>{});
+  else march(std::integral_constant<int, 0>{});
 
   if (d_dt_next) {
     // wavefront max of w with shuffles, then across the block's waves; the
@@ -386,7 +390,7 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
 
 
 template <typename R, int TX, int TY, int RS, bool SUMS, int ST>
-// The register budget: 3 waves per SIMD in FP64 (166 VGPRs), 4 in FP32-mixed
+// The register budget: 3 waves per SIMD in FP64 (162 VGPRs), 4 in FP32-mixed
 // (at most 128).
 __global__ __launch_bounds__((tile_threads<TX, TY>()))
 __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3, 8))) void uniform_godunov_kernel(UniformArgs a, int ntx,
@@ -600,12 +604,12 @@ hipError_t launch_tile(const UniformArgs& a, int TZ, double* d_sums, hipStream_t
 // traced states only).  A CU takes its m workgroups' planes side by side
 // while they fit, then one after the other at full throughput.  The plane
 // times are those measured with 16x12 tiles (hllc, minmod): one workgroup
-// alone 3.9 us a plane in FP64 and 3.1 in FP32-mixed, three FP64 ones 7.2,
-// four FP32-mixed ones 5.6.  The estimate is within 10% of the measured time
+// alone 3.4 us a plane in FP64 and 2.4 in FP32-mixed, three FP64 ones 6.6,
+// four FP32-mixed ones 4.9.  The estimate is within 10% of the measured time
 // for n = 16..512 and z chunks of 2..128 planes.
 inline double level_estimate(long W, int TZ, bool fp32) {
   const double m = (double)((W + 255) / 256);
-  const double plane = fp32 ? (m <= 4 ? 2.3 + 0.82 * m : 1.48 * m) : (m <= 3 ? 2.2 + 1.7 * m : 2.4 * m);
+  const double plane = fp32 ? (m <= 4 ? 1.5 + 0.85 * m : 1.4 * m) : (m <= 3 ? 1.75 + 1.65 * m : 2.2 * m);
   return (TZ + 2) * plane;
 }
 
