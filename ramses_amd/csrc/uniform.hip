@@ -423,7 +423,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3, 8))) void batch_godun
   double* unew = sl.buf[par ^ 1];
   const int n = sl.n;
   const int ntx = (n + TX - 1) / TX, nty = (n + TY - 1) / TY;
-  const int local = b - a.blk0[s];
+  // neighbouring tiles of a slot on one XCD (see uniform_godunov_kernel)
+  const int local = (int)xcd_contiguous(b - a.blk0[s], a.blk0[s + 1] - a.blk0[s]);
   const int tx = local % ntx, ty = (local / ntx) % nty, z0 = local / (ntx * nty) * sl.tz;
   level_tile<R, TX, TY, RS, false, ST>(u, unew, n, sl.dx, st[kDtUse], st + kDtNext, a.hp, tx * TX, ty * TY, z0,
                                       min(sl.tz, n - z0));
