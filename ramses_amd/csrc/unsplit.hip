@@ -71,9 +71,9 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void unsplit_tile(UnsplitArgs a, long
   }
   const HydroParams hp = a.hp;
   const double dt = a.dt;
-  const SolverConsts<R> sc = make_consts<R>(hp);
-  const double dtxhalf = dt * 0.5;
-  const double smalle = hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0);  // hydro/umuscl.f90:884
+  const SolverConsts<R> sc = scalar(make_consts<R>(hp));
+  const double dtxhalf = scalar(dt * 0.5);
+  const double smalle = scalar(hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0));  // hydro/umuscl.f90:884
   // strides between cells and between variables
   const size_t cs = a.compact ? (size_t)nv * 5 : (size_t)nv, vs = a.compact ? (size_t)nv : (size_t)nv * 216;
   const size_t gcs = a.compact ? (size_t)nv * 3 : (size_t)nv;
@@ -99,7 +99,12 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void unsplit_tile(UnsplitArgs a, long
                                      dtxhalf, smalle, hp));
   }
   __syncthreads();
-  const R dtdx[3] = {(R)(dt / a.dx[0]), (R)(dt / a.dx[1]), (R)(dt / a.dx[2])};
+  // the scaling of a direction is formed again only where its dx differs from
+  // the last one's (two divisions each)
+  FluxScale fs = scalar(make_scale(dt, a.dx[0]));
+  R dtdx[3] = {(R)fs.dtdx, (R)fs.dtdx, (R)fs.dtdx};
+  if (a.dx[1] != a.dx[0]) dtdx[1] = scalar((R)(dt / a.dx[1]));
+  if (a.dx[2] != a.dx[0]) dtdx[2] = scalar((R)(dt / a.dx[2]));
   trace_tile<R, ST>(s, t, sc, dtdx);
   const size_t fvs = (size_t)nv * 27;
   for (int k = 0; k < 2; ++k) {
@@ -108,7 +113,8 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void unsplit_tile(UnsplitArgs a, long
     const int d = __builtin_amdgcn_readfirstlane(f) / 12;  // the four faces of a wavefront share their direction
     const Face<R> fl = get_side(s, f, 0, l), fr = get_side(s, f, 1, l);
     const Flux6<R> fg = riemann_fixed<R, RS>(fl, fr, sc);
-    const FluxScale fs = make_scale(dt, d == 0 ? a.dx[0] : (d == 1 ? a.dx[1] : a.dx[2]));
+    const double dxd = d == 0 ? a.dx[0] : (d == 1 ? a.dx[1] : a.dx[2]);
+    if (dxd != fs.dx) fs = scalar(make_scale(dt, dxd));
     const R val[7] = {fg.f[0], fg.f[1], fg.f[3], fg.f[4], fg.f[2], (R)0.5 * (fl.un + fr.un), fg.f[5]};  // :845
     double out[7];
     scale_flux<7>(val, fs, out);  // :106,111,129,153
