@@ -614,23 +614,29 @@ inline double level_estimate(long W, int TZ, bool fp32) {
   return (TZ + 2) * plane;
 }
 
+// The same for 32x16 tiles, of which a CU holds one: 6.2 us a plane in FP64,
+// 3.6 in FP32-mixed.
+inline double wide_estimate(long W, int TZ, bool fp32) { return (TZ + 2) * (fp32 ? 3.6 : 6.2) * (double)((W + 255) / 256); }
+
 // The z chunk with the least estimate, at least 2 planes and at most
 // max_blocks workgroups.  Long chunks repeat fewer planes, short ones fill
 // the chip: 2 planes at n <= 64, 6 at 96, 16 at 128, 32 at 256 and 64 at 512
 // in FP64 (with max_blocks out of the way), the fastest or within 3% of it
 // among those measured.
-inline int best_tz(int n, long tiles, bool fp32, long max_blocks) {
+inline int best_tz(int n, long tiles, bool fp32, long max_blocks, double (*estimate)(long, int, bool) = level_estimate,
+                   double* time = nullptr) {
   int best = n;
   double least = 1e300;
   for (int tz = n < 2 ? n : 2; tz <= n; ++tz) {
     const long W = tiles * ((n + tz - 1) / tz);
     if (W > max_blocks && tz < n) continue;
-    const double t = level_estimate(W, tz, fp32);
+    const double t = estimate(W, tz, fp32);
     if (t < least) {
       least = t;
       best = tz;
     }
   }
+  if (time) *time = least;
   return best;
 }
 
@@ -760,7 +766,15 @@ size_t uniform_sums_work_bytes(int n) { return (size_t)sums_blocks(n) * 3 * size
 // Tile choice: the launch-shape knob when it divides n, else 16x12 (three
 // interior waves and one ring wave: the ring's work is a third of a tile's,
 // against a half for 16x8), whose last tiles may reach past the level, or
-// 16x8 for n <= 24, where a third of a 16x12 tile's rows would.
+// 16x8 for n <= 24, where a third of a 16x12 tile's rows would.  Where the
+// estimates say so, 32x16, one workgroup of 10 waves on each CU, whose ring
+// is a fifth of the tile: at 64^3 (256 workgroups of 2 planes) 24 against 27
+// us in FP64 and 17 against 20 in FP32-mixed, at 128^3 100 against 118 in
+// FP64.  The margin leaves out 128^3 in FP32-mixed (63.5 against 68.2 us with
+// hllc and minmod, but 80.5 against 76.2 with llf and moncen); at 96^3 (58
+// against 56) and 192^3 (452 against 370) the estimates do.  Larger levels
+// take longer for a plane than the estimate says (512^3 FP32-mixed 4.4
+// against 3.8 ms): 16x12 above 160.
 hipError_t launch_uniform_godunov(const double* u, double* unew, int n, double dx, const double* d_dt,
                                   double* d_dt_next, const HydroParams& hp, bool fp32, hipStream_t s,
                                   double* partials, double* d_sums) {
@@ -771,11 +785,19 @@ hipError_t launch_uniform_godunov(const double* u, double* unew, int n, double d
   else if (tile == 3 || n < 16) { TX = 8; TY = 8; }
   else if (tile == 4 && n % 32 == 0) { TX = 32; TY = 16; }
   else if ((tile == 2 && n % 16 == 0) || (tile == 0 && n <= 24)) { TX = 16; TY = 8; }
-  const long tiles = (long)((n + TX - 1) / TX) * ((n + TY - 1) / TY);
+  const auto tiles_of = [n](int tx, int ty) { return (long)((n + tx - 1) / tx) * ((n + ty - 1) / ty); };
   // with sums, three doubles per workgroup have to fit the caller's buffer
   const long max_blocks = partials ? sums_blocks(n) : 0x7fffffffL;
   int TZ = tuning().level_tz;
-  if (TZ < 4 || TZ > n || n % TZ != 0 || tiles * (n / TZ) > max_blocks) TZ = best_tz(n, tiles, fp32, max_blocks);
+  if (tile == 0 && TZ == 0 && TY == 12 && n >= 32 && n <= 160) {
+    double narrow, wide;
+    best_tz(n, tiles_of(16, 12), fp32, max_blocks, level_estimate, &narrow);
+    best_tz(n, tiles_of(32, 16), fp32, max_blocks, wide_estimate, &wide);
+    if (wide < 0.93 * narrow) { TX = 32; TY = 16; }
+  }
+  const long tiles = tiles_of(TX, TY);
+  if (TZ < 4 || TZ > n || n % TZ != 0 || tiles * (n / TZ) > max_blocks) 
+    TZ = best_tz(n, tiles, fp32, max_blocks, TX == 32 && TY == 16 ? wide_estimate : level_estimate);
   if (fp32) {
     if (TY == 12) return launch_tile<float, 16, 12>(a, TZ, d_sums, s);
     if (TX == 32 && TY == 16) return launch_tile<float, 32, 16>(a, TZ, d_sums, s);
