@@ -385,16 +385,16 @@ RefineWork refine_work(void* work, long nslot, int nf) {
 
 // What a refinement is decided from.  With dn, dnf and dfree the level's and
 // the next level's oct counts and the free list {head, numbf, used_mem} are
-// in device memory and brought up to date there; else they are the host's.
+// read from device memory; else they are the host's.
 struct RefineScan {
   AmrTreeView t;
   const int* active;
   const int* fine;  // the next level's list
   const int* flag1;
   const int* dn;
-  int* dnf;
-  int* dfree;
-  int noct, nfine, head, numbf, cap, capacity;
+  const int* dnf;
+  const int* dfree;
+  int noct, nfine, head, numbf, capacity;
   int* error;  // or null
   RefineWork w;
 };
@@ -408,6 +408,10 @@ struct RefineScan {
 // amr/refine_utils.f90:415-423: error bit 4, nothing is modified).  A
 // refinement that would take the next level beyond `capacity` octs (the
 // workspace of a captured step) is refused the same way (error bit 8).
+//
+// A workgroup knows from the counts whether it works, and only the working
+// ones are waited for: one that starts after the decision has to read the
+// same counts, so nothing here writes them (refine_apply does).
 __global__ __launch_bounds__(kScanThreads) void refine_scan(RefineScan r) {
   __shared__ long long sh[kScanThreads / 64];
   __shared__ int last;
@@ -485,12 +489,6 @@ __global__ __launch_bounds__(kScanThreads) void refine_scan(RefineScan r) {
   r.w.ctrl[kFine] = nf;
   r.w.ctrl[kHead] = head;
   r.w.ctrl[kNumbf] = numbf;
-  if (ok && r.dnf) {
-    *r.dnf = nf - nk + nc;
-    r.dfree[0] = (int)(((long)head + nc) % r.cap);
-    if (nc > 0) r.dfree[2] = r.cap - (numbf - nc);  // make_grid_fine's last used_mem
-    r.dfree[1] = numbf - nc + nk;
-  }
 }
 
 struct RefineRun {
@@ -499,6 +497,8 @@ struct RefineRun {
   const int* active;  // level ilevel
   const int* dn;      // its oct count in device memory, or null
   int noct;
+  int* dnf;           // the next level's count and the free list in device memory, or null
+  int* dfree;
   int* fine;          // the next level's list
   int* pos;
   int* ring;
@@ -584,13 +584,22 @@ __device__ void kill_slot(const RefineRun& r, long p) {
 // grids that were free before, the killed ones clear the next level's and go
 // behind the free list's tail, and the next level's list is rebuilt:
 // survivors in order (from its copy; nothing moves when nothing is killed),
-// then the new octs; pos follows.  No part reads what another writes.
+// then the new octs; pos follows.  One thread brings counts in device memory
+// up to date, which this kernel takes from ctrl.  No part reads what another
+// writes.
 __global__ __launch_bounds__(128) void refine_apply(RefineRun r) {
   const int* ctrl = r.w.ctrl;
   if (!ctrl[kOk]) return;
   const long n = (long)((level_count(r.noct, r.dn) + 31) / 32) * 256;
   const long stride = (long)gridDim.x * blockDim.x, id = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const int nc = ctrl[kCreate], nk = ctrl[kKill], nf = ctrl[kFine];
+  if (id == 0 && r.dnf) {
+    const int numbf = ctrl[kNumbf];
+    *r.dnf = nf - nk + nc;
+    r.dfree[0] = (int)(((long)ctrl[kHead] + nc) % r.cap);
+    if (nc > 0) r.dfree[2] = r.cap - (numbf - nc);  // make_grid_fine's last used_mem
+    r.dfree[1] = numbf - nc + nk;
+  }
   for (long i = (nk > 0 ? 0 : nf) + id; i < (long)nf + nc; i += stride) {
     int g, at;
     if (i < nf) {
@@ -663,7 +672,7 @@ hipError_t launch_refine_fine(const int* active, int noct, int ilevel, const Amr
   hipError_t e = launch_set_ints((int*)w.done, 1, 0, s);
   if (e != hipSuccess) return e;
   const RefineScan scan{t, active, active_fine, flag1, nullptr, nullptr, nullptr, noct, nf, *head, *numbf,
-                        t.ngridmax, 0x7fffffff, nullptr, w};
+                        0x7fffffff, nullptr, w};
   const unsigned tiles = nblk(nslot, kScanTile) + nblk(nf, kScanTile);
   hipLaunchKernelGGL(refine_scan, dim3(tiles), dim3(kScanThreads), 0, s, scan);
   if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -676,7 +685,7 @@ hipError_t launch_refine_fine(const int* active, int noct, int ilevel, const Amr
     *nofree = 1;
     return hipSuccess;
   }
-  const RefineRun r{t, m, active, nullptr, noct, active_fine, pos, ring, t.ngridmax, uold, unew, t.ncell + 1, flag1,
+  const RefineRun r{t, m, active, nullptr, noct, nullptr, nullptr, active_fine, pos, ring, t.ngridmax, uold, unew, t.ncell + 1, flag1,
                     flag2, xg, __builtin_ldexp(1.0, -ilevel), interpol_type, interpol_var, smallr, d_error, w};
   hipLaunchKernelGGL(refine_apply, dim3(nblk(nslot, 128)), dim3(128), 0, s, r);
   if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -701,9 +710,9 @@ hipError_t launch_refine_fine_dev(const int* active, const int* dn_l, int ilevel
                                   int capacity, hipStream_t s) {
   RefineWork w = refine_work(work, refine_slots(capacity), capacity);
   w.done = done;
-  const RefineScan scan{t, active, active_fine, flag1, dn_l, dn_f, dfree, 0, 0, 0, 0, t.ngridmax, capacity, d_error, w};
+  const RefineScan scan{t, active, active_fine, flag1, dn_l, dn_f, dfree, 0, 0, 0, 0, capacity, d_error, w};
   hipLaunchKernelGGL(refine_scan, dim3(persist_blocks() / 2), dim3(kScanThreads), 0, s, scan);
-  const RefineRun r{t, m, active, dn_l, 0, active_fine, pos, ring, t.ngridmax, uold, unew, t.ncell + 1, flag1,
+  const RefineRun r{t, m, active, dn_l, 0, dn_f, dfree, active_fine, pos, ring, t.ngridmax, uold, unew, t.ncell + 1, flag1,
                     flag2, xg, __builtin_ldexp(1.0, -ilevel), interpol_type, interpol_var, smallr, d_error, w};
   hipLaunchKernelGGL(refine_apply, dim3(persist_blocks()), dim3(128), 0, s, r);
   return hipGetLastError();
