@@ -743,25 +743,28 @@ hipError_t launch_set_double(double* p, double v, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The workgroups that a launch with sums may have, 3 doubles each in the
+// caller's buffer (the level launch: 8x8 tiles of 4 planes).
+static long sums_blocks(int n) {
+  const long blocks = (long)n * n * n / 256;
+  return blocks > 1 ? blocks : 1;
+}
+size_t uniform_sums_work_bytes(int n) { return (size_t)sums_blocks(n) * 3 * sizeof(double); }
+
 hipError_t launch_courant(const double* u, int n, double dx, const HydroParams& hp, double* d_dt, hipStream_t s,
                           double* partials, double* d_sums) {
   const long ncell = (long)n * n * n;
   long blocks = (ncell + 255) / 256;
   if (blocks > 4096) blocks = 4096;
+  // n^3 need not be a multiple of 256: the kernel strides over the cells, so
+  // the workgroups that the buffer has room for take the rest
+  if (partials && blocks > sums_blocks(n)) blocks = sums_blocks(n);
   hipLaunchKernelGGL(courant_kernel, dim3((unsigned)blocks), dim3(256), 0, s, u, ncell, dx, hp, d_dt, partials);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !partials) return e;
   hipLaunchKernelGGL(cons_finish, dim3(1), dim3(256), 0, s, (const double*)partials, blocks, d_sums, 0);
   return hipGetLastError();
 }
-
-// Workgroups of the largest level launch with sums (8x8 tiles of 4 planes;
-// the courant reduction uses at most as many), 3 doubles each.
-long sums_blocks(int n) {
-  const long blocks = (long)n * n * n / 256;
-  return blocks > 1 ? blocks : 1;
-}
-size_t uniform_sums_work_bytes(int n) { return (size_t)sums_blocks(n) * 3 * sizeof(double); }
 
 // Tile choice: the launch-shape knob when it divides n, else 16x12 (three
 // interior waves and one ring wave: the ring's work is a third of a tile's,
