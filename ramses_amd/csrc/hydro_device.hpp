@@ -139,6 +139,11 @@ __device__ __forceinline__ float copysign_w(float a, float b) { return __builtin
 // that range quotients by one divisor share its reciprocal (five
 // instructions) and cost three each, bit for bit the same.  The callers test
 // the range and a wavefront with a lane outside it takes a / b instead.
+//
+// Both forms in one kernel take registers.  SHARE = false leaves the shared
+// one out: the oct-tree's staged solve spilled with it (FP64 hllc minmod:
+// 155 VGPRs without, 168 and 136 bytes of scratch with; 22.6 against 30.6 us
+// for 5,600 octs).
 __device__ __forceinline__ double rcp_newton(double d) {
   double y = __builtin_amdgcn_rcp(d);
   double e = __builtin_fma(-d, y, 1.0);
@@ -306,9 +311,9 @@ struct Source {
 // underflow.  Minmod (ST = 1) gives slopes of the positive p that are never
 // larger than p itself, and no -0.0, so it needs neither their test nor the
 // fixup that keeps a zero's sign.
-template <typename R, int ST>
+template <typename R, int ST, bool SHARE>
 __device__ __forceinline__ void pressure_terms(const Prim<R>& q, R px, R py, R pz, unsigned div_hi, R& ax, R& ay, R& az) {
-  if constexpr (sizeof(R) == 8) {
+  if constexpr (SHARE && sizeof(R) == 8) {
     const double y = rcp_newton(q.r);
     ax = quot(px, q.r, y);
     ay = quot(py, q.r, y);
@@ -332,12 +337,12 @@ __device__ __forceinline__ void pressure_terms(const Prim<R>& q, R px, R py, R p
   }
 }
 
-template <typename R, int ST = -1>
+template <typename R, int ST = -1, bool SHARE = true>
 __device__ __forceinline__ Source<R> trace_sources(const Prim<R>& q, const Prim<R>& dx_,
                                                    const Prim<R>& dy_, const Prim<R>& dz_, R gamma, unsigned div_hi) {
   const R r = q.r, u = q.u, v = q.v, w = q.w, p = q.p;
   R ax, ay, az;
-  pressure_terms<R, ST>(q, dx_.p, dy_.p, dz_.p, div_hi, ax, ay, az);
+  pressure_terms<R, ST, SHARE>(q, dx_.p, dy_.p, dz_.p, div_hi, ax, ay, az);
   Source<R> s;
   s.sr0 = -u * dx_.r - v * dy_.r - w * dz_.r - (dx_.u + dy_.v + dz_.w) * r;
   s.sp0 = -u * dx_.p - v * dy_.p - w * dz_.p - (dx_.u + dy_.v + dz_.w) * gamma * p;
@@ -390,9 +395,9 @@ __device__ __forceinline__ Face<R> rotate(const Prim<R>& q, int d) {
 // is zero, infinite, a NaN (v_frexp gives them exponent 0, and the fixup
 // their quotients) or in [2^-800, 2^800): a wavefront with a lane outside
 // divides in full.  y = rcp_newton(d) (FP64).
-template <int N, typename R>
+template <int N, bool SHARE = true, typename R>
 __device__ __forceinline__ void quotients(const R* n, R d, R y, R* out) {
-  if constexpr (sizeof(R) == 8) {
+  if constexpr (SHARE && sizeof(R) == 8) {
     int lo = 0, hi = 0;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
@@ -416,10 +421,10 @@ struct Flux6 {
 
 // The sound speeds sqrt(gamma*p/rho) of both sides of a face, p and rho at
 // or above their floors.
-template <typename R>
+template <typename R, bool SHARE>
 __device__ __forceinline__ void sound_speeds(R rl, R pl, R rr, R pr, R gamma, unsigned div_hi, R& cl, R& cr) {
   const R nl = gamma * pl, nr = gamma * pr;
-  if constexpr (sizeof(R) == 8) {
+  if constexpr (SHARE && sizeof(R) == 8) {
     cl = sqrt_normal(quot(nl, rl, rcp_newton(rl)));
     cr = sqrt_normal(quot(nr, rr, rcp_newton(rr)));
     if (!any_not(max_u(max_u(hi_word(rl), hi_word(rr)), max_u(hi_word(pl), hi_word(pr))) < div_hi)) return;
@@ -429,10 +434,10 @@ __device__ __forceinline__ void sound_speeds(R rl, R pl, R rr, R pr, R gamma, un
 }
 
 // The larger of the two, with one root in FP64 (see riemann_hllc).
-template <typename R>
+template <typename R, bool SHARE>
 __device__ __forceinline__ R larger_sound_speed(R rl, R pl, R rr, R pr, R gamma, unsigned div_hi) {
   const R nl = gamma * pl, nr = gamma * pr;
-  if constexpr (sizeof(R) == 8) {
+  if constexpr (SHARE && sizeof(R) == 8) {
     const R c = sqrt_normal(fmax_f(quot(nl, rl, rcp_newton(rl)), quot(nr, rr, rcp_newton(rr))));
     if (!any_not(max_u(max_u(hi_word(rl), hi_word(rr)), max_u(hi_word(pl), hi_word(pr))) < div_hi)) return c;
   }
@@ -440,14 +445,14 @@ __device__ __forceinline__ R larger_sound_speed(R rl, R pl, R rr, R pr, R gamma,
 }
 
 // riemann_llf: hydro/godunov_utils.f90:660-820
-template <typename R>
+template <typename R, bool SHARE>
 __device__ __forceinline__ Flux6<R> riemann_llf(const Face<R>& L, const Face<R>& Rt, R gamma, R smallr,
                                                 R smallp, R entho, unsigned div_hi) {
   const R half = (R)0.5;
   const R rl = fmax_f(L.r, smallr), ul = L.un, pl = fmax_f(L.p, rl * smallp);
   const R rr = fmax_f(Rt.r, smallr), ur = Rt.un, pr = fmax_f(Rt.p, rr * smallp);
   R cl, cr;
-  sound_speeds(rl, pl, rr, pr, gamma, div_hi, cl, cr);
+  sound_speeds<R, SHARE>(rl, pl, rr, pr, gamma, div_hi, cl, cr);
   const R cmax = fmax_f(abs_w(ul) + cl, abs_w(ur) + cr);
   R uL[6], uR[6], fL[6], fR[6];
   uL[0] = L.r;
@@ -484,13 +489,13 @@ __device__ __forceinline__ Flux6<R> riemann_llf(const Face<R>& L, const Face<R>&
 }
 
 // riemann_hll: hydro/godunov_utils.f90:825-983
-template <typename R>
+template <typename R, bool SHARE>
 __device__ __forceinline__ Flux6<R> riemann_hll(const Face<R>& L, const Face<R>& Rt, R gamma, R smallr,
                                                 R smallp, R entho, unsigned div_hi) {
   const R half = (R)0.5, zero = (R)0;
   const R rl = fmax_f(L.r, smallr), ul = L.un, pl = fmax_f(L.p, rl * smallp);
   const R rr = fmax_f(Rt.r, smallr), ur = Rt.un, pr = fmax_f(Rt.p, rr * smallp);
-  const R c = larger_sound_speed(rl, pl, rr, pr, gamma, div_hi);
+  const R c = larger_sound_speed<R, SHARE>(rl, pl, rr, pr, gamma, div_hi);
   const R SL = fmin_f(fmin_f(ul, ur) - c, zero);
   const R SR = fmax_f(fmax_f(ul, ur) + c, zero);
   R uL[6], uR[6], fL[6], fR[6];
@@ -527,8 +532,8 @@ __device__ __forceinline__ Flux6<R> riemann_hll(const Face<R>& L, const Face<R>&
 #pragma unroll
   for (int n = 0; n < 6; ++n) num[n] = SR * fL[n] - SL * fR[n] + SR * SL * (uR[n] - uL[n]);
   R y{};
-  if constexpr (sizeof(R) == 8) y = rcp_newton(den);
-  quotients<6>(num, den, y, g.f);
+  if constexpr (SHARE && sizeof(R) == 8) y = rcp_newton(den);
+  quotients<6, SHARE>(num, den, y, g.f);
   return g;
 }
 
@@ -546,7 +551,7 @@ __device__ __forceinline__ Flux6<R> riemann_hll(const Face<R>& L, const Face<R>&
 // only the velocities can be tiny, and the test of ustar's numerator excludes
 // it.  |S - ustar| >= 2^-90 and a total energy below 2^800 (which also
 // excludes infinite and NaN tangential velocities) close the star state.
-template <typename R>
+template <typename R, bool SHARE>
 __device__ __forceinline__ Flux6<R> riemann_hllc(const Face<R>& L, const Face<R>& Rt, R gamma, R smallr,
                                                  R smallp, R entho, R smallc2, unsigned div_hi) {
   const R half = (R)0.5, zero = (R)0;
@@ -568,7 +573,7 @@ __device__ __forceinline__ Flux6<R> riemann_hllc(const Face<R>& L, const Face<R>
     den = rcr + rcl;
   };
   bool full = true;
-  if constexpr (sizeof(R) == 8) {
+  if constexpr (SHARE && sizeof(R) == 8) {
     // max(sqrt(a), sqrt(b)) is sqrt(max(a, b)): a correctly rounded root is
     // monotonic
     const R cl2 = floor_at(quot(gamma * Pl, rl, rcp_newton(rl)), smallc2);
@@ -604,7 +609,7 @@ __device__ __forceinline__ Flux6<R> riemann_hllc(const Face<R>& L, const Face<R>
   const R nr = r0 * (S - u0), ne = (S - u0) * et0 - P0 * u0 + Ptotstar * ustar, ni = e0 * (S - u0);
   R rs = zero, ets = zero, es = zero;
   bool fulls = true;
-  if constexpr (sizeof(R) == 8) {
+  if constexpr (SHARE && sizeof(R) == 8) {
     const double y = rcp_newton(dS);
     rs = quot(nr, dS, y);
     ets = quot(ne, dS, y);
@@ -782,7 +787,7 @@ __device__ inline FluxScale make_scale(double dt, double dx) {
 
 // N values of a face at once: one scalar branch for all, and where dx is no
 // power of two its reciprocal shared by their divisions.
-template <int N, typename R>
+template <int N, bool SHARE = true, typename R>
 __device__ __forceinline__ void scale_flux(const R* f, const FluxScale& s, double* out) {
   if constexpr (sizeof(R) == 8) {
     double fd[N];
@@ -792,7 +797,7 @@ __device__ __forceinline__ void scale_flux(const R* f, const FluxScale& s, doubl
 #pragma unroll
       for (int k = 0; k < N; ++k) out[k] = fd[k] * s.inv_dx;
     } else {
-      quotients<N>(fd, s.dx, s.rcp_dx, out);
+      quotients<N, SHARE>(fd, s.dx, s.rcp_dx, out);
     }
   } else {
 #pragma unroll
@@ -801,16 +806,16 @@ __device__ __forceinline__ void scale_flux(const R* f, const FluxScale& s, doubl
 }
 
 // Solver constants in working precision.
-template <typename R>
+template <typename R, bool SHARE = true>
 struct SolverConsts {
   R gamma, smallr, smallp, entho, smallc2, theta, smallc;
   unsigned div_hi;
   int riemann, slope_type, niter;
 };
 
-template <typename R>
-__host__ __device__ inline SolverConsts<R> make_consts(const HydroParams& hp) {
-  SolverConsts<R> c;
+template <typename R, bool SHARE = true>
+__host__ __device__ inline SolverConsts<R, SHARE> make_consts(const HydroParams& hp) {
+  SolverConsts<R, SHARE> c;
   c.gamma = (R)hp.gamma;
   c.smallr = (R)hp.smallr;
   c.smallp = (R)(hp.smallc * hp.smallc / hp.gamma);  // :683, :1017
@@ -825,13 +830,14 @@ __host__ __device__ inline SolverConsts<R> make_consts(const HydroParams& hp) {
   return c;
 }
 
-template <typename R>
-__device__ __forceinline__ Flux6<R> riemann_solve(const Face<R>& L, const Face<R>& Rt, const SolverConsts<R>& c) {
-  if (c.riemann == kHLLC) return riemann_hllc(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc2, c.div_hi);
-  if (c.riemann == kHLL) return riemann_hll(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
+template <typename R, bool SHARE>
+__device__ __forceinline__ Flux6<R> riemann_solve(const Face<R>& L, const Face<R>& Rt,
+                                                  const SolverConsts<R, SHARE>& c) {
+  if (c.riemann == kHLLC) return riemann_hllc<R, SHARE>(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc2, c.div_hi);
+  if (c.riemann == kHLL) return riemann_hll<R, SHARE>(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
   if (c.riemann == kACOUSTIC) return riemann_acoustic(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc);
   if (c.riemann == kEXACT) return riemann_exact(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc, c.niter);
-  return riemann_llf(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
+  return riemann_llf<R, SHARE>(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
 }
 
 // A value that all lanes of a wavefront share, held in scalar registers: a
@@ -866,12 +872,13 @@ __device__ __forceinline__ FluxScale scalar(FluxScale s) {
   return s;
 }
 
-template <typename R, int RS>
-__device__ __forceinline__ Flux6<R> riemann_fixed(const Face<R>& L, const Face<R>& Rt, const SolverConsts<R>& c) {
-  if constexpr (RS == kHLLC) return riemann_hllc(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc2, c.div_hi);
-  else if constexpr (RS == kHLL) return riemann_hll(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
+template <typename R, int RS, bool SHARE>
+__device__ __forceinline__ Flux6<R> riemann_fixed(const Face<R>& L, const Face<R>& Rt,
+                                                  const SolverConsts<R, SHARE>& c) {
+  if constexpr (RS == kHLLC) return riemann_hllc<R, SHARE>(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.smallc2, c.div_hi);
+  else if constexpr (RS == kHLL) return riemann_hll<R, SHARE>(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
   else if constexpr (RS == kDynamicRiemann) return riemann_solve(L, Rt, c);
-  else return riemann_llf(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
+  else return riemann_llf<R, SHARE>(L, Rt, c.gamma, c.smallr, c.smallp, c.entho, c.div_hi);
 }
 
 // Conservative-variable flux of a face in (rho, mx, my, mz, E) order

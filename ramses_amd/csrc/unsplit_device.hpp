@@ -100,7 +100,7 @@ __device__ void slope_27(const Ctx& c, int i, int j, int k, Prim<R>& dqx, Prim<R
   dqz = Prim<R>{oz[0], oz[1], oz[2], oz[3], oz[4]};
 }
 
-template <typename R>
+template <bool SHARE, typename R>
 __device__ __forceinline__ void store_face(double* flux, double* tmp, size_t fbase, size_t tbase, size_t fvs,
                                            int d, const Flux6<R>& g, const Face<R>& L, const Face<R>& Rt,
                                            const FluxScale& fs) {
@@ -108,8 +108,8 @@ __device__ __forceinline__ void store_face(double* flux, double* tmp, size_t fba
   unrotate(g, d, fc);
   const R t[2] = {(R)0.5 * (L.un + Rt.un), g.f[5]};  // :845
   double o[5], ot[2];
-  scale_flux<5>(fc, fs, o);                          // :106,129,153
-  scale_flux<2>(t, fs, ot);                          // :111
+  scale_flux<5, SHARE>(fc, fs, o);                   // :106,129,153
+  scale_flux<2, SHARE>(t, fs, ot);                   // :111
 #pragma unroll
   for (int v = 0; v < 5; ++v) flux[fbase + (size_t)v * fvs] = o[v];
   tmp[tbase] = ot[0];
@@ -121,9 +121,9 @@ __device__ __forceinline__ void store_face(double* flux, double* tmp, size_t fba
 // with a flagged cell on either side stores a zero flux: the value the
 // reference's reset leaves there (hydro/godunov_fine.f90:720-749).
 // Ctx supplies prim(i,j,k) and nv (RowCtx).  ST: the 7-point slope type
-// fixed at compile time, or -1 (see slope1).
-template <typename R, int D, int RS, bool S27, bool ZR, int ST, typename Ctx>
-__device__ __forceinline__ void row_faces(const Ctx& c, const SolverConsts<R>& sc, int a1, int b1,
+// fixed at compile time, or -1 (see slope1).  SHARE: see rcp_newton.
+template <typename R, int D, int RS, bool S27, bool ZR, int ST, bool SHARE, typename Ctx>
+__device__ __forceinline__ void row_faces(const Ctx& c, const SolverConsts<R, SHARE>& sc, int a1, int b1,
                                           R dtdx, double* flux, double* tmp, size_t fvs, const FluxScale fs,
                                           const unsigned char* ok) {
   constexpr int T1 = (D == 0) ? 1 : 0;  // first transverse axis
@@ -160,7 +160,7 @@ __device__ __forceinline__ void row_faces(const Ctx& c, const SolverConsts<R>& s
     const Prim<R>& dqx = (D == 0) ? dqd : dq1;
     const Prim<R>& dqy = (D == 1) ? dqd : ((D == 0) ? dq1 : dq2);
     const Prim<R>& dqz = (D == 2) ? dqd : dq2;
-    const Source<R> src = trace_sources<R, S27 ? -1 : ST>(qb, dqx, dqy, dqz, sc.gamma, sc.div_hi);
+    const Source<R> src = trace_sources<R, S27 ? -1 : ST, SHARE>(qb, dqx, dqy, dqz, sc.gamma, sc.div_hi);
     Prim<R> qp, qm;
     trace_dir(qb, dqd, src, dtdx, sc.smallr, qp, qm);
     if (s >= 1) {
@@ -168,7 +168,7 @@ __device__ __forceinline__ void row_faces(const Ctx& c, const SolverConsts<R>& s
       const Face<R> fr = rotate(qp, D);
       const Flux6<R> g = riemann_fixed<R, RS>(fl_prev, fr, sc);
       const size_t fslot = (size_t)((i - 1) + 3 * ((j - 1) + 3 * (k - 1))) * c.nv;
-      store_face(flux, tmp, fslot + (size_t)D * 5 * fvs, fslot + (size_t)D * 2 * fvs, fvs, D, g, fl_prev, fr, fs);
+      store_face<SHARE>(flux, tmp, fslot + (size_t)D * 5 * fvs, fslot + (size_t)D * 2 * fvs, fvs, D, g, fl_prev, fr, fs);
       if (ZR) {
         int li = i, lj = j, lk = k;  // left cell of the face
         if (D == 0) --li; else if (D == 1) --lj; else --lk;
@@ -187,8 +187,8 @@ __device__ __forceinline__ void row_faces(const Ctx& c, const SolverConsts<R>& s
 // Slopes of cell (i,j,k) and its traced states along D (qp on the minus
 // side, qm on the plus side), exactly as row_faces computes them for a cell
 // of a row: the same routines on the same primitives.
-template <typename R, int D, bool S27, int ST, typename Ctx>
-__device__ __forceinline__ void trace_cell(const Ctx& c, const SolverConsts<R>& sc, int i, int j, int k,
+template <typename R, int D, bool S27, int ST, bool SHARE, typename Ctx>
+__device__ __forceinline__ void trace_cell(const Ctx& c, const SolverConsts<R, SHARE>& sc, int i, int j, int k,
                                            R dtdx, Prim<R>& qp, Prim<R>& qm) {
   const Prim<R> q = c.prim(i, j, k);
   Prim<R> dqx, dqy, dqz;
@@ -199,13 +199,13 @@ __device__ __forceinline__ void trace_cell(const Ctx& c, const SolverConsts<R>& 
     dqy = slope_prim<R, ST>(c.prim(i, j - 1, k), q, c.prim(i, j + 1, k), sc.slope_type, sc.theta);
     dqz = slope_prim<R, ST>(c.prim(i, j, k - 1), q, c.prim(i, j, k + 1), sc.slope_type, sc.theta);
   }
-  const Source<R> src = trace_sources<R, S27 ? -1 : ST>(q, dqx, dqy, dqz, sc.gamma, sc.div_hi);
+  const Source<R> src = trace_sources<R, S27 ? -1 : ST, SHARE>(q, dqx, dqy, dqz, sc.gamma, sc.div_hi);
   trace_dir(q, D == 0 ? dqx : (D == 1 ? dqy : dqz), src, dtdx, sc.smallr, qp, qm);
 }
 
 // The face of direction D whose right cell is (i,j,k) (ZR: see row_faces).
-template <typename R, int D, int RS, bool S27, bool ZR, int ST, typename Ctx>
-__device__ __forceinline__ void face_dir(const Ctx& c, const SolverConsts<R>& sc, int i, int j, int k,
+template <typename R, int D, int RS, bool S27, bool ZR, int ST, bool SHARE, typename Ctx>
+__device__ __forceinline__ void face_dir(const Ctx& c, const SolverConsts<R, SHARE>& sc, int i, int j, int k,
                                          R dtdx, double* flux, double* tmp, size_t fvs, const FluxScale fs,
                                          const unsigned char* ok) {
   constexpr int di = D == 0, dj = D == 1, dk = D == 2;
@@ -215,7 +215,7 @@ __device__ __forceinline__ void face_dir(const Ctx& c, const SolverConsts<R>& sc
   const Face<R> fl = rotate(qmL, D), fr = rotate(qpR, D);
   const Flux6<R> g = riemann_fixed<R, RS>(fl, fr, sc);
   const size_t fslot = (size_t)((i - 1) + 3 * ((j - 1) + 3 * (k - 1))) * c.nv;
-  store_face(flux, tmp, fslot + (size_t)D * 5 * fvs, fslot + (size_t)D * 2 * fvs, fvs, D, g, fl, fr, fs);
+  store_face<SHARE>(flux, tmp, fslot + (size_t)D * 5 * fvs, fslot + (size_t)D * 2 * fvs, fvs, D, g, fl, fr, fs);
   if (ZR && (ok[(size_t)cell6(i - di, j - dj, k - dk) * c.nv] || ok[(size_t)cell6(i, j, k) * c.nv])) {
 #pragma unroll
     for (int v = 0; v < 5; ++v) flux[fslot + (size_t)D * 5 * fvs + (size_t)v * fvs] = 0.0;
@@ -258,7 +258,7 @@ __device__ __forceinline__ void face_task(const UnsplitArgs& a, long t, long ngr
   c.dtxhalf = dt * 0.5;
   c.smalle = hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0);  // hydro/umuscl.f90:884
   c.hp = &hp;
-  const SolverConsts<R> sc = make_consts<R>(hp);
+  const SolverConsts<R, !ZR> sc = make_consts<R, !ZR>(hp);  // the staged solve (ZR) divides in full
   double* flux = a.flux + gidx * gsz_f + l;
   double* tmp = a.tmp + gidx * gsz_t + l;
   const size_t fvs = (size_t)nv * 27;
@@ -303,7 +303,7 @@ __device__ __forceinline__ void unsplit_task(const UnsplitArgs& a, long t, long 
   c.dtxhalf = dt * 0.5;
   c.smalle = hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0);  // :884
   c.hp = &hp;
-  const SolverConsts<R> sc = make_consts<R>(hp);
+  const SolverConsts<R, !ZR> sc = make_consts<R, !ZR>(hp);  // the staged solve (ZR) divides in full
 
   double* flux = a.flux + gidx * gsz_f + l;
   double* tmp = a.tmp + gidx * gsz_t + l;
