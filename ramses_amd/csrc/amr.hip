@@ -418,8 +418,11 @@ void with_solver(int riemann, F f) {
   }
 }
 
-constexpr unsigned kRefluxSplit = 1u << 16;
-__host__ __device__ inline bool reflux_from_coarse(unsigned nf, unsigned nc) { return 8ULL * nc <= 6ULL * nf; }
+constexpr unsigned kRefluxSplit = 1u << 16;  // (see reflux_tasks)
+constexpr unsigned kRefluxFew = 1u << 12;
+__host__ __device__ inline bool reflux_from_coarse(unsigned nf, unsigned nc) {
+  return nc <= kRefluxFew || 8ULL * nc <= 6ULL * nf;
+}
 
 // Conservative correction of the coarser leaf cells next to the level's
 // octs.  A coarse leaf c receives from each fine oct o that sits across one
@@ -457,9 +460,12 @@ __device__ __forceinline__ void reflux_cell(const AmrLevelArgs& a, int g, int in
 #pragma unroll
   for (int in = 1; in <= 6; ++in) {
     const int ax = (in - 1) >> 1, plus = (in - 1) & 1;
-    // c is on o's minus side when n is c's plus neighbour
-    const long long key = (long long)(pz[in - 1] / a.nv) * 6 + 2 * ax + (plus ? 0 : 1);
-    kp[in - 1] = so[in - 1] > 0 ? key << 32 | (long long)pz[in - 1] : kNone;
+    kp[in - 1] = kNone;
+    if (any_lane(so[in - 1] > 0)) {
+      // c is on o's minus side when n is c's plus neighbour
+      const long long key = (long long)(pz[in - 1] / a.nv) * 6 + 2 * ax + (plus ? 0 : 1);
+      if (so[in - 1] > 0) kp[in - 1] = key << 32 | (long long)pz[in - 1];
+    }
   }
   auto order = [&](int i, int k) {
     const long long lo = kp[i] < kp[k] ? kp[i] : kp[k], hi = kp[i] < kp[k] ? kp[k] : kp[i];
@@ -473,6 +479,23 @@ __device__ __forceinline__ void reflux_cell(const AmrLevelArgs& a, int g, int in
   const int nv = a.nv;
   const size_t fvs = (size_t)nv * 27;
   const double oneontwotondim = 1.0 / 8.0;
+  // The oct side's 2x2 faces: the transverse coordinates run over {1,2} and
+  // the normal one is 1 (side 0, the oct's minus face) or 3 (side 1).  Formed
+  // only for as many contributors as some lane has.
+  const double* fe[6];
+  int f1[6], f2[6];  // steps along the lower and the upper transverse axis
+#pragma unroll
+  for (int e = 0; e < 6; ++e) {
+    fe[e] = nullptr;
+    f1[e] = f2[e] = 0;
+    if (any_lane(kp[e] != kNone)) {
+      const int key = (int)(kp[e] >> 32), pos = (int)kp[e];
+      const int b = key / 6, d = (key - 6 * b) >> 1, side = key & 1;
+      f1[e] = d == 0 ? 3 * nv : nv;
+      f2[e] = d == 2 ? 3 * nv : 9 * nv;
+      fe[e] = a.flux + (size_t)b * fvs * 15 + (pos - b * nv) + (27 * 5 * d + side * (d == 0 ? 2 : (d == 1 ? 6 : 18))) * nv;
+    }
+  }
   // All contributions are loaded first (independent loads, issued together),
   // then summed in the reference's order: contributor e by key, and within
   // it the 4 faces of the oct side in (k3, j3, i3) loop order.
@@ -481,41 +504,32 @@ __device__ __forceinline__ void reflux_cell(const AmrLevelArgs& a, int g, int in
 #pragma unroll
     for (int e = 0; e < 6; ++e) {
       if (kp[e] == kNone) break;
-      const int key = (int)(kp[e] >> 32), pos = (int)kp[e];
-      const int d = (key % 6) >> 1, side = key & 1;
-      const int b = pos / nv, lane = pos % nv;
-      const double* flux = a.flux + (size_t)b * fvs * 15 + lane + (size_t)27 * (v + 5 * d) * nv;
-      // the side's 2x2 faces: the transverse coordinates run over {1,2} and the
-      // normal one is 1 (side 0, the oct's minus face) or 3 (side 1)
+      const double* flux = fe[e] + (size_t)v * fvs;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int t1 = 1 + (q & 1), t2 = 1 + (q >> 1);  // inner loop first
-        int i3, j3, k3;
-        if (d == 0) { i3 = side ? 3 : 1; j3 = t1; k3 = t2; }
-        else if (d == 1) { i3 = t1; j3 = side ? 3 : 1; k3 = t2; }
-        else { i3 = t1; j3 = t2; k3 = side ? 3 : 1; }
-        fv[e][q] = flux[fslot(i3, j3, k3) * nv];
-      }
-  }
-  double s = a.unew[(long)v * a.ustride + c];
+      for (int q = 0; q < 4; ++q) fv[e][q] = flux[(q & 1) * f1[e] + (q >> 1) * f2[e]];
+    }
+    double s = a.unew[(long)v * a.ustride + c];
 #pragma unroll
-  for (int e = 0; e < 6; ++e) {
-    if (kp[e] == kNone) break;
-    const int side = (int)(kp[e] >> 32) & 1;
+    for (int e = 0; e < 6; ++e) {
+      if (kp[e] == kNone) break;
+      const int side = (int)(kp[e] >> 32) & 1;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) s = side ? s + fv[e][q] * oneontwotondim : s - fv[e][q] * oneontwotondim;
-  }
-  a.unew[(long)v * a.ustride + c] = s;
+      for (int q = 0; q < 4; ++q) s = side ? s + fv[e][q] * oneontwotondim : s - fv[e][q] * oneontwotondim;
+    }
+    a.unew[(long)v * a.ustride + c] = s;
   }
 }
 
-// The leaves are found from the side with fewer octs: every cell of the
+// The leaves are found from the side with fewer tasks: every cell of the
 // coarser level, or every side of the level's own octs where the neighbour
 // oct is missing (its cell is the leaf), of which the first in the
-// reference's order takes the cell.  Behind 1,000 octs on a level of 32,768
-// the first way took 28 us, the second 7.  Where that is few tasks, each
-// variable is a task of its own: the walk is repeated, but the kernel is
-// bound by latency then.  blk of nblk workgroups.
+// reference's order takes the cell.  Behind 2,000 octs on a level of 32,768
+// the first way takes 8.1 us, the second 6.8; behind 95,000 14.3 and 21.7.
+// The first walk is two dependent loads shorter, so coarser levels of few
+// octs, where latency is all there is, always take it (4,096 octs: 5.3
+// against 6.8 us behind 2,000 and 5.6 against 7.7 behind 400).  Where that is
+// few tasks, each variable is a task of its own: the walk is repeated, but
+// the kernel is bound by latency then.  blk of nblk workgroups.
 __device__ __forceinline__ void reflux_tasks(const AmrLevelArgs& a, unsigned blk, unsigned nblk) {
   const AmrTreeView& t = a.t;
   const unsigned nf = (unsigned)level_count(a.noct, a.dnoct), nc = (unsigned)level_count(a.noct_coarse, a.dnoct_coarse);
@@ -524,23 +538,27 @@ __device__ __forceinline__ void reflux_tasks(const AmrLevelArgs& a, unsigned blk
   const bool coarse = reflux_from_coarse(nf, nc);
   const unsigned per = coarse ? 8 * nc : 6 * nf;  // below 2^31, as cell indices are
   const unsigned split = per < kRefluxSplit ? 5 : 1;
+  const unsigned octs = coarse ? nc : nf;
   for (unsigned i = id; i < per * split; i += stride) {
     const unsigned v0 = split == 1 ? 0 : i / per, r = split == 1 ? i : i - v0 * per;
     const int v1 = split == 1 ? 5 : (int)v0 + 1;
-    if (coarse) {  // (cell, oct), the oct fastest
-      const unsigned ind = r / nc;
-      const int g = a.active_coarse[r - ind * nc];
-      const long c = cell_of(t, (int)ind + 1, g);
-      if (t.son[c] == 0) reflux_cell(a, g, (int)ind + 1, c, (int)v0, v1, -1);  // only leaves (:811,863)
-    } else {  // (side, oct)
-      const unsigned side = r / nf, o = r - side * nf;
-      const int c = nbor_of(t, a.active[o], (int)side + 1);
-      if (c <= t.ncoarse || t.son[c] != 0) continue;
-      const unsigned q = (unsigned)(c - t.ncoarse - 1), ind = q / (unsigned)t.ngridmax;
-      // c lies on the oct's side `side`: the same key as reflux_cell's
-      reflux_cell(a, (int)(q - ind * (unsigned)t.ngridmax) + 1, (int)ind + 1, c, (int)v0, v1,
-                  (int)(o / a.nv) * 6 + (int)side);
+    const unsigned k = r / octs, o = r - k * octs;  // (cell or side, oct), the oct fastest
+    int g, ind, first;
+    long c;
+    if (coarse) {
+      g = a.active_coarse[o];
+      ind = (int)k + 1;
+      c = cell_of(t, ind, g);
+      first = -1;
+    } else {
+      c = nbor_of(t, a.active[o], (int)k + 1);
+      if (c <= t.ncoarse) continue;
+      const unsigned q = (unsigned)(c - t.ncoarse - 1), m = q / (unsigned)t.ngridmax;
+      g = (int)(q - m * (unsigned)t.ngridmax) + 1;
+      ind = (int)m + 1;
+      first = (int)(o / a.nv) * 6 + (int)k;  // c lies on the oct's side k: the same key as reflux_cell's
     }
+    if (t.son[c] == 0) reflux_cell(a, g, ind, c, (int)v0, v1, first);  // only leaves (:811,863)
   }
 }
 

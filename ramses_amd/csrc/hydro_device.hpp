@@ -171,6 +171,8 @@ __device__ __forceinline__ unsigned hi_word(double x) {
   return (unsigned)((unsigned long long)__builtin_bit_cast(long long, x) >> 32);
 }
 __device__ __forceinline__ unsigned max_u(unsigned a, unsigned b) { return a > b ? a : b; }
+// Whether any active lane has the flag set: a scalar branch.
+__device__ __forceinline__ bool any_lane(bool f) { return __builtin_amdgcn_ballot_w64(f) != 0; }
 // Whether any active lane has a flag clear: a scalar branch.  The lanes'
 // masks are combined rather than their flags: a compare alone is its mask,
 // and a combination would first become 0 or 1 in a vector register.
