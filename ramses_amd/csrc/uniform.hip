@@ -240,8 +240,10 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
     constexpr bool interior = decltype(waves_tag)::value == 0;
     // FP32-mixed has the registers to keep the own column's conserved state
     // for its update two planes later (541 us at 256^3, 590 with it loaded
-    // again); in FP64 it is loaded again
-    constexpr bool kKeep = interior && sizeof(R) == 4;
+    // again); in FP64 it is loaded again, and with the solvers that are not
+    // fixed at compile time and minmod, where it spills (acoustic, 288^3: 897
+    // us, 960 with it kept)
+    constexpr bool kKeep = interior && sizeof(R) == 4 && !(RS == kDynamicRiemann && ST == 1);
     const bool ring = kind > kInterior;
     const bool xdir = kind == kLeft || kind == kRight;
     if (interior || ring) put_q(qcur, qo);
@@ -622,14 +624,15 @@ inline double wide_estimate(long W, int TZ, bool fp32) { return (TZ + 2) * (fp32
 // max_blocks workgroups.  Long chunks repeat fewer planes, short ones fill
 // the chip: 2 planes at n <= 64, 6 at 96, 16 at 128, 32 at 256 and 64 at 512
 // in FP64 (with max_blocks out of the way), the fastest or within 3% of it
-// among those measured.
-inline int best_tz(int n, long tiles, bool fp32, long max_blocks, double (*estimate)(long, int, bool) = level_estimate,
-                   double* time = nullptr) {
-  int best = n;
+// among those measured.  No chunk is longer than `longest`.
+inline int best_tz(int n, long tiles, bool fp32, long max_blocks, int longest,
+                   double (*estimate)(long, int, bool) = level_estimate, double* time = nullptr) {
+  const int last = longest < n ? longest : n;
+  int best = last;
   double least = 1e300;
-  for (int tz = n < 2 ? n : 2; tz <= n; ++tz) {
+  for (int tz = n < 2 ? n : 2; tz <= last; ++tz) {
     const long W = tiles * ((n + tz - 1) / tz);
-    if (W > max_blocks && tz < n) continue;
+    if (W > max_blocks && tz < last) continue;
     const double t = estimate(W, tz, fp32);
     if (t < least) {
       least = t;
@@ -791,16 +794,27 @@ hipError_t launch_uniform_godunov(const double* u, double* unew, int n, double d
   const auto tiles_of = [n](int tx, int ty) { return (long)((n + tx - 1) / tx) * ((n + ty - 1) / ty); };
   // with sums, three doubles per workgroup have to fit the caller's buffer
   const long max_blocks = partials ? sums_blocks(n) : 0x7fffffffL;
+  // The estimates were measured with hllc.  In FP32-mixed they ask for long
+  // chunks on large levels, up to n / 2 planes.  Workgroups of the exact
+  // solver, whose faces iterate for as long as their states need, end far
+  // apart, and of long ones the last run alone: 192^3 takes 507 us in chunks
+  // of 16 planes and 568 in those of 39, 288^3 1595 and 2012 (of 144).
+  // acoustic: 192^3 the same, 288^3 818 in chunks of 36 and 897.  Up to 160^3
+  // the estimated chunks are the better ones (160^3, exact: 349 us in chunks
+  // of 23 planes, 364 of 16), and FP64 has no such long ones.
+  int longest = n;
+  if (fp32 && n > 160 && hp.riemann == kEXACT) longest = 16;
+  if (fp32 && n > 160 && hp.riemann == kACOUSTIC) longest = 40;
   int TZ = tuning().level_tz;
   if (tile == 0 && TZ == 0 && TY == 12 && n >= 32 && n <= 160) {
     double narrow, wide;
-    best_tz(n, tiles_of(16, 12), fp32, max_blocks, level_estimate, &narrow);
-    best_tz(n, tiles_of(32, 16), fp32, max_blocks, wide_estimate, &wide);
+    best_tz(n, tiles_of(16, 12), fp32, max_blocks, longest, level_estimate, &narrow);
+    best_tz(n, tiles_of(32, 16), fp32, max_blocks, longest, wide_estimate, &wide);
     if (wide < 0.93 * narrow) { TX = 32; TY = 16; }
   }
   const long tiles = tiles_of(TX, TY);
   if (TZ < 4 || TZ > n || n % TZ != 0 || tiles * (n / TZ) > max_blocks) 
-    TZ = best_tz(n, tiles, fp32, max_blocks, TX == 32 && TY == 16 ? wide_estimate : level_estimate);
+    TZ = best_tz(n, tiles, fp32, max_blocks, longest, TX == 32 && TY == 16 ? wide_estimate : level_estimate);
   if (fp32) {
     if (TY == 12) return launch_tile<float, 16, 12>(a, TZ, d_sums, s);
     if (TX == 32 && TY == 16) return launch_tile<float, 32, 16>(a, TZ, d_sums, s);
