@@ -331,7 +331,10 @@ int ramses_amr_refine_fine(const ramses_amr_tree *t, const ramses_amr_level *lv,
  * and dtold(l) at index l (RAMSES_MAX_LEVELS+2 entries); time is t.
  * noct, free, the counters and work are updated by the library; work is a
  * device workspace the library grows as needed (start with NULL / 0 and
- * release it with ramses_amr_mesh_release). */
+ * release it with ramses_amr_mesh_release).  A caller may set it to a buffer
+ * of its own, at least 16-byte aligned: steps whose levels it is large enough
+ * for (ramses_amr_work_bytes, and with adaptive
+ * ramses_amr_refine_work_bytes) allocate nothing. */
 typedef struct ramses_amr_mesh {
   ramses_amr_tree tree;
   int *active[RAMSES_MAX_LEVELS + 1];

@@ -719,14 +719,22 @@ int ramses_amr_refine_fine(const ramses_amr_tree* t, const ramses_amr_level* lv,
 // ---------------------------------------------------------------------------
 namespace {
 
+// The device words that amr_begin finds zero and leaves zero.
+struct StepWords {
+  unsigned long long wmax;  // the largest wave speed
+  unsigned done;            // workgroups that have finished
+  unsigned unused;
+};
+
 struct StepCtx {
   ramses_amr_mesh* m;
   hipStream_t s;
   Config cfg;
   bool cons_armed;  // nstep_coarse changed since the last update_time
   bool cons_done;   // the step's first update_time has been passed
-  unsigned long long* wmax;  // zeroed device words of amr_begin
-  unsigned* done;
+  // the workspace whose words this step has zeroed
+  void* work = nullptr;
+  unsigned long work_bytes = 0;
 };
 
 // The grid lists and host counts of every level.
@@ -766,6 +774,20 @@ int ensure_work(ramses_amr_mesh* m, size_t need, hipStream_t s) {
   return 0;
 }
 
+// The words at the end of the workspace, in the 256 bytes by which every
+// need exceeds what is used of an aligned buffer; zeroed on first use in a
+// step.
+int step_words(StepCtx& c, StepWords*& w) {
+  const ramses_amr_mesh* m = c.m;
+  w = (StepWords*)(((uintptr_t)m->work + m->work_bytes - sizeof(StepWords)) & ~(uintptr_t)15);
+  if (c.work == m->work && c.work_bytes == m->work_bytes) return 0;
+  hipError_t e = ramses::launch_set_ints(reinterpret_cast<int*>(w), (int)(sizeof(StepWords) / sizeof(int)), 0, c.s);
+  if (e != hipSuccess) return hip_fail(e, "step words launch");
+  c.work = m->work;
+  c.work_bytes = m->work_bytes;
+  return 0;
+}
+
 int amr_step_rec(StepCtx& c, int l, int icount) {
   ramses_amr_mesh* m = c.m;
   if (m->noct[l] == 0) return 0;
@@ -793,9 +815,13 @@ int amr_step_rec(StepCtx& c, int l, int icount) {
   // finer level has octs, update_time's bookkeeping (and the conservation
   // sums: mass_tot = mass_tot + mass_all etc., hydro/courant_fine.f90:152-154)
   const int nsub_coarser = l > m->levelmin ? m->nsubcycle[l - 1] : 0;
+  size_t need = amr_work(lv.noct, c.cfg.nvector);
+  const size_t sums_need = m->sums ? ramses::amr_begin_partials_bytes(lv.noct, false) + 256 : 0;
+  if (sums_need > need) need = sums_need;
+  StepWords* words = nullptr;
+  if ((rc = ensure_work(m, need, c.s)) || (rc = step_words(c, words))) return rc;
   const ramses::AmrStepDt d{m->dt, m->dtold, m->time, l, nsub_coarser, m->nsubcycle[l], l < m->nlevelmax,
-                            l < m->nlevelmax ? m->noct[l + 1] : 0, start, nullptr, c.wmax, c.done};
-  if (m->sums && (rc = ensure_work(m, ramses::amr_begin_partials_bytes(lv.noct, false), c.s))) return rc;
+                            l < m->nlevelmax ? m->noct[l + 1] : 0, start, nullptr, &words->wmax, &words->done};
   hipError_t e = ramses::launch_amr_begin(lv.active, lv.noct, v, m->uold, m->unew, v.ncell + 1, lv.dx, c.cfg.hp, d, c.s,
                                           nullptr, m->sums ? (double*)m->work : nullptr, m->sums);
   if (e != hipSuccess) return hip_fail(e, "courant / set_unew launch");
@@ -841,9 +867,7 @@ struct AmrDevState {
   int error;         // *m->error after the step
   int cons_armed;    // nstep_coarse changed since the last update_time
   long long cnt[2];  // nstep, cell_updates
-  // zero between the kernels that use them
-  unsigned long long wmax;  // amr_begin's largest wave speed
-  unsigned done;            // workgroups that have finished
+  StepWords words;   // zero between the kernels that use them
 };
 
 struct GraphState {
@@ -874,25 +898,6 @@ struct GraphState {
     cap = nullptr;
   }
 };
-
-// The mesh's library-owned state with its device part, zeroed on stream s.
-int ensure_state(ramses_amr_mesh* m, hipStream_t s, GraphState*& gs) {
-  gs = static_cast<GraphState*>(m->graph_state);
-  if (!gs) {
-    gs = new (std::nothrow) GraphState();
-    if (!gs) return fail(-1, "out of host memory");
-    m->graph_state = gs;
-  }
-  if (gs->dev) return 0;
-  hipError_t e = hipMalloc(&gs->dev, sizeof(AmrDevState));
-  if (e != hipSuccess) {
-    gs->dev = nullptr;
-    return hip_fail(e, "step state");
-  }
-  e = ramses::launch_set_ints(reinterpret_cast<int*>(gs->dev), (int)(sizeof(AmrDevState) / sizeof(int)), 0, s);
-  if (e != hipSuccess) return hip_fail(e, "step state");
-  return 0;
-}
 
 void graph_key(const ramses_amr_mesh* m, int capacity, std::vector<long>& k) {
   k.clear();
@@ -943,7 +948,7 @@ hipError_t gstep(GCtx& g, int l, int icount) {
   if (m->adaptive && m->levelmin < m->nlevelmax && (l == m->levelmin || icount > 1)) {
     for (int i = l; i < m->nlevelmax; ++i) {
       e = ramses::launch_refine_fine_dev(m->active[i], dn + i, i, g.v, g.tm, m->active[i + 1], dn + i + 1, m->pos,
-                                         m->free.ring, g.dev->free, &g.dev->done, m->flag1, m->flag2, m->xg, m->uold,
+                                         m->free.ring, g.dev->free, &g.dev->words.done, m->flag1, m->flag2, m->xg, m->uold,
                                          m->unew, g.c.interpol_type, g.c.interpol_var, g.c.hp.smallr, g.work, m->error,
                                          g.capacity, g.s);
       if (e != hipSuccess) return e;
@@ -955,7 +960,7 @@ hipError_t gstep(GCtx& g, int l, int icount) {
   if (capdt < start) start = capdt;
   const int nsub_coarser = l > m->levelmin ? m->nsubcycle[l - 1] : 0;
   const ramses::AmrStepDt d{m->dt, m->dtold, m->time, l, nsub_coarser, m->nsubcycle[l], l < m->nlevelmax, 0, start,
-                            g.dev->cnt, &g.dev->wmax, &g.dev->done};
+                            g.dev->cnt, &g.dev->words.wmax, &g.dev->words.done};
   double* partials = m->sums ? (double*)(((uintptr_t)g.work + 255) & ~(uintptr_t)255) : nullptr;
   e = ramses::launch_amr_begin(m->active[l], 0, g.v, m->uold, m->unew, us, dx, g.c.hp, d, g.s, dn + l, partials,
                                m->sums);
@@ -1044,12 +1049,26 @@ int coarse_step_graph(ramses_amr_mesh* m, hipStream_t s) {
   ramses::AmrTreeView v;
   int rc = amr_view(&m->tree, v);
   if (rc) return rc;
-  GraphState* gs = nullptr;
-  if ((rc = ensure_state(m, s, gs))) return rc;
+  GraphState* gs = static_cast<GraphState*>(m->graph_state);
   hipError_t e;
-  if (!gs->cap && (e = hipStreamCreate(&gs->cap)) != hipSuccess) return hip_fail(e, "capture stream");
-  if (!gs->host && (e = hipHostMalloc(&gs->host, sizeof(AmrDevState))) != hipSuccess)
+  if (!gs) {
+    gs = new (std::nothrow) GraphState();
+    if (!gs) return fail(-1, "out of host memory");
+    m->graph_state = gs;
+  }
+  // each by itself: a call after a failed one makes what is still missing
+  if (!gs->cap && (e = hipStreamCreate(&gs->cap)) != hipSuccess) {
+    gs->cap = nullptr;
+    return hip_fail(e, "capture stream");
+  }
+  if (!gs->dev && (e = hipMalloc(&gs->dev, sizeof(AmrDevState))) != hipSuccess) {
+    gs->dev = nullptr;
+    return hip_fail(e, "graph state");
+  }
+  if (!gs->host && (e = hipHostMalloc(&gs->host, sizeof(AmrDevState))) != hipSuccess) {
+    gs->host = nullptr;
     return hip_fail(e, "graph staging");
+  }
   if (gs->capacity != capacity || !gs->work) {
     if (gs->work) {
       if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "graph workspace sync");
@@ -1135,17 +1154,13 @@ int ramses_amr_coarse_step(ramses_amr_mesh* m, void* stream) {
       return fail(-1, "free list head/numbf out of range");
   }
   if (m->graph) return coarse_step_graph(m, (hipStream_t)stream);
-  GraphState* gs = nullptr;
-  int rc = ensure_state(m, (hipStream_t)stream, gs);
-  if (rc) return rc;
-  StepCtx c{m,     (hipStream_t)stream, current(),    m->nstep_coarse != m->nstep_coarse_old,
-            false, &gs->dev->wmax,      &gs->dev->done};
+  StepCtx c{m, (hipStream_t)stream, current(), m->nstep_coarse != m->nstep_coarse_old, false};
   // adaptive_loop resets the totals at every coarse step (amr/adaptive_loop.f90:89-91)
   if (m->sums) {
     hipError_t e = ramses::launch_set_doubles(m->sums, 3, 0.0, c.s);
     if (e != hipSuccess) return hip_fail(e, "sums reset launch");
   }
-  rc = amr_step_rec(c, m->levelmin, 1);
+  int rc = amr_step_rec(c, m->levelmin, 1);
   if (rc) return rc;
   m->nstep_coarse_old = m->nstep_coarse;  // update_time's bookkeeping (amr/update_time.f90:310)
   m->nstep_coarse += 1;
