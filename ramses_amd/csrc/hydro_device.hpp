@@ -36,12 +36,13 @@ struct HydroParams {
 // The bound on densities and pressures for the unscaled FP64 division and
 // square root below (quotients): 2^50, as the upper word of the double, when
 // the floors keep every value that is divided by, and every root's argument,
-// far from underflow; else 0, and no value passes.
+// far from underflow, and theta the slopes that are not zero; else 0, and no
+// value passes.
 inline unsigned div_range(const HydroParams& hp) {
-  const double lo = 0x1p-60, hi = 0x1p40;
+  const double lo = 0x1p-60, hi = 0x1p40, theta = __builtin_fabs(hp.slope_theta);
   const bool ok = hp.smallr >= lo && hp.smallr <= hi && hp.smallc >= lo && hp.smallc <= hi &&
-                  hp.gamma - 1.0 >= 0x1p-20 && hp.gamma <= 0x1p10 && hp.slope_theta >= -0x1p10 &&
-                  hp.slope_theta <= 0x1p10;
+                  hp.gamma - 1.0 >= 0x1p-20 && hp.gamma <= 0x1p10 && (theta == 0.0 || theta >= lo) &&
+                  theta <= 0x1p10;
   return ok ? (1023u + 50u) << 20 : 0u;
 }
 
