@@ -41,7 +41,9 @@ def _time(fn, reps=5):
 
 
 def tune_unsplit(run, key, blocks=(128, 192, 256, 320, 384, 512, 768), verbose=False):
-    """run(): one unsplit launch on the real inputs.  Returns (block, ms)."""
+    """run(): one unsplit launch on the real inputs, of the 27-point slopes:
+    the other slope types' tiles have one workgroup size, and the knob no
+    effect on them.  Returns (block, ms)."""
     if key in _cache:
         _set(UNSPLIT_BLOCK, _cache[key][0])
         return _cache[key]

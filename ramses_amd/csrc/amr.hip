@@ -193,11 +193,15 @@ __global__ __launch_bounds__(256) void amr_update(AmrLevelArgs a) {
 // variable at a time, which keeps a task's prolongation in registers.
 // interpol_var 0 only: the other modes mix the variables.
 //
-// What bounds it is the gather's chain of dependent loads (vector issue is
-// busy half the time).  Tiles next to each other in the level's list run on
-// one XCD, whose L2 then holds the cells that their stencils share (on 10^5
-// octs 262 -> 250 us, on 3 10^4 98 -> 90), and the state to update is
-// loaded while the faces are solved (another 1%).
+// What bounds it is the gather: on 10^5 octs in FP64 17,000 of a tile's
+// 30,000 cycles (FP32-mixed 16,300 of 26,400), which the other workgroup of
+// the CU fills in part (vector issue is busy half the time).  The wavefronts
+// of the corner neighbours, which only walk the tree, take 4,400 of them, the
+// edges' 7,500 and the two of centre and sides, eight cells of five variables
+// and their sons, 15,000 and 17,000.  Tiles next to each other in the level's
+// list run on one XCD, whose L2 then holds the cells that their stencils share
+// (on 10^5 octs 262 -> 250 us, on 3 10^4 98 -> 90), and the state to update
+// is loaded while the faces are solved (another 1%).
 template <typename R, int RS, int ST>
 __global__ __launch_bounds__(oct_tile::kThreads)
 __attribute__((amdgpu_waves_per_eu(4, 8))) void amr_tile(AmrLevelArgs a, double dx, const double* d_dt) {

@@ -29,7 +29,7 @@
 // What bounds it: vector issue (75% of the cycles, at the 2.0 GHz that this
 // load leaves of 2.4).  At 256^3 a pass takes 816 us in FP64 and 520 us in
 // FP32-mixed (918 and 578 with five and seven barriers, energies of both
-// sides of a face and two roots a face), at 512^3 6.3 ms.  Four FP64 waves a
+// sides of a face and two roots a face), at 512^3 6.4 ms.  Four FP64 waves a
 // SIMD (128 VGPRs, one LDS area more shared and a third barrier) ran 3%
 // slower.
 // Each primitive is computed by one ctoprim per cell per workgroup, each
@@ -773,14 +773,17 @@ hipError_t launch_courant(const double* u, int n, double dx, const HydroParams& 
 // interior waves and one ring wave: the ring's work is a third of a tile's,
 // against a half for 16x8), whose last tiles may reach past the level, or
 // 16x8 for n <= 24, where a third of a 16x12 tile's rows would.  Where the
-// estimates say so, 32x16, one workgroup of 10 waves on each CU, whose ring
-// is a fifth of the tile: at 64^3 (256 workgroups of 2 planes) 24 against 27
-// us in FP64 and 17 against 20 in FP32-mixed, at 128^3 100 against 118 in
-// FP64.  The margin leaves out 128^3 in FP32-mixed (63.5 against 68.2 us with
-// hllc and minmod, but 80.5 against 76.2 with llf and moncen); at 96^3 (58
-// against 56) and 192^3 (452 against 370) the estimates do.  Larger levels
-// take longer for a plane than the estimate says (512^3 FP32-mixed 4.4
-// against 3.8 ms): 16x12 above 160.
+// estimates say so by a margin, 32x16, one workgroup of 10 waves on each CU,
+// whose ring is a fifth of the tile.  Of the sides up to 160 that is 64 and
+// 128 in FP64 and 56 and 64 in FP32-mixed, where its workgroups just fill the
+// CUs.  The estimates were measured with hllc and minmod; the choice holds for
+// every solver with minmod, moncen and its generalised form, 32x16's time in
+// 16x12's: 64^3 0.87 to 0.95 in FP64 and 0.81 to 0.90 in FP32-mixed, 128^3
+// 0.80 to 0.90, 56^3 0.83 to 0.97.  What the margin leaves out would gain with
+// some and lose with others (96^3 0.95 to 1.02 and 0.90 to 1.09, 128^3 in
+// FP32-mixed 0.86 to 1.09, 160^3 0.83 to 1.01 and 0.94 to 1.22), and 32^3
+// loses (1.13 to 1.51).  Larger levels take longer for a plane than the
+// estimate says (512^3 FP32-mixed 4.4 against 3.8 ms): 16x12 above 160.
 hipError_t launch_uniform_godunov(const double* u, double* unew, int n, double dx, const double* d_dt,
                                   double* d_dt_next, const HydroParams& hp, bool fp32, hipStream_t s,
                                   double* partials, double* d_sums) {
