@@ -116,6 +116,12 @@ __device__ __forceinline__ void store_face(double* flux, double* tmp, size_t fba
   tmp[tbase + fvs] = ot[1];
 }
 
+// Whether a row or face shares reciprocals (see rcp_newton).  Not where the
+// registers do not hold both forms: the staged solve (ZR), and the solvers
+// that are not fixed at compile time (27-point slopes of 65,536 octs, exact:
+// 664 us in full, 675 shared; acoustic 485 and 496).
+constexpr bool share_divisions(bool zr, int rs) { return !zr && rs != kDynamicRiemann; }
+
 // One row of faces along direction D of one oct (see the file comment).
 // With ZR, ok points at the batch's refinement flags (+ lane) and a face
 // with a flagged cell on either side stores a zero flux: the value the
@@ -258,7 +264,8 @@ __device__ __forceinline__ void face_task(const UnsplitArgs& a, long t, long ngr
   c.dtxhalf = dt * 0.5;
   c.smalle = hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0);  // hydro/umuscl.f90:884
   c.hp = &hp;
-  const SolverConsts<R, !ZR> sc = make_consts<R, !ZR>(hp);  // the staged solve (ZR) divides in full
+  constexpr bool kShare = share_divisions(ZR, RS);
+  const SolverConsts<R, kShare> sc = make_consts<R, kShare>(hp);
   double* flux = a.flux + gidx * gsz_f + l;
   double* tmp = a.tmp + gidx * gsz_t + l;
   const size_t fvs = (size_t)nv * 27;
@@ -303,7 +310,8 @@ __device__ __forceinline__ void unsplit_task(const UnsplitArgs& a, long t, long 
   c.dtxhalf = dt * 0.5;
   c.smalle = hp.smallc * hp.smallc / hp.gamma / (hp.gamma - 1.0);  // :884
   c.hp = &hp;
-  const SolverConsts<R, !ZR> sc = make_consts<R, !ZR>(hp);  // the staged solve (ZR) divides in full
+  constexpr bool kShare = share_divisions(ZR, RS);
+  const SolverConsts<R, kShare> sc = make_consts<R, kShare>(hp);
 
   double* flux = a.flux + gidx * gsz_f + l;
   double* tmp = a.tmp + gidx * gsz_t + l;
