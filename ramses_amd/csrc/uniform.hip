@@ -240,10 +240,10 @@ __device__ __forceinline__ void level_tile(const double* __restrict__ u, double*
     constexpr bool interior = decltype(waves_tag)::value == 0;
     // FP32-mixed has the registers to keep the own column's conserved state
     // for its update two planes later (541 us at 256^3, 590 with it loaded
-    // again); in FP64 it is loaded again, and with the solvers that are not
-    // fixed at compile time and minmod, where it spills (acoustic, 288^3: 897
-    // us, 960 with it kept)
-    constexpr bool kKeep = interior && sizeof(R) == 4 && !(RS == kDynamicRiemann && ST == 1);
+    // again); in FP64 it is loaded again, and where the solvers that are not
+    // fixed at compile time spill with it: with minmod (acoustic, 288^3: 897
+    // us, 960 with it kept) and with sums
+    constexpr bool kKeep = interior && sizeof(R) == 4 && !(RS == kDynamicRiemann && (ST == 1 || SUMS));
     const bool ring = kind > kInterior;
     const bool xdir = kind == kLeft || kind == kRight;
     if (interior || ring) put_q(qcur, qo);
@@ -797,15 +797,17 @@ hipError_t launch_uniform_godunov(const double* u, double* unew, int n, double d
   const auto tiles_of = [n](int tx, int ty) { return (long)((n + tx - 1) / tx) * ((n + ty - 1) / ty); };
   // with sums, three doubles per workgroup have to fit the caller's buffer
   const long max_blocks = partials ? sums_blocks(n) : 0x7fffffffL;
-  // The estimates were measured with hllc.  In FP32-mixed they ask for long
-  // chunks on large levels, up to n / 2 planes.  Workgroups of the exact
-  // solver, whose faces iterate for as long as their states need, end far
-  // apart, and of long ones the last run alone: 192^3 takes 507 us in chunks
-  // of 16 planes and 568 in those of 39, 288^3 1595 and 2012 (of 144).
-  // acoustic: 192^3 the same, 288^3 818 in chunks of 36 and 897.  Up to 160^3
-  // the estimated chunks are the better ones (160^3, exact: 349 us in chunks
-  // of 23 planes, 364 of 16), and FP64 has no such long ones.
-  int longest = n;
+  // The estimates were measured with hllc up to 256^3.  On larger levels they
+  // ask for chunks of up to all n planes, whose workgroups end too far apart:
+  // 64 planes at most there (384^3 in FP32-mixed 1696 us in chunks of 64
+  // planes, 1805 in one of 384, llf and moncen with sums 2044 and 2313; FP64
+  // 2832 and, of 192, 2965).  In FP32-mixed workgroups of the exact solver,
+  // whose faces iterate for as long as their states need, end farther apart
+  // still: 192^3 takes 507 us in chunks of 16 planes and 568 in those of 39,
+  // 288^3 1595 and 2012 (of 144).  acoustic: 192^3 the same, 288^3 818 in
+  // chunks of 36 and 897.  Up to 160^3 the estimated chunks are the better
+  // ones (160^3, exact: 349 us in chunks of 23 planes, 364 of 16).
+  int longest = n > 256 ? 64 : n;
   if (fp32 && n > 160 && hp.riemann == kEXACT) longest = 16;
   if (fp32 && n > 160 && hp.riemann == kACOUSTIC) longest = 40;
   int TZ = tuning().level_tz;
