@@ -609,7 +609,8 @@ hipError_t launch_tile(const UniformArgs& a, int TZ, double* d_sums, hipStream_t
 // times are those measured with 16x12 tiles (hllc, minmod): one workgroup
 // alone 3.4 us a plane in FP64 and 2.4 in FP32-mixed, three FP64 ones 6.6,
 // four FP32-mixed ones 4.9.  The estimate is within 10% of the measured time
-// for n = 16..512 and z chunks of 2..128 planes.
+// for n = 16..256 and z chunks of 2..128 planes (larger levels: see
+// launch_uniform_godunov).
 inline double level_estimate(long W, int TZ, bool fp32) {
   const double m = (double)((W + 255) / 256);
   const double plane = fp32 ? (m <= 4 ? 1.5 + 0.85 * m : 1.4 * m) : (m <= 3 ? 1.75 + 1.65 * m : 2.2 * m);
